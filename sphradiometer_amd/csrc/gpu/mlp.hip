@@ -6,9 +6,9 @@
  *   h_0 = x (n_in), z_i = h_{i-1} W_i + b_i, h_i = GELU(z_i) (i = 1..depth),
  *   y = h_depth W_out + b_out (3 K outputs), candidate k = y[3k..3k+2] / |.|
  *
- * Weights are kept in float32 (master copy, Adam state) and in the
- * operand type of the products: bfloat16 (MFMA 16x16x16 bf16, float32
- * accumulation) or float32 (MFMA 16x16x4 f32, used to check gradients).
+ * Weights are kept in float32 (master copy, Adam state).  The products run
+ * on bfloat16 operands with float32 accumulation (mlp_bf16.hip) or, to
+ * check gradients, on float32 operands (MFMA 16x16x4 f32, this file).
  *
  * Loss per sample, with t the unit target and d_k = 1 - c_k . t:
  *   min_k d_k + (lambda / K) sum_k d_k,
@@ -24,41 +24,12 @@
 #include "../sphr_internal.h"
 #include "kernels.h"
 #include "runtime.h"
-
-typedef uint16_t bf16_t;
+#include "mlp_bf16.h"
 
 extern "C" int sphr_mlp_set_params(struct sphr_mlp *, const float *);
 
-__host__ __device__ inline bf16_t f2bf(float f)
-{
-	/* round to nearest even; NaN stays NaN */
-	union {
-		float f;
-		uint32_t u;
-	} v;
-	v.f = f;
-	if((v.u & 0x7fffffffu) > 0x7f800000u)
-		return (bf16_t) ((v.u >> 16) | 0x40);
-	const uint32_t r = 0x7fffu + ((v.u >> 16) & 1u);
-	return (bf16_t) ((v.u + r) >> 16);
-}
-
-__host__ __device__ inline float bf2f(bf16_t h)
-{
-	union {
-		float f;
-		uint32_t u;
-	} v;
-	v.u = (uint32_t) h << 16;
-	return v.f;
-}
-
-template <typename TI> __device__ inline TI to_op(float f);
-template <> __device__ inline float to_op<float>(float f) { return f; }
-template <> __device__ inline bf16_t to_op<bf16_t>(float f) { return f2bf(f); }
-
 /* ------------------------------------------------------------------ */
-/* GEMM C[M][N] (f32) = op(A)[M][K] op(B)[K][N], operands of type TI   */
+/* GEMM C[M][N] = op(A)[M][K] op(B)[K][N], float32                     */
 /* ------------------------------------------------------------------ */
 
 #define MG_BM 64
@@ -66,33 +37,13 @@ template <> __device__ inline bf16_t to_op<bf16_t>(float f) { return f2bf(f); }
 #define MG_KC 32
 #define MG_PAD 4
 
-typedef short s4v __attribute__((ext_vector_type(4)));
 typedef float f4v __attribute__((ext_vector_type(4)));
 
-template <typename TI> struct mg_mma;
-template <> struct mg_mma<float> {
-	enum { KS = 4 };
-	static __device__ inline f4v step(const float *a, const float *b, int lq, f4v c)
-	{
-		return __builtin_amdgcn_mfma_f32_16x16x4f32(a[lq], b[lq], c, 0, 0, 0);
-	}
-};
-template <> struct mg_mma<bf16_t> {
-	enum { KS = 16 };
-	/* lane i + 16 q holds k = 4 q .. 4 q + 3 of its row / column */
-	static __device__ inline f4v step(const bf16_t *a, const bf16_t *b, int lq, f4v c)
-	{
-		const s4v av = *reinterpret_cast<const s4v *>(a + 4 * lq);
-		const s4v bv = *reinterpret_cast<const s4v *>(b + 4 * lq);
-		return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, c, 0, 0, 0);
-	}
-};
-
-template <typename TI, int TA, int TB>
-__global__ void __launch_bounds__(256) k_mlp_gemm(int M, int N, int K, const TI *__restrict__ A, int lda, const TI *__restrict__ B, int ldb, float *__restrict__ C, int ldc)
+template <int TA, int TB>
+__global__ void __launch_bounds__(256) k_mlp_gemm(int M, int N, int K, const float *__restrict__ A, int lda, const float *__restrict__ B, int ldb, float *__restrict__ C, int ldc)
 {
-	__shared__ __align__(16) TI sA[MG_BM][MG_KC + MG_PAD];	/* [row][k] */
-	__shared__ __align__(16) TI sB[MG_BN][MG_KC + MG_PAD];	/* [col][k] */
+	__shared__ __align__(16) float sA[MG_BM][MG_KC + MG_PAD];	/* [row][k] */
+	__shared__ __align__(16) float sB[MG_BN][MG_KC + MG_PAD];	/* [col][k] */
 	const int m0 = blockIdx.y * MG_BM, n0 = blockIdx.x * MG_BN;
 	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 	const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
@@ -101,7 +52,6 @@ __global__ void __launch_bounds__(256) k_mlp_gemm(int M, int N, int K, const TI 
 	for(int a = 0; a < 2; a++)
 		for(int b = 0; b < 2; b++)
 			acc[a][b] = (f4v) 0;
-	const TI zero = to_op<TI>(0.f);
 	for(int k0 = 0; k0 < K; k0 += MG_KC) {
 		for(int idx = threadIdx.x; idx < MG_BM * MG_KC; idx += 256) {
 			int i, k;
@@ -113,7 +63,7 @@ __global__ void __launch_bounds__(256) k_mlp_gemm(int M, int N, int K, const TI 
 				k = idx - i * MG_KC;
 			}
 			const int gi = m0 + i, gk = k0 + k;
-			TI v = zero;
+			float v = 0.f;
 			if(gi < M && gk < K)
 				v = TA ? A[(size_t) gk * lda + gi] : A[(size_t) gi * lda + gk];
 			sA[i][k] = v;
@@ -128,16 +78,16 @@ __global__ void __launch_bounds__(256) k_mlp_gemm(int M, int N, int K, const TI 
 				j = idx - k * MG_BN;
 			}
 			const int gj = n0 + j, gk = k0 + k;
-			TI v = zero;
+			float v = 0.f;
 			if(gj < N && gk < K)
 				v = TB ? B[(size_t) gj * ldb + gk] : B[(size_t) gk * ldb + gj];
 			sB[j][k] = v;
 		}
 		__syncthreads();
-		for(int ks = 0; ks < MG_KC; ks += mg_mma<TI>::KS)
+		for(int ks = 0; ks < MG_KC; ks += 4)
 			for(int a = 0; a < 2; a++)
 				for(int b = 0; b < 2; b++)
-					acc[a][b] = mg_mma<TI>::step(&sA[wm + 16 * a + li][ks], &sB[wn + 16 * b + li][ks], lq, acc[a][b]);
+					acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(sA[wm + 16 * a + li][ks + lq], sB[wn + 16 * b + li][ks + lq], acc[a][b], 0, 0, 0);
 		__syncthreads();
 	}
 	for(int a = 0; a < 2; a++)
@@ -153,16 +103,15 @@ __global__ void __launch_bounds__(256) k_mlp_gemm(int M, int N, int K, const TI 
 		}
 }
 
-template <typename TI>
-static int mlp_gemm(int ta, int tb, int M, int N, int K, const TI *A, int lda, const TI *B, int ldb, float *C, int ldc, hipStream_t st)
+static int mlp_gemm(int ta, int tb, int M, int N, int K, const float *A, int lda, const float *B, int ldb, float *C, int ldc, hipStream_t st)
 {
 	dim3 grid((N + MG_BN - 1) / MG_BN, (M + MG_BM - 1) / MG_BM);
 	if(!ta && !tb)
-		hipLaunchKernelGGL((k_mlp_gemm<TI, 0, 0>), grid, dim3(256), 0, st, M, N, K, A, lda, B, ldb, C, ldc);
+		hipLaunchKernelGGL((k_mlp_gemm<0, 0>), grid, dim3(256), 0, st, M, N, K, A, lda, B, ldb, C, ldc);
 	else if(ta && !tb)
-		hipLaunchKernelGGL((k_mlp_gemm<TI, 1, 0>), grid, dim3(256), 0, st, M, N, K, A, lda, B, ldb, C, ldc);
+		hipLaunchKernelGGL((k_mlp_gemm<1, 0>), grid, dim3(256), 0, st, M, N, K, A, lda, B, ldb, C, ldc);
 	else if(!ta && tb)
-		hipLaunchKernelGGL((k_mlp_gemm<TI, 0, 1>), grid, dim3(256), 0, st, M, N, K, A, lda, B, ldb, C, ldc);
+		hipLaunchKernelGGL((k_mlp_gemm<0, 1>), grid, dim3(256), 0, st, M, N, K, A, lda, B, ldb, C, ldc);
 	else
 		return -1;
 	return hipGetLastError() == hipSuccess ? 0 : -1;
@@ -182,16 +131,15 @@ __device__ inline float gelu_d(float z)
 	return 0.5f * (1.f + erff(z * 0.70710678118654752f)) + z * 0.39894228040143268f * expf(-0.5f * z * z);
 }
 
-/* z += b; h = GELU(z) as the operand type (hidden layers) */
-template <typename TI>
-__global__ void k_bias_gelu(float *__restrict__ Z, const float *__restrict__ b, int rows, int n, TI *__restrict__ H)
+/* z += b; h = GELU(z) (hidden layers) */
+__global__ void k_bias_gelu(float *__restrict__ Z, const float *__restrict__ b, int rows, int n, float *__restrict__ H)
 {
 	const long i = (long) blockIdx.x * blockDim.x + threadIdx.x;
 	if(i >= (long) rows * n)
 		return;
 	const float z = Z[i] + b[i % n];
 	Z[i] = z;
-	H[i] = to_op<TI>(gelu(z));
+	H[i] = gelu(z);
 }
 
 __global__ void k_bias(float *__restrict__ Z, const float *__restrict__ b, int rows, int n)
@@ -202,36 +150,29 @@ __global__ void k_bias(float *__restrict__ Z, const float *__restrict__ b, int r
 	Z[i] += b[i % n];
 }
 
-/* dZ = dH * GELU'(Z), also as the operand type */
-template <typename TI>
-__global__ void k_gelu_back(const float *__restrict__ dH, const float *__restrict__ Z, long count, float *__restrict__ dZ, TI *__restrict__ dZo)
+/* dZ = dH * GELU'(Z) */
+__global__ void k_gelu_back(const float *__restrict__ dH, const float *__restrict__ Z, long count, float *__restrict__ dZ)
 {
 	const long i = (long) blockIdx.x * blockDim.x + threadIdx.x;
 	if(i >= count)
 		return;
-	const float d = dH[i] * gelu_d(Z[i]);
-	dZ[i] = d;
-	dZo[i] = to_op<TI>(d);
+	dZ[i] = dH[i] * gelu_d(Z[i]);
 }
 
-template <typename TI>
-__global__ void k_to_op(const float *__restrict__ x, long count, TI *__restrict__ y)
+/* db[j] = sum_r dZ[r][j]: 64 columns per workgroup, the rows over its four
+ * waves */
+__global__ void __launch_bounds__(256) k_colsum(const float *__restrict__ dZ, int rows, int n, float *__restrict__ db)
 {
-	const long i = (long) blockIdx.x * blockDim.x + threadIdx.x;
-	if(i < count)
-		y[i] = to_op<TI>(x[i]);
-}
-
-/* db[j] = sum_r dZ[r][j] */
-__global__ void k_colsum(const float *__restrict__ dZ, int rows, int n, float *__restrict__ db)
-{
-	const int j = blockIdx.x * blockDim.x + threadIdx.x;
-	if(j >= n)
-		return;
+	__shared__ float part[4][64];
+	const int c = threadIdx.x & 63, w = threadIdx.x >> 6, j = blockIdx.x * 64 + c;
 	float s = 0.f;
-	for(int r = 0; r < rows; r++)
-		s += dZ[(size_t) r * n + j];
-	db[j] = s;
+	if(j < n)
+		for(int r = w; r < rows; r += 4)
+			s += dZ[(size_t) r * n + j];
+	part[w][c] = s;
+	__syncthreads();
+	if(w == 0 && j < n)
+		db[j] = (part[0][c] + part[1][c]) + (part[2][c] + part[3][c]);
 }
 
 /* candidate loss and its gradient; one thread per sample */
@@ -340,34 +281,28 @@ __global__ void k_seeds(const float *__restrict__ Y, int rows, int K, double *__
 /* the network object                                                  */
 /* ------------------------------------------------------------------ */
 
-#define MLP_MAX_LAYERS 8
-
 struct sphr_mlp {
 	int n_in, width, depth, K, max_batch, bf16;
 	int nl;				/* layers = depth + 1 */
 	int din[MLP_MAX_LAYERS], dout[MLP_MAX_LAYERS];
 	size_t ow[MLP_MAX_LAYERS], ob[MLP_MAX_LAYERS];
 	size_t nparam;
-	float *p, *g, *m, *v;		/* params, grads, Adam moments (float32) */
-	void *wop;			/* weights in the operand type (same offsets as p) */
-	void *xin;			/* [max_batch][n_in] operand type */
+	float *p, *g, *m, *v;		/* params, grads, Adam moments */
+	struct mlp_bf bf;		/* the bfloat16 form's buffers */
+	/* the float32 form's */
 	float *Z[MLP_MAX_LAYERS];	/* pre-activations [max_batch][dout] */
-	void *H[MLP_MAX_LAYERS];	/* activations (operand type) */
+	float *H[MLP_MAX_LAYERS];	/* activations */
 	float *dA, *dZ;			/* [max_batch][max width] */
-	void *dZo;			/* operand type */
 	float *loss;			/* [max_batch] */
+	/* [max_batch][3 K] outputs of the last forward */
+	const float *y;
 };
-
-static size_t op_size(const struct sphr_mlp *m)
-{
-	return m->bf16 ? sizeof(bf16_t) : sizeof(float);
-}
 
 extern "C" void sphr_mlp_free(struct sphr_mlp *m)
 {
 	if(!m)
 		return;
-	void *ptrs[] = { m->p, m->g, m->m, m->v, m->wop, m->xin, m->dA, m->dZ, m->dZo, m->loss };
+	void *ptrs[] = { m->p, m->g, m->m, m->v, m->dA, m->dZ, m->loss };
 	for(unsigned i = 0; i < sizeof(ptrs) / sizeof(ptrs[0]); i++)
 		if(ptrs[i])
 			hipFree(ptrs[i]);
@@ -377,6 +312,7 @@ extern "C" void sphr_mlp_free(struct sphr_mlp *m)
 		if(m->H[l])
 			hipFree(m->H[l]);
 	}
+	mlp_bf_free(&m->bf);
 	free(m);
 }
 
@@ -411,13 +347,17 @@ extern "C" struct sphr_mlp *sphr_mlp_new(int n_in, int width, int depth, int n_c
 	const size_t wmax = width > 3 * n_candidates ? width : 3 * n_candidates;
 	const size_t B = max_batch;
 	int bad = sphr_rt_check(hipMalloc(&m->p, off * 4), "hipMalloc") || sphr_rt_check(hipMalloc(&m->g, off * 4), "hipMalloc")
-		  || sphr_rt_check(hipMalloc(&m->m, off * 4), "hipMalloc") || sphr_rt_check(hipMalloc(&m->v, off * 4), "hipMalloc")
-		  || sphr_rt_check(hipMalloc(&m->wop, off * op_size(m)), "hipMalloc")
-		  || sphr_rt_check(hipMalloc(&m->xin, B * n_in * op_size(m)), "hipMalloc")
-		  || sphr_rt_check(hipMalloc(&m->dA, B * wmax * 4), "hipMalloc") || sphr_rt_check(hipMalloc(&m->dZ, B * wmax * 4), "hipMalloc")
-		  || sphr_rt_check(hipMalloc(&m->dZo, B * wmax * op_size(m)), "hipMalloc") || sphr_rt_check(hipMalloc(&m->loss, B * 4), "hipMalloc");
-	for(int l = 0; l < m->nl && !bad; l++)
-		bad = sphr_rt_check(hipMalloc(&m->Z[l], B * m->dout[l] * 4), "hipMalloc") || sphr_rt_check(hipMalloc(&m->H[l], B * m->dout[l] * op_size(m)), "hipMalloc");
+		  || sphr_rt_check(hipMalloc(&m->m, off * 4), "hipMalloc") || sphr_rt_check(hipMalloc(&m->v, off * 4), "hipMalloc");
+	if(m->bf16) {
+		bad = bad || mlp_bf_alloc(&m->bf, m->nl, m->din, m->dout, m->ow, m->ob, m->K, max_batch);
+		m->y = m->bf.Z[m->nl - 1];
+	} else {
+		bad = bad || sphr_rt_check(hipMalloc(&m->dA, B * wmax * 4), "hipMalloc") || sphr_rt_check(hipMalloc(&m->dZ, B * wmax * 4), "hipMalloc")
+		      || sphr_rt_check(hipMalloc(&m->loss, B * 4), "hipMalloc");
+		for(int l = 0; l < m->nl && !bad; l++)
+			bad = sphr_rt_check(hipMalloc(&m->Z[l], B * m->dout[l] * 4), "hipMalloc") || sphr_rt_check(hipMalloc(&m->H[l], B * m->dout[l] * 4), "hipMalloc");
+		m->y = m->Z[m->nl - 1];
+	}
 	if(bad) {
 		sphr_mlp_free(m);
 		return NULL;
@@ -454,20 +394,10 @@ extern "C" struct sphr_mlp *sphr_mlp_new(int n_in, int width, int depth, int n_c
 	return m;
 }
 
-static int refresh_op_weights(struct sphr_mlp *m, hipStream_t st)
-{
-	const long n = (long) m->nparam;
-	if(m->bf16)
-		hipLaunchKernelGGL((k_to_op<bf16_t>), dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, st, m->p, n, (bf16_t *) m->wop);
-	else
-		hipLaunchKernelGGL((k_to_op<float>), dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, st, m->p, n, (float *) m->wop);
-	return hipGetLastError() == hipSuccess ? 0 : -1;
-}
-
 extern "C" int sphr_mlp_set_params(struct sphr_mlp *m, const float *host)
 {
 	hipStream_t st = sphr_rt_stream();
-	if(sphr_rt_check(hipMemcpyAsync(m->p, host, m->nparam * 4, hipMemcpyHostToDevice, st), "hipMemcpy") || refresh_op_weights(m, st))
+	if(sphr_rt_check(hipMemcpyAsync(m->p, host, m->nparam * 4, hipMemcpyHostToDevice, st), "hipMemcpy") || (m->bf16 && mlp_bf_refresh(&m->bf, m->p, st)))
 		return -1;
 	return sphr_rt_check(hipStreamSynchronize(st), "synchronize");
 }
@@ -487,45 +417,39 @@ extern "C" long sphr_mlp_n_params(const struct sphr_mlp *m)
 	return (long) m->nparam;
 }
 
-template <typename TI>
-static int forward_t(struct sphr_mlp *m, const float *x, int B, hipStream_t st)
+static int forward_f32(struct sphr_mlp *m, const float *x, int B, hipStream_t st)
 {
-	const long nx = (long) B * m->n_in;
-	hipLaunchKernelGGL((k_to_op<TI>), dim3((unsigned) ((nx + 255) / 256)), dim3(256), 0, st, x, nx, (TI *) m->xin);
-	const TI *in = (const TI *) m->xin;
-	const TI *W = (const TI *) m->wop;
+	const float *in = x;
 	for(int l = 0; l < m->nl; l++) {
-		if(mlp_gemm<TI>(0, 0, B, m->dout[l], m->din[l], in, m->din[l], W + m->ow[l], m->dout[l], m->Z[l], m->dout[l], st))
+		if(mlp_gemm(0, 0, B, m->dout[l], m->din[l], in, m->din[l], m->p + m->ow[l], m->dout[l], m->Z[l], m->dout[l], st))
 			return -1;
 		const long n = (long) B * m->dout[l];
 		if(l < m->depth)
-			hipLaunchKernelGGL((k_bias_gelu<TI>), dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, st, m->Z[l], m->p + m->ob[l], B, m->dout[l], (TI *) m->H[l]);
+			hipLaunchKernelGGL(k_bias_gelu, dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, st, m->Z[l], m->p + m->ob[l], B, m->dout[l], m->H[l]);
 		else
 			hipLaunchKernelGGL(k_bias, dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, st, m->Z[l], m->p + m->ob[l], B, m->dout[l]);
-		in = (const TI *) m->H[l];
+		in = m->H[l];
 	}
 	return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-template <typename TI>
-static int backward_t(struct sphr_mlp *m, int B, hipStream_t st)
+static int backward_f32(struct sphr_mlp *m, const float *x, int B, hipStream_t st)
 {
-	const TI *W = (const TI *) m->wop;
-	/* dY is in dZ (float) on entry; its operand copy in dZo */
+	/* dY is in dZ on entry */
 	for(int l = m->nl - 1; l >= 0; l--) {
 		const int di = m->din[l], dn = m->dout[l];
-		const TI *in = l ? (const TI *) m->H[l - 1] : (const TI *) m->xin;
+		const float *in = l ? m->H[l - 1] : x;
 		/* dW = in^T dZ, db = colsum dZ */
-		if(mlp_gemm<TI>(1, 0, di, dn, B, in, di, (const TI *) m->dZo, dn, m->g + m->ow[l], dn, st))
+		if(mlp_gemm(1, 0, di, dn, B, in, di, m->dZ, dn, m->g + m->ow[l], dn, st))
 			return -1;
-		hipLaunchKernelGGL(k_colsum, dim3((dn + 255) / 256), dim3(256), 0, st, m->dZ, B, dn, m->g + m->ob[l]);
+		hipLaunchKernelGGL(k_colsum, dim3((dn + 63) / 64), dim3(256), 0, st, m->dZ, B, dn, m->g + m->ob[l]);
 		if(l == 0)
 			break;
 		/* dA = dZ W^T, then through GELU of layer l-1 */
-		if(mlp_gemm<TI>(0, 1, B, di, dn, (const TI *) m->dZo, dn, W + m->ow[l], dn, m->dA, di, st))
+		if(mlp_gemm(0, 1, B, di, dn, m->dZ, dn, m->p + m->ow[l], dn, m->dA, di, st))
 			return -1;
 		const long n = (long) B * di;
-		hipLaunchKernelGGL((k_gelu_back<TI>), dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, st, m->dA, m->Z[l - 1], n, m->dZ, (TI *) m->dZo);
+		hipLaunchKernelGGL(k_gelu_back, dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, st, m->dA, m->Z[l - 1], n, m->dZ);
 	}
 	return hipGetLastError() == hipSuccess ? 0 : -1;
 }
@@ -540,11 +464,10 @@ extern "C" int sphr_mlp_forward(struct sphr_mlp *m, const float *x, int B, float
 	if(!m || !x || B < 1 || B > m->max_batch)
 		return -1;
 	hipStream_t st = pick(stream);
-	const int r = m->bf16 ? forward_t<bf16_t>(m, x, B, st) : forward_t<float>(m, x, B, st);
-	if(r)
+	if(m->bf16 ? mlp_bf_forward(&m->bf, m->p, x, B, st) : forward_f32(m, x, B, st))
 		return -1;
 	if(y)
-		return sphr_rt_check(hipMemcpyAsync(y, m->Z[m->nl - 1], (size_t) B * 3 * m->K * 4, hipMemcpyDeviceToDevice, st), "hipMemcpy");
+		return sphr_rt_check(hipMemcpyAsync(y, m->y, (size_t) B * 3 * m->K * 4, hipMemcpyDeviceToDevice, st), "hipMemcpy");
 	return 0;
 }
 
@@ -555,33 +478,39 @@ extern "C" int sphr_mlp_loss_grad(struct sphr_mlp *m, const float *x, const floa
 	if(!m || !x || !target || B < 1 || B > m->max_batch)
 		return -1;
 	hipStream_t st = pick(stream);
-	if(sphr_mlp_forward(m, x, B, NULL, st))
-		return -1;
-	const int L = m->nl - 1;
-	hipLaunchKernelGGL(k_loss, dim3((B + 255) / 256), dim3(256), 0, st, m->Z[L], target, B, m->K, lambda, loss ? loss : m->loss, m->dZ);
-	const long n = (long) B * 3 * m->K;
 	if(m->bf16)
-		hipLaunchKernelGGL((k_to_op<bf16_t>), dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, st, m->dZ, n, (bf16_t *) m->dZo);
-	else
-		hipLaunchKernelGGL((k_to_op<float>), dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, st, m->dZ, n, (float *) m->dZo);
+		return mlp_bf_loss_grad(&m->bf, m->p, m->g, x, target, B, lambda, loss, NULL, NULL, NULL, st);
+	if(forward_f32(m, x, B, st))
+		return -1;
+	hipLaunchKernelGGL(k_loss, dim3((B + 255) / 256), dim3(256), 0, st, m->Z[m->nl - 1], target, B, m->K, lambda, loss ? loss : m->loss, m->dZ);
 	if(hipGetLastError() != hipSuccess)
 		return -1;
-	return m->bf16 ? backward_t<bf16_t>(m, B, st) : backward_t<float>(m, B, st);
+	return backward_f32(m, x, B, st);
+}
+
+static struct mlp_adam adam_args(float lr, float beta1, float beta2, float eps, int step)
+{
+	struct mlp_adam a = { lr, beta1, beta2, eps, 1.f - powf(beta1, (float) step), 1.f - powf(beta2, (float) step) };
+	return a;
 }
 
 extern "C" int sphr_mlp_adam(struct sphr_mlp *m, float lr, float beta1, float beta2, float eps, int step, void *stream)
 {
 	hipStream_t st = pick(stream);
+	const struct mlp_adam a = adam_args(lr, beta1, beta2, eps, step);
+	if(m->bf16)
+		return mlp_bf_adam(&m->bf, m->p, m->g, m->m, m->v, &a, st);
 	const long n = (long) m->nparam;
-	const float c1 = 1.f - powf(beta1, (float) step), c2 = 1.f - powf(beta2, (float) step);
-	hipLaunchKernelGGL(k_adam, dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, st, m->p, m->g, m->m, m->v, n, lr, beta1, beta2, eps, c1, c2);
-	if(hipGetLastError() != hipSuccess)
-		return -1;
-	return refresh_op_weights(m, st);
+	hipLaunchKernelGGL(k_adam, dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, st, m->p, m->g, m->m, m->v, n, a.lr, a.b1, a.b2, a.eps, a.c1, a.c2);
+	return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 extern "C" int sphr_mlp_train_step(struct sphr_mlp *m, const float *x, const float *target, int B, float lambda, float lr, int step, float *loss, void *stream)
 {
+	if(m && m->bf16 && x && target && B >= 1 && B <= m->max_batch) {
+		const struct mlp_adam a = adam_args(lr, 0.9f, 0.999f, 1e-8f, step);
+		return mlp_bf_loss_grad(&m->bf, m->p, m->g, x, target, B, lambda, loss, &a, m->m, m->v, pick(stream));
+	}
 	if(sphr_mlp_loss_grad(m, x, target, B, lambda, loss, stream))
 		return -1;
 	return sphr_mlp_adam(m, lr, 0.9f, 0.999f, 1e-8f, step, stream);
@@ -592,7 +521,7 @@ extern "C" int sphr_mlp_seeds(struct sphr_mlp *m, int B, double *seeds, void *st
 {
 	hipStream_t st = pick(stream);
 	const int n = B * m->K;
-	hipLaunchKernelGGL(k_seeds, dim3((n + 255) / 256), dim3(256), 0, st, m->Z[m->nl - 1], B, m->K, seeds);
+	hipLaunchKernelGGL(k_seeds, dim3((n + 255) / 256), dim3(256), 0, st, m->y, B, m->K, seeds);
 	return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -607,28 +536,13 @@ extern "C" int sphr_features(const void *alm, int alm_f32, int S, int L, float *
 }
 
 /* test hook: one GEMM of the network's operand type on device float
- * inputs (converted on the way), C = op(A) op(B) */
+ * inputs, C = op(A) op(B) */
 extern "C" int sphr_mlp_gemm_check(int bf16, int ta, int tb, int M, int N, int K, const float *A, const float *B, float *C)
 {
 	hipStream_t st = sphr_rt_stream();
-	const size_t na = (size_t) M * K, nb = (size_t) K * N, es = bf16 ? 2 : 4;
-	void *dA = NULL, *dB = NULL;
-	int rc = -1;
-	if(sphr_rt_check(hipMalloc(&dA, na * es), "hipMalloc") || sphr_rt_check(hipMalloc(&dB, nb * es), "hipMalloc"))
-		goto done;
-	if(bf16) {
-		hipLaunchKernelGGL((k_to_op<bf16_t>), dim3((unsigned) ((na + 255) / 256)), dim3(256), 0, st, A, (long) na, (bf16_t *) dA);
-		hipLaunchKernelGGL((k_to_op<bf16_t>), dim3((unsigned) ((nb + 255) / 256)), dim3(256), 0, st, B, (long) nb, (bf16_t *) dB);
-		rc = mlp_gemm<bf16_t>(ta, tb, M, N, K, (const bf16_t *) dA, ta ? M : K, (const bf16_t *) dB, tb ? K : N, C, N, st);
-	} else {
-		hipLaunchKernelGGL((k_to_op<float>), dim3((unsigned) ((na + 255) / 256)), dim3(256), 0, st, A, (long) na, (float *) dA);
-		hipLaunchKernelGGL((k_to_op<float>), dim3((unsigned) ((nb + 255) / 256)), dim3(256), 0, st, B, (long) nb, (float *) dB);
-		rc = mlp_gemm<float>(ta, tb, M, N, K, (const float *) dA, ta ? M : K, (const float *) dB, tb ? K : N, C, N, st);
-	}
-	if(!rc)
-		rc = sphr_rt_check(hipStreamSynchronize(st), "synchronize");
-done:
-	hipFree(dA);
-	hipFree(dB);
-	return rc;
+	if(bf16)
+		return ta && tb ? -1 : mlp_bf_gemm(ta, tb, M, N, K, A, B, C, st);
+	if(mlp_gemm(ta, tb, M, N, K, A, ta ? M : K, B, tb ? K : N, C, N, st))
+		return -1;
+	return sphr_rt_check(hipStreamSynchronize(st), "synchronize");
 }

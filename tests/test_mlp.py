@@ -269,3 +269,66 @@ def test_gpu_jobs_sky_factory(P):
     assert np.all(out["value"] >= out["grid_max"] - 1e-5 * np.abs(out["grid_max"]))
     t = d_t.to_numpy(np.float32, (Sg, 3))
     assert np.max(np.abs(np.linalg.norm(t, axis=1) - 1.0)) < 1e-5
+
+
+def bf16_loss_grad(p, x, t, n_in, width, depth, K, lam):
+    """The bfloat16 network's gradients with 64-bit sums: weights, inputs,
+    activations and output gradients rounded where the kernels round."""
+    def r(v):
+        return bf16_round(np.asarray(v, dtype=np.float32)).astype(np.float64)
+    layers = OM.unpack(np.asarray(p, dtype=np.float64), n_in, width, depth, K)
+    hs, zs = [r(x)], []
+    for i, (W, b) in enumerate(layers):
+        zs.append((hs[-1] @ r(W) + b).astype(np.float32).astype(np.float64))
+        hs.append(r(OM.gelu(zs[-1])))
+    rows = len(x)
+    Y = zs[-1].reshape(rows, K, 3)
+    nrm = np.linalg.norm(Y, axis=2)
+    dot = np.einsum("rkj,rj->rk", Y, t) / nrm
+    w = np.full((rows, K), lam / K)
+    w[np.arange(rows), np.argmin(1 - dot, axis=1)] += 1.0
+    dz = (-(w[:, :, None] * (t[:, None, :] - dot[:, :, None] * Y / nrm[:, :, None]) / nrm[:, :, None]) / rows).reshape(rows, 3 * K)
+    grads = []
+    for i in range(len(layers) - 1, -1, -1):
+        grads.insert(0, np.concatenate([(hs[i].T @ r(dz)).ravel(), dz.sum(axis=0)]))
+        if i:
+            dz = (r(dz) @ r(layers[i][0]).T) * OM.gelu_d(zs[i - 1])
+    return zs[-1], np.concatenate(grads)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shp,rows", [((1, 1, 1, 1), 1), ((61, 40, 3, 4), 50), ((64, 128, 1, 11), 127), ((127, 129, 2, 16), 128),
+                                      ((130, 70, 7, 5), 129), ((1089, 512, 3, 4), 300), ((200, 96, 2, 4), 1500)])
+def test_gpu_mlp_bf16_matches_rounded_oracle(P, shp, rows):
+    """bfloat16 forward, gradients and the fused update at the edges of the
+    tiles (rows, widths, 3 K past 32).  float32 sums move a value by about
+    1e-6, across a bfloat16 rounding boundary in about 1e-6 / 2^-9 = 5e-4
+    of the cases, by 2^-8 each: 1e-4 per layer in the 2-norm."""
+    rng = np.random.default_rng(21)
+    m = P.MLP(*shp, max_batch=rows, bf16=True, seed=4)
+    p = m.params()
+    x = rng.standard_normal((rows, shp[0])).astype(np.float32)
+    t = rng.standard_normal((rows, 3))
+    t = (t / np.linalg.norm(t, axis=1, keepdims=True)).astype(np.float32)
+    dx, dt, dy = S.DeviceBuffer.from_numpy(x), S.DeviceBuffer.from_numpy(t), S.DeviceBuffer(rows * 3 * shp[3] * 4)
+    y, g = bf16_loss_grad(p, x, t.astype(np.float64), *shp, 0.05)
+    m.forward(dx.ptr, rows, dy.ptr)
+    S.synchronize()
+    assert rel(dy.to_numpy(np.float32, y.shape), y) < 1e-3
+    m.loss_grad(dx.ptr, dt.ptr, rows, 0.05)
+    S.synchronize()
+    g0 = m.grads()
+    assert rel(g0, g) < 1e-3 * (shp[2] + 1)
+    # the update alone and in the training step's last launch: the same bits
+    assert S.lib().sphr_mlp_adam(m.h, 1e-3, 0.9, 0.999, 1e-8, 1, None) == 0
+    S.synchronize()
+    p1 = m.params()
+    want = p - np.float32(1e-3) * g0 / (np.abs(g0) + np.float32(1e-8))
+    assert np.max(np.abs(p1 - want)) < 2e-5
+    m.forward(dx.ptr, rows, dy.ptr)
+    S.synchronize()
+    assert rel(dy.to_numpy(np.float32, y.shape), bf16_loss_grad(p1, x, t.astype(np.float64), *shp, 0.05)[0]) < 1e-3
+    m2 = P.MLP(*shp, max_batch=rows + 200, bf16=True, seed=4)
+    m2.train_step(dx.ptr, dt.ptr, rows, 0.05, 1e-3)
+    S.synchronize()
+    assert np.array_equal(m2.params(), p1) and np.array_equal(m2.grads(), g0)
