@@ -313,3 +313,35 @@ def test_gpu_batch_peaks_are_local_maxima(oracle, local_minimum):
         seps.append(math.acos(min(1.0, cosd)))
     print("mixed vs fp64 peak separation: max %.3g rad median %.3g" % (max(seps), np.median(seps)), flush=True)
     assert np.median(seps) < 1e-4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L", [1, 2, 5, 31, 35, 36, 78, 79, 150])
+@pytest.mark.parametrize("f32", [0, 1])
+def test_gpu_refinement_from_seeds(oracle, local_minimum, L, f32):
+    """the refinement at the edges of its lane and LDS shapes (four, two
+    series per workgroup, coefficients from global memory), from seeds that
+    include both poles, an odd number of series, two seeds per series, and
+    a series that is not a number (which stays one)"""
+    from sphradiometer_amd import proposal
+    proposal._protos()
+    rng = np.random.default_rng(900 + L)
+    n, nc = 3, (L + 1) ** 2
+    l = np.concatenate([np.arange(abs(m), L + 1) for m in list(range(L + 1)) + list(range(-L, 0))])
+    c = (rng.standard_normal((n + 1, nc)) + 1j * rng.standard_normal((n + 1, nc))) * np.exp(-0.4 * l)
+    c[n, nc // 2] = np.nan
+    cdt = np.complex64 if f32 else np.complex128
+    c = c.astype(cdt)
+    seeds = np.stack([np.arccos(rng.uniform(-1, 1, 2 * n + 1)), rng.uniform(0, 2 * math.pi, 2 * n + 1)], axis=1)
+    seeds[0, 0], seeds[3, 0] = 0.0, math.pi
+    d_c, d_s = S.DeviceBuffer.from_numpy(c), S.DeviceBuffer.from_numpy(seeds)
+    d_r = [S.DeviceBuffer(8 * (2 * n + 1)) for _ in range(3)]
+    print(f"refine L={L} f32={f32}", flush=True)
+    assert S.lib().sphr_refine_peaks(d_c.ptr, f32, 2 * n + 1, 2, L, d_s.ptr, 0, d_r[0].ptr, d_r[1].ptr, d_r[2].ptr, None) == 0
+    S.synchronize()
+    th, ph, v = (d.to_numpy(np.float64, (2 * n + 1,)) for d in d_r)
+    assert np.isnan(v[2 * n]) and np.isnan(th[2 * n]) and np.isnan(ph[2 * n])
+    for k in range(2 * n):
+        full = c[k // 2].astype(np.complex128)
+        local_minimum(full, L, th[k], ph[k], v[k], 1e-10 * np.abs(full).max() * (L + 1), seed=False)
+        assert v[k] <= oracle.eval_series(full, L, 0, *seeds[k]).real + 1e-10
