@@ -16,25 +16,18 @@
  *   south cap: the mirror of the north cap,
  * pixels numbered ring by ring from the north pole, phi ascending.
  *
- * Kernel: workgroup = one series, its coefficients staged in LDS once;
- * the northern rings (through the equator) in chunks of HP_RC, each with
- * its mirror ring 4 nside - i (same nphi and phi_0, z -> -z).  Per chunk,
- * task (|m|, ring) - rings fastest, so that the lanes of a wave share m
- * and read the same coefficients - runs the Legendre recurrence at the
- * ring's z once for the ring and its mirror (even and odd l - m sums,
- * Pbar_lm(-z) = (-1)^(l+m) Pbar_lm(z)) (float64,
- * from Pbar_mm = cm[m] sin^m theta and the division-free coefficient
- * pairs of the plan), giving F_m and F_-m; with G_m = F_m exp(i m phi_0)
- * the ring's values are
- *   f(phi_0 + 2 pi j / nphi) = Re sum_m G_m exp(i m phi'),  phi' = 2 pi j / nphi,
- *     = G_0.re + sum_{m>0} A_m cos(m phi') - B_m sin(m phi'),
- *   A_m = Re (G_m + G_-m), B_m = Im (G_m - G_-m),
- * kept in LDS per (ring, m); then one thread per four pixels of a ring
- * (a quarter turn apart) sums over m with exp(i m phi') advanced by one
- * complex rotation per m.
+ * With b_lm = a_lm + (-1)^m conj(a_l,-m) (m > 0), b_l0 = Re a_l0 and
+ * F_m(z) = sum_l b_lm Pbar_lm(z), a ring's values are
+ *   f(phi) = sum_m A_m cos(m phi) - B_m sin(m phi),  A_m + i B_m = F_m,
+ * so a map is two contractions with tables that all series share: the
+ * Legendre values of the rings and the cosines of the pixels.  k_healpix_mm
+ * runs both on MFMA, eight series per workgroup (see there); orders and
+ * resolutions whose tables would be too large run k_healpix_ring, which
+ * forms them by recurrence.
  */
 #include <hip/hip_runtime.h>
 #include <math.h>
+#include <stdint.h>
 #include <stdlib.h>
 #include <string.h>
 #include <sphradiometer/sh_series.h>
@@ -51,6 +44,11 @@ struct sphr_healpix {
 	int L, nside, precision;
 	double *d_cf;	/* [nal][2]: alpha_lm, alpha_lm / alpha_{l-1,m} at the (l, m >= 0) slots */
 	double *d_cm;	/* [L + 1]: Pbar_mm(cos theta) = cm[m] sin^m theta */
+	/* the tables of k_healpix_mm, NULL where k_healpix_ring runs */
+	double *P;	/* Legendre values */
+	void *W;	/* cosines and sines of the pixels */
+	int *off;	/* [L + 1] first step of an order, then [2 nside + 1] first tile of a ring */
+	int k0, k2, k1, steps, rc;
 };
 
 /* ring geometry: z, sin theta (without cancellation near the poles), the
@@ -82,201 +80,368 @@ __device__ inline void hp_ring(int nside, int i, double *z, double *st, int *nph
 	}
 }
 
-#define HP_RC 16		/* rings per chunk */
 #define HP_SPW 4		/* series per workgroup of the per-ring form */
 
-/* sin and cos of pi a / b in the map's precision */
-__device__ inline void hp_sincospi(int a, int b, double *sn, double *cs)
+/*
+ * The maps of eight series on 2 RC rings per workgroup (RC northern rings
+ * and their mirrors), eight waves.
+ *
+ *  A. Legendre sums, in float64 whatever the maps' type: per order m the
+ *     product [16 rings] x [l] x [8 series x (re, im)] on
+ *     v_mfma_f64_16x16x4f64, the l of each parity apart: Pbar_lm(-z) =
+ *     (-1)^(l+m) Pbar_lm(z), so the even and odd sums E and O give the ring
+ *     (E + O) and its mirror (E - O).  The Legendre table is laid out in the
+ *     operand's lane order; the coefficients come straight from the a_lm.
+ *     The orders are dealt to the waves, results go to LDS as the next
+ *     product's left operand [ring][north / south, series][m, (A, B)].
+ *  B. Pixel sums: nphi is a multiple of 4 and the pixels j + q nphi / 4
+ *     (q = 0..3) sit at phi + q pi / 2.  With C_m = A_m cos m phi -
+ *     B_m sin m phi, D_m = A_m sin m phi + B_m cos m phi and
+ *       S0, S2 = sums of C_m over m = 0, 2 mod 4,
+ *       U = sum of C_m over odd m, V = sum of +-D_m over m = 1, 3 mod 4,
+ *     the four pixels are S0 + S2 + U, S0 - S2 - V, S0 + S2 - U,
+ *     S0 - S2 + V: four products over a quarter of the ring, rows =
+ *     (north / south) x 8 series, columns = 16 pixels, on MFMA in the maps'
+ *     type; the phase of the first pixel is in the table.  LDS columns are
+ *     ordered by m mod 4 for it: m = 0 | m = 2 | odd.
+ *
+ * RC is 16, or fewer where the LDS operand would not fit (the Legendre
+ * product then computes 16 rows and drops the rest).  What bounds it: at
+ * l_max 50, nside 32 and 16384 series the products are 5.6 TFLOP in
+ * float64 (77 us at the matrix peak) and 18 in float32 (113 us), the maps
+ * 805 MB (165 us at the rate of a large copy); the phases of the one
+ * workgroup that fits a CU do not overlap (A takes 0.43 of 0.9 ms).  It
+ * replaces a recurrence per (series, m, ring) and a pass over m per pixel:
+ * 2.99 -> 0.91 ms (float64 coefficients fetched one value per lane, 31 cache
+ * accesses per load: 1.1; eight waves instead of sixteen, 1.2), nine events
+ * of l_max 120 at nside 64 in float64 0.43 -> 0.09 ms.
+ */
+#define HM_W 16
+#define HM_NT (64 * HM_W)
+#define HM_R 4
+#define HM_S 8			/* series per workgroup */
+#define HM_STAGE (HM_W * 2 * 64 * 16)	/* bytes of the waves' fetches */
+
+typedef double d4 __attribute__((ext_vector_type(4)));
+typedef float f4 __attribute__((ext_vector_type(4)));
+
+template <typename T> struct hm_ops;
+template <> struct hm_ops<float> {
+	typedef f4 acc;
+	typedef float2 pair;
+	/* two complex values, and the steps of a parity that 8 x 8 of them hold */
+	typedef float piece __attribute__((ext_vector_type(4), aligned(8)));
+	enum { STEPS = 2 };
+	static __device__ inline acc mma(float a, float b, acc c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+	static __device__ inline int row(int lq, int e) { return 4 * lq + e; }
+};
+template <> struct hm_ops<double> {
+	typedef d4 acc;
+	typedef double2 pair;
+	typedef double piece __attribute__((ext_vector_type(2), aligned(8)));
+	enum { STEPS = 1 };
+	static __device__ inline acc mma(double a, double b, acc c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+	static __device__ inline int row(int lq, int e) { return lq + 4 * e; }
+};
+
+struct hm_geom {
+	int L, nside, n, rc;
+	int k0, k2, k1;		/* padded columns of the three classes of m */
+	int ld, rs;		/* LDS strides: row, ring */
+	int steps, chunks, groups;
+	const double *P;
+	const int *off;
+};
+
+/* the LDS column of order m's A (B follows) */
+__device__ inline int hm_col(const struct hm_geom &g, int m)
 {
-	sincospi((double) a / b, sn, cs);
-}
-__device__ inline void hp_sincospi(int a, int b, float *sn, float *cs)
-{
-	sincospif((float) a / (float) b, sn, cs);
+	return m & 1 ? g.k0 + g.k2 + (m - 1) : m & 2 ? g.k0 + (m - 2) / 2 : m / 2;
 }
 
 template <typename T>
-__global__ void __launch_bounds__(HP_NT) k_healpix(const cplx<T> *__restrict__ alm, int n, int L, int nside, const double *__restrict__ cf, const double *__restrict__ cm, T *__restrict__ map)
+__global__ void __launch_bounds__(HM_NT) k_healpix_mm(const cplx<T> *__restrict__ alm, struct hm_geom g, const T *__restrict__ W, T *__restrict__ map)
 {
-	extern __shared__ __align__(16) unsigned char hp_sm[];
-	const int s = blockIdx.x, L1 = L + 1, N2 = 2 * nside;
-	const int ncoef = L1 * L1;
-	const long npix = 12L * nside * nside;
-	cplx<T> *a = reinterpret_cast<cplx<T> *>(hp_sm);		/* [ncoef] */
-	T *AB = reinterpret_cast<T *>(a + ncoef);			/* [2 HP_RC][L + 1][2]: north rows, then their mirrors */
-	/* the chunk's rings: first pixel, pixel count, AB row, prefix sums of
-	 * the quarter rings */
-	__shared__ long es[2 * HP_RC];
-	__shared__ int en[2 * HP_RC], ea[2 * HP_RC], eq[2 * HP_RC + 1], ne_s;
-	for(int t = threadIdx.x; t < ncoef; t += HP_NT)
-		a[t] = alm[(size_t) s * ncoef + t];
+	typedef hm_ops<T> ops;
+	typedef T vec4 __attribute__((ext_vector_type(4)));
+	extern __shared__ __align__(16) unsigned char hm_sm[];
+	T *AB = reinterpret_cast<T *>(hm_sm);	/* [rc][16][ld], then the waves' fetches */
+	/* the chunks of a group of series run on one XCD, side by side */
+	const int id = blockIdx.x, grp = id / (8 * g.chunks) * 8 + id % 8, chunk = id / 8 % g.chunks;
+	if(grp >= g.groups)
+		return;
+	const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 15, lq = lane >> 4;
+	const int L = g.L, L1 = L + 1, s0 = grp * HM_S, r0 = chunk * g.rc, N2 = 2 * g.nside;
+	/* the columns past the orders multiply zeros of the table: finite */
+	for(int i = threadIdx.x; i < g.rc * g.rs / 4; i += HM_NT)
+		reinterpret_cast<vec4 *>(AB)[i] = (vec4) 0;
 	__syncthreads();
-	T *out = map + (size_t) s * npix;
-	for(int r0 = 1; r0 <= N2; r0 += HP_RC) {
-		const int nr = N2 - r0 + 1 < HP_RC ? N2 - r0 + 1 : HP_RC;
-		if(threadIdx.x == 0) {
-			int ne = 0;
-			eq[0] = 0;
-			for(int rr = 0; rr < nr; rr++)
-				for(int h = 0; h < 2; h++) {
-					/* ring r0 + rr and its mirror 4 nside - r0 - rr (the
-					 * equator ring is its own mirror) */
-					const int ring = h ? 4 * nside - r0 - rr : r0 + rr;
-					if(h && ring == r0 + rr)
+	{
+		constexpr int ST = ops::STEPS, CP = 8 * ST;	/* coefficients of a series per fetch */
+		typedef typename ops::piece piece;
+		/* this wave's fetches of a+ and a-: [2][8 series][8 pieces, piece q
+		 * at q ^ series: the series' reads fall on distinct banks] */
+		piece *stage = reinterpret_cast<piece *>(AB + (size_t) g.rc * g.rs) + wave * 128;
+		auto staged = [&](int h, int k) -> T {
+			return reinterpret_cast<const T *>(stage + 64 * h + (li >> 1) * 8 + ((k / ST) ^ (li >> 1)))[2 * (k % ST) + (li & 1)];
+		};
+		const int ring = r0 + li < N2 ? r0 + li : N2 - 1;	/* 0-based northern ring of operand row li */
+		const double *P = g.P + ((size_t) (ring >> 4) * g.steps * 64 + lq * 16 + (ring & 15));
+		const int comp = li & 1;
+		/* lane (series, piece): eight lanes read 128 consecutive bytes of
+		 * a series; fetches past an order's last l run into the next
+		 * order, past the series' last order they stay inside the array,
+		 * and their values are not used */
+		const long last = (long) g.n * L1 * L1 - ST;
+		const int fs = s0 + (lane >> 3) < g.n ? s0 + (lane >> 3) : g.n - 1;
+		const long fo = (long) fs * L1 * L1 + (lane & 7) * ST;
+		const T *a0 = reinterpret_cast<const T *>(alm), *af = a0 + 2 * fo;
+		struct fetch {
+			piece p, n;
+			double pe[ST], po[ST];
+		};
+		auto order = [&](int i) -> int { return HM_W * i + (i & 1 ? HM_W - 1 - wave : wave); };
+		auto piece_at = [&](int o) -> piece {
+			if(o + CP <= L1 * L1)
+				return *reinterpret_cast<const piece *>(af + 2 * o);
+			const long c = fo + o < last ? fo + o : last;
+			piece v = *reinterpret_cast<const piece *>(a0 + 2 * c);
+			if(ST == 2 && fo + o > last) {
+				/* the array's last coefficient alone */
+				v[0] = v[2 * (ST - 1)];
+				v[1] = v[2 * (ST - 1) + 1];
+			}
+			return v;
+		};
+		auto get = [&](int m, int tb) -> struct fetch {
+			struct fetch f;
+			f.p = piece_at(lm_offset(L, m, m) + tb * CP);
+			f.n = piece_at(lm_offset(L, m, -m) + tb * CP);
+			const int n = L - m, ke = (n / 2 + 4) / 4, ko = ((n + 1) / 2 + 3) / 4;
+			const double *Pe = P + (size_t) g.off[m] * 64, *Po = ko ? Pe + (size_t) ke * 64 : Pe;
+#pragma unroll
+			for(int u = 0; u < ST; u++) {
+				const int t = ST * tb + u;
+				f.pe[u] = Pe[(size_t) (t < ke ? t : ke - 1) * 64];
+				f.po[u] = Po[(size_t) (t < ko ? t : ko ? ko - 1 : 0) * 64];
+			}
+			return f;
+		};
+		int i = 0, tb = 0, m = order(0);
+		struct fetch f;
+		if(m <= L)
+			f = get(m, 0);
+		d4 E = (d4) 0, O = (d4) 0;
+		while(m <= L) {
+			stage[lane ^ (lane >> 3)] = f.p;
+			stage[64 + (lane ^ (lane >> 3))] = f.n;
+			double pe[ST], po[ST];
+#pragma unroll
+			for(int u = 0; u < ST; u++) {
+				pe[u] = f.pe[u];
+				po[u] = f.po[u];
+			}
+			/* the next fetch, in flight during this one's products */
+			const int mc = m, n = L - m, d0 = CP * tb;
+			const bool end = d0 + CP > n;
+			if(end) {
+				tb = 0;
+				m = order(++i);
+			} else
+				tb++;
+			if(m <= L)
+				f = get(m, tb);
+			__builtin_amdgcn_wave_barrier();
+			/* b = a+ + (-1)^m conj a-: re +-, im -+; m = 0: Re a */
+			const double sg = (mc & 1) != comp ? -1. : 1.;
+#pragma unroll
+			for(int u = 0; u < ST; u++) {
+				const int k = 2 * (4 * u + lq);
+				double be = (double) staged(0, k), bo = (double) staged(0, k + 1);
+				if(mc) {
+					be = fma(sg, (double) staged(1, k), be);
+					bo = fma(sg, (double) staged(1, k + 1), bo);
+				} else if(comp)
+					be = bo = 0.;
+				if(end) {
+					be = d0 + k <= n ? be : 0.;
+					bo = d0 + k < n ? bo : 0.;
+				}
+				E = hm_ops<double>::mma(pe[u], be, E);
+				O = hm_ops<double>::mma(po[u], bo, O);
+			}
+			__builtin_amdgcn_wave_barrier();
+			if(end) {
+				const int col = hm_col(g, mc) + comp;
+#pragma unroll
+				for(int e = 0; e < 4; e++) {
+					const int rr = lq + 4 * e;
+					if(rr < g.rc) {
+						T *o = AB + rr * g.rs + (li >> 1) * g.ld + col;
+						o[0] = (T) (E[e] + O[e]);
+						o[8 * g.ld] = (T) (E[e] - O[e]);
+					}
+				}
+				E = (d4) 0;
+				O = (d4) 0;
+			}
+		}
+	}
+	__syncthreads();
+	const long npix = 12L * g.nside * g.nside;
+	const int g0 = g.k0 / 8, g2 = g.k2 / 8, g1 = g.k1 / 8;
+	const size_t tile = (size_t) 64 * (g0 + g2 + 2 * g1);	/* pairs of one tile's table */
+	for(int rr = wave; rr < g.rc && r0 + rr < N2; rr += HM_W) {
+		const int ring = r0 + rr + 1, n4 = ring < g.nside ? ring : g.nside, nt = (n4 + 15) / 16;
+		const T *A = AB + rr * g.rs + li * g.ld + 2 * lq;
+		const typename ops::pair *Wr = reinterpret_cast<const typename ops::pair *>(W) + (size_t) g.off[L1 + ring] * tile + lane;
+		/* first pixels of the ring and of its mirror */
+		const long sn = ring < g.nside ? 2L * ring * (ring - 1) : 2L * g.nside * (g.nside - 1) + 4L * g.nside * (ring - g.nside);
+		const long ss = npix - sn - 4L * n4;
+		for(int t0 = 0; t0 < nt; t0 += 2) {
+			const typename ops::pair *w0 = Wr + (size_t) t0 * tile, *w1 = t0 + 1 < nt ? w0 + tile : w0;
+			typename ops::acc acc[2][4];
+#pragma unroll
+			for(int u = 0; u < 2; u++)
+#pragma unroll
+				for(int c = 0; c < 4; c++)
+					acc[u][c] = (typename ops::acc) 0;
+			/* groups in runs of HM_R, the run's table loads ahead of its
+			 * products; group k of all: S0, S2, then U and V in turn */
+			auto run = [&](int k0, int cnt, int col0, int c, int cs, int div) {
+				for(int k = 0; k < cnt; k += HM_R) {
+					typename ops::pair b0[HM_R], b1[HM_R], av[HM_R];
+#pragma unroll
+					for(int q = 0; q < HM_R; q++) {
+						const int kq = k + q < cnt ? k + q : cnt - 1;
+						b0[q] = w0[(size_t) (k0 + kq) * 64];
+						b1[q] = w1[(size_t) (k0 + kq) * 64];
+						av[q] = *reinterpret_cast<const typename ops::pair *>(A + col0 + 8 * (kq / div));
+					}
+#pragma unroll
+					for(int q = 0; q < HM_R; q++)
+						if(k + q < cnt) {
+							const int cc = c + (cs ? (q & 1) : 0);
+							acc[0][cc] = ops::mma(av[q].x, b0[q].x, acc[0][cc]);
+							acc[1][cc] = ops::mma(av[q].x, b1[q].x, acc[1][cc]);
+							acc[0][cc] = ops::mma(av[q].y, b0[q].y, acc[0][cc]);
+							acc[1][cc] = ops::mma(av[q].y, b1[q].y, acc[1][cc]);
+						}
+				}
+			};
+			run(0, g0, 0, 0, 0, 1);
+			run(g0, g2, g.k0, 1, 0, 1);
+			run(g0 + g2, 2 * g1, g.k0 + g.k2, 2, 1, 2);
+#pragma unroll
+			for(int u = 0; u < 2; u++) {
+				const int j = 16 * (t0 + u) + li;
+				if(j >= n4)
+					continue;
+#pragma unroll
+				for(int e = 0; e < 4; e++) {
+					const int row = ops::row(lq, e), ser = s0 + (row & 7);
+					const bool south = row >= 8;
+					if(ser >= g.n || (south && ring == N2))
 						continue;
-					double z, st, phi0;
-					int nphi;
-					long start;
-					hp_ring(nside, ring, &z, &st, &nphi, &start, &phi0);
-					es[ne] = start;
-					en[ne] = nphi;
-					ea[ne] = h ? HP_RC + rr : rr;
-					eq[ne + 1] = eq[ne] + nphi / 4;
-					ne++;
-				}
-			ne_s = ne;
-		}
-		/* Legendre sums: task (|m|, northern ring of the chunk), split by
-		 * the parity of l - m: Pbar_lm(-z) = (-1)^(l+m) Pbar_lm(z), so the
-		 * ring gets E + O and its mirror E - O */
-		for(int t = threadIdx.x; t < HP_RC * L1; t += HP_NT) {
-			const int m = t / HP_RC, rr = t - m * HP_RC;
-			double arn = 0., bin = 0., ars = 0., bis = 0.;
-			if(rr < nr) {
-				double z, st, phi0;
-				int nphi;
-				long start;
-				hp_ring(nside, r0 + rr, &z, &st, &nphi, &start, &phi0);
-				/* Pbar_mm = cm[m] sin^m theta, the power by squaring */
-				double p2 = cm[m], b = st;
-				for(int e = m; e; e >>= 1) {
-					if(e & 1)
-						p2 *= b;
-					b *= b;
-				}
-				const cplx<T> *ap = a + lm_offset(L, m, m);
-				const cplx<T> *an = m ? a + lm_offset(L, m, -m) : ap;
-				/* even (e) and odd (o) l - m sums of +m (p) and -m (n) */
-				double epr = (double) ap[0].re * p2, epi = (double) ap[0].im * p2;
-				double enr = (double) an[0].re * p2, eni = (double) an[0].im * p2;
-				double opr = 0., opi = 0., onr = 0., oni = 0.;
-				const double *c = cf + 2 * lm_offset(L, m, m);
-				double p1 = 0.;
-				if(m < L) {
-					p1 = c[2] * z * p2;
-					opr = (double) ap[1].re * p1;
-					opi = (double) ap[1].im * p1;
-					onr = (double) an[1].re * p1;
-					oni = (double) an[1].im * p1;
-				}
-				int d = 2;
-				for(; d + 1 <= L - m; d += 2) {
-					const double pe = c[2 * d] * z * p1 - c[2 * d + 1] * p2;
-					const double po = c[2 * d + 2] * z * pe - c[2 * d + 3] * p1;
-					epr = fma((double) ap[d].re, pe, epr);
-					epi = fma((double) ap[d].im, pe, epi);
-					enr = fma((double) an[d].re, pe, enr);
-					eni = fma((double) an[d].im, pe, eni);
-					opr = fma((double) ap[d + 1].re, po, opr);
-					opi = fma((double) ap[d + 1].im, po, opi);
-					onr = fma((double) an[d + 1].re, po, onr);
-					oni = fma((double) an[d + 1].im, po, oni);
-					p2 = pe;
-					p1 = po;
-				}
-				if(d <= L - m) {
-					const double pe = c[2 * d] * z * p1 - c[2 * d + 1] * p2;
-					epr = fma((double) ap[d].re, pe, epr);
-					epi = fma((double) ap[d].im, pe, epi);
-					enr = fma((double) an[d].re, pe, enr);
-					eni = fma((double) an[d].im, pe, eni);
-				}
-				double sn, cs;
-				sincos(m * phi0, &sn, &cs);
-				/* the ring (h = 0) and its mirror (h = 1): F = E +- O;
-				 * Pbar_l,-m = (-1)^m Pbar_lm; G_+-m = F_+-m exp(+-i m phi_0) */
-				for(int h = 0; h < 2; h++) {
-					const double sg = h ? -1. : 1.;
-					const double fpr = epr + sg * opr, fpi = epi + sg * opi;
-					double fnr = enr + sg * onr, fni = eni + sg * oni;
-					if(m & 1) {
-						fnr = -fnr;
-						fni = -fni;
-					}
-					const double gpr = fpr * cs - fpi * sn, gpi = fpr * sn + fpi * cs;
-					const double gnr = fnr * cs + fni * sn, gni = -fnr * sn + fni * cs;
-					const double ar = m ? gpr + gnr : gpr, bi = m ? gpi - gni : 0.;
-					if(h) {
-						ars = ar;
-						bis = bi;
-					} else {
-						arn = ar;
-						bin = bi;
-					}
+					T *o = map + (size_t) ser * npix + (south ? ss : sn) + j;
+					const T s = acc[u][0][e] + acc[u][1][e], d = acc[u][0][e] - acc[u][1][e], U = acc[u][2][e], V = acc[u][3][e];
+					o[0] = s + U;
+					o[n4] = d - V;
+					o[2 * n4] = s - U;
+					o[3 * n4] = d + V;
 				}
 			}
-			AB[2 * (rr * L1 + m)] = (T) arn;
-			AB[2 * (rr * L1 + m) + 1] = (T) bin;
-			AB[2 * ((HP_RC + rr) * L1 + m)] = (T) ars;
-			AB[2 * ((HP_RC + rr) * L1 + m) + 1] = (T) bis;
 		}
-		__syncthreads();
-		/* pixels of the chunk's rings, four at once: nphi is a multiple of
-		 * 4, and the pixels j + q nphi / 4 (q = 0..3) sit at phi' + q pi / 2,
-		 * where exp(i m (phi' + q pi / 2)) = i^(m q) exp(i m phi').  With
-		 * C_m = A_m cos(m phi') - B_m sin(m phi'),
-		 * D_m = A_m sin(m phi') + B_m cos(m phi') and S_k, T_k the sums
-		 * of C_m, D_m over m = k mod 4:
-		 *   q = 0: S0 + S1 + S2 + S3,   q = 1: S0 - T1 - S2 + T3,
-		 *   q = 2: S0 - S1 + S2 - S3,   q = 3: S0 + T1 - S2 - T3 */
-		const int ne = ne_s;
-		/* u only grows, so each thread's ring search resumes where its
-		 * last one stopped */
-		int k = 0;
-		for(int u = threadIdx.x; u < eq[ne]; u += HP_NT) {
-			while(k + 1 < ne && u >= eq[k + 1])
-				k++;
-			const int j = u - eq[k], n4 = en[k] / 4;
-			T sn, cs;
-			hp_sincospi(2 * j, en[k], &sn, &cs);
-			const T *ab = AB + 2 * ea[k] * L1;
-			const T er = cs, ei = sn;
-			T cr = er, ci = ei;	/* exp(i m phi') for m = 1 */
-			T s0 = ab[0], s1 = 0, s2 = 0, s3 = 0, t1 = 0, t3 = 0;
-			for(int m = 1; m <= L; m++) {
-				const T A = ab[2 * m], B = ab[2 * m + 1];
-				const T c = fma(A, cr, -B * ci);
-				switch(m & 3) {
-				case 0:
-					s0 += c;
-					break;
-				case 1:
-					s1 += c;
-					t1 = fma(A, ci, fma(B, cr, t1));
-					break;
-				case 2:
-					s2 += c;
-					break;
-				default:
-					s3 += c;
-					t3 = fma(A, ci, fma(B, cr, t3));
-					break;
-				}
-				const T nr_ = cr * er - ci * ei;
-				ci = fma(cr, ei, ci * er);
-				cr = nr_;
-			}
-			T *o = out + es[k] + j;
-			o[0] = (s0 + s2) + (s1 + s3);
-			o[n4] = (s0 - s2) - (t1 - t3);
-			o[2 * n4] = (s0 + s2) - (s1 + s3);
-			o[3 * n4] = (s0 - s2) + (t1 - t3);
-		}
-		__syncthreads();
 	}
 }
 
-/* orders whose coefficients do not fit in LDS: workgroup = one ring x
+/* the Legendre table: [16 rings][step][lane], the steps of an order those of
+ * its even l - m and then of its odd ones, lane i + 16 q of step t holding
+ * ring i at l - m = 2 (4 t + q) (+ 1); zeros past the last l and ring */
+__global__ void k_hm_legendre(int L, int nside, int steps, const int *__restrict__ off, const double *__restrict__ cf, const double *__restrict__ cm, double *__restrict__ P)
+{
+	const int ring = blockIdx.x * 16 + (threadIdx.x & 15), m = blockIdx.y * (blockDim.x / 16) + threadIdx.x / 16;
+	if(m > L)
+		return;
+	double z = 0., st = 0., phi0;
+	int nphi;
+	long start;
+	const bool in = ring < 2 * nside;
+	if(in)
+		hp_ring(nside, ring + 1, &z, &st, &nphi, &start, &phi0);
+	double p2 = in ? cm[m] : 0., b = st, p1 = 0.;
+	for(int e = m; e; e >>= 1) {
+		if(e & 1)
+			p2 *= b;
+		b *= b;
+	}
+	const int ke = ((L - m) / 2 + 4) / 4, ko = ((L - m + 1) / 2 + 3) / 4;
+	double *o = P + ((size_t) blockIdx.x * steps + off[m]) * 64 + (threadIdx.x & 15);
+	const double *c = cf + 2 * lm_offset(L, m, m);
+	for(int d = 0; d < 8 * ke || d < 8 * ko; d++) {
+		double v = 0.;
+		if(d == 0)
+			v = p2;
+		else if(d <= L - m) {
+			v = d == 1 ? c[2] * z * p2 : c[2 * d] * z * p1 - c[2 * d + 1] * p2;
+			if(d > 1)
+				p2 = p1;
+			p1 = v;
+		}
+		const int k = d >> 1, t = k >> 2;
+		if(d & 1) {
+			if(t < ko)
+				o[(size_t) (ke + t) * 64 + (k & 3) * 16] = v;
+		} else if(t < ke)
+			o[(size_t) t * 64 + (k & 3) * 16] = v;
+	}
+}
+
+/* the pixel table: per tile of 16 pixels of a quarter ring the groups of
+ * eight columns of S0, S2, then U and V in turn, [group][lane][2]: lane
+ * i + 16 q holds pixel i at columns 2 q, 2 q + 1 */
+template <typename T>
+__global__ void k_hm_pixels(struct hm_geom g, T *__restrict__ W)
+{
+	const int ring = blockIdx.x + 1, L1 = g.L + 1;
+	/* the rings past nside alternate between two tables: those of rings
+	 * nside and nside + 1 */
+	if(ring > g.nside + 1)
+		return;
+	const int n4 = ring < g.nside ? ring : g.nside, nt = (n4 + 15) / 16;
+	const int g0 = g.k0 / 8, g2 = g.k2 / 8, g1 = g.k1 / 8;
+	const long tile = 128L * (g0 + g2 + 2 * g1);
+	T *o = W + (size_t) g.off[L1 + ring] * tile;
+	const int half = ring < g.nside || !((ring + g.nside) & 1);	/* first pixel half a step in */
+	for(long i = threadIdx.x; i < nt * tile; i += blockDim.x) {
+		const int t = (int) (i / tile), r = (int) (i - t * tile);
+		const int grp = r / 128, lane = (r >> 1) & 63, j = 16 * t + (lane & 15);
+		const int col = 2 * (lane >> 4) + (r & 1), comp = col & 1;
+		int m, v = 0;
+		if(grp < g0)
+			m = 2 * (8 * grp + col - comp);
+		else if(grp < g0 + g2)
+			m = 2 + 2 * (8 * (grp - g0) + col - comp);
+		else {
+			v = (grp - g0 - g2) & 1;
+			m = 1 + 8 * ((grp - g0 - g2) >> 1) + col - comp;
+		}
+		T w = 0;
+		if(m <= g.L && j < n4) {
+			/* m phi = pi m (2 j + half) / (4 n4), the fraction reduced
+			 * exactly */
+			double sn, cs;
+			sincospi((double) ((long) m * (2 * j + half) % (8L * n4)) / (4. * n4), &sn, &cs);
+			if(!v)
+				w = (T) (comp ? -sn : cs);
+			else
+				w = (T) ((m & 2) ? -(comp ? cs : sn) : (comp ? cs : sn));
+		}
+		o[i] = w;
+	}
+}
+
+/* orders and resolutions without tables: workgroup = one ring x
  * HP_SPW series, the coefficients read from global memory, the ring's
  * twiddles in LDS at exact integer indices (m j mod nphi) */
 template <typename T>
@@ -374,63 +539,118 @@ __global__ void __launch_bounds__(HP_NT) k_healpix_ring(const cplx<T> *__restric
 	}
 }
 
-/* the posterior of the two beta skies of each event (RapidLocalization.py:
+/*
+ * The posterior of the two beta skies of each event (RapidLocalization.py:
  * 498-530): prob = (e_p / sum e_p + e_n / sum e_n) / 2, e = exp(map -
- * max map); maps [2][E][npix], one workgroup per event */
-template <typename T>
-__global__ void __launch_bounds__(HP_NT) k_healpix_posterior(const T *__restrict__ maps, int E, long npix, T *__restrict__ prob)
+ * max map); maps [2][E][npix], one workgroup of NT threads per event.  Two
+ * reads of the maps: the first keeps a running maximum and the sum relative
+ * to it per thread (rescaled when the maximum grows), the second forms the
+ * probabilities; the maps of the events in flight fit the last-level cache,
+ * so the second read is not one of HBM: 8192 events at nside 32 in float32
+ * 0.46 -> 0.30 ms (1.2 GB), nine at nside 64 in float64 with 1024 threads
+ * each 0.14 -> 0.065 ms.
+ *
+ * VW values per load: 16 bytes where the arrays are aligned for it (npix is
+ * a multiple of 12, so every event's row then is).
+ */
+template <typename T, int VW, int NT>
+__global__ void __launch_bounds__(NT) k_healpix_posterior(const T *__restrict__ maps, int E, long npix, T *__restrict__ prob)
 {
+	typedef T vec __attribute__((ext_vector_type(VW)));
 	/* exp(x - max) in the maps' precision (float32 maps: float32
 	 * exponentials, float64 sums) */
 	auto ex = [](T x, double m) -> double { return sizeof(T) == sizeof(float) ? (double) expf((float) ((double) x - m)) : exp((double) x - m); };
-	__shared__ double red[2][HP_NT / 64];
+	__shared__ double red[4][NT / 64];
 	const int e = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-	const T *mp = maps + (size_t) e * npix, *mn = maps + ((size_t) E + e) * npix;
-	double xp = -INFINITY, xn = -INFINITY;
-	for(long p = threadIdx.x; p < npix; p += HP_NT) {
-		xp = fmax(xp, (double) mp[p]);
-		xn = fmax(xn, (double) mn[p]);
+	const vec *mp = reinterpret_cast<const vec *>(maps + (size_t) e * npix), *mn = reinterpret_cast<const vec *>(maps + ((size_t) E + e) * npix);
+	const long nv = npix / VW;
+	double x[2] = { -INFINITY, -INFINITY }, s[2] = { 0., 0. };
+	auto take = [&](vec v, int k) {
+		T m = v[0];
+#pragma unroll
+		for(int i = 1; i < VW; i++)
+			m = v[i] > m ? v[i] : m;
+		if((double) m > x[k]) {
+			/* the first values come with s = 0; NaN stays */
+			s[k] = s[k] > 0. ? s[k] * exp(x[k] - (double) m) : s[k];
+			x[k] = m;
+		}
+		/* values of minus infinity ahead of the first finite one add
+		 * nothing, NaN does */
+#pragma unroll
+		for(int i = 0; i < VW; i++)
+			s[k] += x[k] > -INFINITY || v[i] != v[i] ? ex(v[i], x[k]) : 0.;
+	};
+	constexpr int U = 4;	/* loads of each map in flight */
+	long p = threadIdx.x;
+	for(; p + (U - 1) * NT < nv; p += U * NT) {
+		vec a[U], b[U];
+#pragma unroll
+		for(int u = 0; u < U; u++) {
+			a[u] = mp[p + u * NT];
+			b[u] = mn[p + u * NT];
+		}
+#pragma unroll
+		for(int u = 0; u < U; u++) {
+			take(a[u], 0);
+			take(b[u], 1);
+		}
 	}
-	for(int o = 32; o; o >>= 1) {
-		xp = fmax(xp, __shfl_xor(xp, o));
-		xn = fmax(xn, __shfl_xor(xn, o));
+	for(; p < nv; p += NT) {
+		take(mp[p], 0);
+		take(mn[p], 1);
 	}
-	if(!lane) {
-		red[0][wave] = xp;
-		red[1][wave] = xn;
+	double xm[2], ip[2];
+#pragma unroll
+	for(int k = 0; k < 2; k++) {
+		double m = x[k];
+		for(int o = 32; o; o >>= 1)
+			m = fmax(m, __shfl_xor(m, o));
+		if(!lane)
+			red[k][wave] = m;
 	}
 	__syncthreads();
-	xp = red[0][0];
-	xn = red[1][0];
-	for(int w = 1; w < HP_NT / 64; w++) {
-		xp = fmax(xp, red[0][w]);
-		xn = fmax(xn, red[1][w]);
+#pragma unroll
+	for(int k = 0; k < 2; k++) {
+		xm[k] = red[k][0];
+		for(int w = 1; w < NT / 64; w++)
+			xm[k] = fmax(xm[k], red[k][w]);
+		/* a thread without pixels has nothing to add */
+		double t = s[k] > 0. ? s[k] * exp(x[k] - xm[k]) : s[k];
+		for(int o = 32; o; o >>= 1)
+			t += __shfl_xor(t, o);
+		if(!lane)
+			red[2 + k][wave] = t;
 	}
 	__syncthreads();
-	double sp = 0., sn = 0.;
-	for(long p = threadIdx.x; p < npix; p += HP_NT) {
-		sp += ex(mp[p], xp);
-		sn += ex(mn[p], xn);
+#pragma unroll
+	for(int k = 0; k < 2; k++) {
+		double t = 0.;
+		for(int w = 0; w < NT / 64; w++)
+			t += red[2 + k][w];
+		ip[k] = 0.5 / t;
 	}
-	for(int o = 32; o; o >>= 1) {
-		sp += __shfl_xor(sp, o);
-		sn += __shfl_xor(sn, o);
+	vec *pr = reinterpret_cast<vec *>(prob + (size_t) e * npix);
+	auto put = [&](long q, vec a, vec b) {
+		vec o;
+#pragma unroll
+		for(int i = 0; i < VW; i++)
+			o[i] = (T) (ex(a[i], xm[0]) * ip[0] + ex(b[i], xm[1]) * ip[1]);
+		pr[q] = o;
+	};
+	for(p = threadIdx.x; p + (U - 1) * NT < nv; p += U * NT) {
+		vec a[U], b[U];
+#pragma unroll
+		for(int u = 0; u < U; u++) {
+			a[u] = mp[p + u * NT];
+			b[u] = mn[p + u * NT];
+		}
+#pragma unroll
+		for(int u = 0; u < U; u++)
+			put(p + u * NT, a[u], b[u]);
 	}
-	if(!lane) {
-		red[0][wave] = sp;
-		red[1][wave] = sn;
-	}
-	__syncthreads();
-	sp = 0.;
-	sn = 0.;
-	for(int w = 0; w < HP_NT / 64; w++) {
-		sp += red[0][w];
-		sn += red[1][w];
-	}
-	const double ip = 0.5 / sp, in = 0.5 / sn;
-	T *pr = prob + (size_t) e * npix;
-	for(long p = threadIdx.x; p < npix; p += HP_NT)
-		pr[p] = (T) (ex(mp[p], xp) * ip + ex(mn[p], xn) * in);
+	for(; p < nv; p += NT)
+		put(p, mp[p], mn[p]);
 }
 
 /* ---------------------------------------------------------------- C ABI */
@@ -443,6 +663,81 @@ extern "C" int sphr_healpix_nside(unsigned l_max)
 		if(i >= x)
 			return i;
 	return -1;
+}
+
+static struct hm_geom hm_geom_of(const struct sphr_healpix *h, int n)
+{
+	struct hm_geom g;
+	memset(&g, 0, sizeof(g));
+	g.L = h->L;
+	g.nside = h->nside;
+	g.n = n;
+	g.rc = h->rc;
+	g.k0 = h->k0;
+	g.k2 = h->k2;
+	g.k1 = h->k1;
+	/* row strides whose 16 rows start on distinct banks */
+	const int f = h->precision == SPHR_MIXED;
+	g.ld = h->k0 + h->k2 + h->k1 + (f ? 4 : 2);
+	g.rs = 16 * g.ld + (f ? 16 : 8);
+	g.steps = h->steps;
+	g.chunks = h->rc ? (2 * h->nside + h->rc - 1) / h->rc : 0;
+	g.groups = (n + HM_S - 1) / HM_S;
+	g.P = h->P;
+	g.off = h->off;
+	return g;
+}
+
+/* the tables of k_healpix_mm; left out, for the recurrences of
+ * k_healpix_ring, where they would pass 512 MB or one ring's operand does
+ * not fit in LDS */
+template <typename T>
+static int build_mm(struct sphr_healpix *h)
+{
+	const int L = h->L, ns = h->nside, n0 = L / 4 + 1, n2 = L >= 2 ? (L - 2) / 4 + 1 : 0, n1 = (L + 1) / 2;
+	h->k0 = (2 * n0 + 7) / 8 * 8;
+	h->k2 = (2 * n2 + 7) / 8 * 8;
+	h->k1 = (2 * n1 + 7) / 8 * 8;
+	struct hm_geom g = hm_geom_of(h, 1);
+	int rc = 16;
+	while(rc && (size_t) rc * g.rs * sizeof(T) + HM_STAGE > 160 * 1024)
+		rc >>= 1;
+	int *off = (int *) malloc((L + 1 + 2 * (size_t) ns + 1) * sizeof(int));
+	if(!off) {
+		sphr_set_error("sphr_healpix_new: out of memory");
+		return -1;
+	}
+	long steps = 0, tiles = 0;
+	for(int m = 0; m <= L; m++) {
+		off[m] = (int) steps;
+		steps += ((L - m) / 2 + 4) / 4 + ((L - m + 1) / 2 + 3) / 4;
+	}
+	off[L + 1] = 0;
+	for(int r = 1; r <= 2 * ns; r++) {
+		off[L + 1 + r] = r > ns + 1 ? off[L + 1 + r - 2] : (int) tiles;
+		if(r <= ns + 1)
+			tiles += ((r < ns ? r : ns) + 15) / 16;
+	}
+	const size_t bP = (size_t) ((2 * ns + 15) / 16) * steps * 64 * sizeof(double);
+	const size_t bW = (size_t) tiles * 16 * (h->k0 + h->k2 + 2 * h->k1) * sizeof(T);
+	/* order 0 has no second coefficient to fetch */
+	if(!rc || L == 0 || bP + bW > (size_t) 512 << 20) {
+		free(off);
+		return 0;
+	}
+	h->rc = rc;
+	h->steps = (int) steps;
+	hipStream_t st = sphr_rt_stream();
+	int bad = sphr_rt_check(hipMalloc(&h->P, bP), "hipMalloc") || sphr_rt_check(hipMalloc(&h->W, bW), "hipMalloc")
+		  || sphr_rt_check(hipMalloc(&h->off, (L + 1 + 2 * (size_t) ns + 1) * sizeof(int)), "hipMalloc")
+		  || sphr_rt_check(hipMemcpy(h->off, off, (L + 1 + 2 * (size_t) ns + 1) * sizeof(int), hipMemcpyHostToDevice), "hipMemcpy");
+	free(off);
+	if(bad)
+		return -1;
+	hipLaunchKernelGGL(k_hm_legendre, dim3((2 * ns + 15) / 16, (L + 16) / 16), dim3(256), 0, st, L, ns, (int) steps, h->off, h->d_cf, h->d_cm, h->P);
+	g = hm_geom_of(h, 1);
+	hipLaunchKernelGGL((k_hm_pixels<T>), dim3(ns + 1), dim3(256), 0, st, g, (T *) h->W);
+	return sphr_rt_check(hipGetLastError(), "healpix tables") || sphr_rt_check(hipStreamSynchronize(st), "healpix tables") ? -1 : 0;
 }
 
 extern "C" struct sphr_healpix *sphr_healpix_new(unsigned l_max, int nside, int precision)
@@ -488,6 +783,10 @@ extern "C" struct sphr_healpix *sphr_healpix_new(unsigned l_max, int nside, int 
 	}
 	h->d_cm = h->d_cf + 2 * (size_t) nal;
 	free(hc);
+	if(precision == SPHR_MIXED ? build_mm<float>(h) : build_mm<double>(h)) {
+		sphr_healpix_free(h);
+		return NULL;
+	}
 	return h;
 }
 
@@ -495,8 +794,10 @@ extern "C" void sphr_healpix_free(struct sphr_healpix *h)
 {
 	if(!h)
 		return;
-	if(h->d_cf)
-		hipFree(h->d_cf);
+	void *p[] = { h->d_cf, h->P, h->W, h->off };
+	for(unsigned i = 0; i < sizeof(p) / sizeof(p[0]); i++)
+		if(p[i])
+			hipFree(p[i]);
 	free(h);
 }
 
@@ -515,13 +816,14 @@ extern "C" int sphr_healpix_maps(const struct sphr_healpix *h, const void *alm, 
 		return 0;
 	hipStream_t st = stream ? (hipStream_t) stream : sphr_rt_stream();
 	const size_t esz = h->precision == SPHR_MIXED ? sizeof(float) : sizeof(double);
-	const size_t lds = (2 * (size_t) (h->L + 1) * (h->L + 1) + 4 * HP_RC * (size_t) (h->L + 1)) * esz;
-	if(lds <= 150 * 1024) {
-		/* one workgroup per series, its coefficients in LDS */
+	if(h->rc) {
+		const struct hm_geom g = hm_geom_of(h, n);
+		const unsigned grid = (unsigned) ((g.groups + 7) / 8 * 8) * g.chunks;
+		const size_t lds = (size_t) g.rc * g.rs * esz + HM_STAGE;
 		if(h->precision == SPHR_MIXED)
-			hipLaunchKernelGGL(k_healpix<float>, dim3(n), dim3(HP_NT), lds, st, (const cplx<float> *) alm, n, h->L, h->nside, h->d_cf, h->d_cm, (float *) map);
+			hipLaunchKernelGGL(k_healpix_mm<float>, dim3(grid), dim3(HM_NT), lds, st, (const cplx<float> *) alm, g, (const float *) h->W, (float *) map);
 		else
-			hipLaunchKernelGGL(k_healpix<double>, dim3(n), dim3(HP_NT), lds, st, (const cplx<double> *) alm, n, h->L, h->nside, h->d_cf, h->d_cm, (double *) map);
+			hipLaunchKernelGGL(k_healpix_mm<double>, dim3(grid), dim3(HM_NT), lds, st, (const cplx<double> *) alm, g, (const double *) h->W, (double *) map);
 	} else {
 		/* one workgroup per (ring, HP_SPW series) */
 		const size_t lr = (2 * HP_SPW * (size_t) (h->L + 1) + 2 * 4 * (size_t) h->nside) * esz;
@@ -538,6 +840,24 @@ extern "C" int sphr_healpix_maps(const struct sphr_healpix *h, const void *alm, 
 	return sphr_rt_check(hipGetLastError(), "k_healpix") ? -1 : 0;
 }
 
+/* 1024 threads per event where the events are too few to fill the chip with
+ * smaller workgroups (one per CU) */
+template <typename T>
+static void launch_posterior(const T *maps, int E, long npix, T *prob, hipStream_t st)
+{
+	constexpr int V = 16 / sizeof(T);
+	const bool al = ((uintptr_t) maps | (uintptr_t) prob) % 16 == 0;
+	const bool few = E <= 2 * sphr_rt_cus();
+	if(few && al)
+		hipLaunchKernelGGL((k_healpix_posterior<T, V, 1024>), dim3(E), dim3(1024), 0, st, maps, E, npix, prob);
+	else if(few)
+		hipLaunchKernelGGL((k_healpix_posterior<T, 1, 1024>), dim3(E), dim3(1024), 0, st, maps, E, npix, prob);
+	else if(al)
+		hipLaunchKernelGGL((k_healpix_posterior<T, V, 256>), dim3(E), dim3(256), 0, st, maps, E, npix, prob);
+	else
+		hipLaunchKernelGGL((k_healpix_posterior<T, 1, 256>), dim3(E), dim3(256), 0, st, maps, E, npix, prob);
+}
+
 extern "C" int sphr_healpix_posterior(const struct sphr_healpix *h, const void *maps, int n_events, void *prob, void *stream)
 {
 	if(!h || !maps || !prob || n_events < 0) {
@@ -549,9 +869,9 @@ extern "C" int sphr_healpix_posterior(const struct sphr_healpix *h, const void *
 	hipStream_t st = stream ? (hipStream_t) stream : sphr_rt_stream();
 	const long npix = 12L * h->nside * h->nside;
 	if(h->precision == SPHR_MIXED)
-		hipLaunchKernelGGL(k_healpix_posterior<float>, dim3(n_events), dim3(HP_NT), 0, st, (const float *) maps, n_events, npix, (float *) prob);
+		launch_posterior<float>((const float *) maps, n_events, npix, (float *) prob, st);
 	else
-		hipLaunchKernelGGL(k_healpix_posterior<double>, dim3(n_events), dim3(HP_NT), 0, st, (const double *) maps, n_events, npix, (double *) prob);
+		launch_posterior<double>((const double *) maps, n_events, npix, (double *) prob, st);
 	return sphr_rt_check(hipGetLastError(), "k_healpix_posterior") ? -1 : 0;
 }
 

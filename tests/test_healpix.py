@@ -238,6 +238,59 @@ def test_gpu_healpix_maps_match_oracle(oracle, L, nside):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("L,nside,n", [(1, 4, 1), (2, 3, 7), (3, 17, 8), (16, 9, 9), (31, 20, 17), (63, 33, 2), (64, 16, 65), (129, 40, 3), (520, 2, 2)])
+def test_gpu_healpix_series_counts_and_tiles(oracle, L, nside, n):
+    """groups of eight series with remainders, rings on both sides of the
+    16-pixel tiles and 16-ring chunks, every number of rings per workgroup
+    (the LDS operand of l_max 31 to 129) and the per-ring form (l_max 520,
+    whose operand does not fit); the first, the last and a middle series"""
+    print("healpix tiles L", L, "nside", nside, "n", n, flush=True)
+    rng = np.random.default_rng(L + 7 * n)
+    series = [rand_series(rng, L) for _ in range(n)]
+    m64 = _gpu_maps(series, L, nside, S.FP64)
+    m32 = _gpu_maps(series, L, nside, S.MIXED)
+    for k in sorted({0, n // 2, n - 1}):
+        ref = oracle.healpix_map(series[k], L, nside)
+        assert rel(m64[k], ref) < TOL64, (k, rel(m64[k], ref))
+        ref32 = oracle.healpix_map(series[k].astype(np.complex64).astype(np.complex128), L, nside)
+        assert rel(m32[k], ref32) < TOL_MIXED, (k, rel(m32[k], ref32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", [S.FP64, S.MIXED])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_gpu_posterior_special_values(prec, shift):
+    """maps with minus infinities (zero probability), a map of them alone
+    and maps with NaN (NaN), on arrays that start off 16 bytes too, few
+    events and many"""
+    rdt = np.float64 if prec == S.FP64 else np.float32
+    rng = np.random.default_rng(5)
+    for E in (4, 600):
+        hp = S.Healpix(4, 4, prec)
+        m = rng.standard_normal((2, E, hp.npix)) * 5
+        m[0, 0, :150] = -np.inf
+        m[1, 1, ::3] = -np.inf
+        m[0, 2] = -np.inf
+        m[1, 3, 100] = np.nan
+        m = m.astype(rdt)
+        d_m = S.DeviceBuffer(m.nbytes + 16)
+        d_p = S.DeviceBuffer(m.nbytes // 2 + 16)
+        off = shift * m.itemsize
+        d_m.upload(m, offset=off)
+        print("posterior special values", prec, shift, E, flush=True)
+        hp.posterior(d_m.ptr + off, E, d_p.ptr + off)
+        S.synchronize()
+        p = d_p.to_numpy(rdt, (E, hp.npix), offset=off)
+        with np.errstate(invalid="ignore"):
+            x = m.astype(np.float64)
+            e = np.exp(x - np.max(x, axis=2, keepdims=True))
+            ref = (e[0] / e[0].sum(1, keepdims=True) + e[1] / e[1].sum(1, keepdims=True)) / 2
+        assert np.all(np.isnan(p[2])) and np.all(np.isnan(p[3]))
+        ok = [k for k in range(E) if k not in (2, 3)]
+        assert rel(p[ok], ref[ok]) < (TOL64 if prec == S.FP64 else TOL_MIXED)
+
+
+@pytest.mark.gpu
 def test_gpu_write_healpix_map_file(tmp_path, oracle):
     rng = np.random.default_rng(11)
     for L, polar in ((13, False), (9, True)):
