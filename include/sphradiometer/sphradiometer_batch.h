@@ -242,16 +242,18 @@ int sphr_batch_set_shape(struct sphr_batch *, int index);
 
 /* Shape information: [0] detectors, [1] baselines, [2] N, [3] sky l_max,
  * [4] projection columns, [5] K splits, [6] precision, [7] K per split,
- * [8] 1 when the sky stage runs as the one fused kernel (orders it is
- * compiled for), 0 for the two-kernel form, [9] projection tiles per wave,
+ * [8] 1 when the sky stage runs as the fused kernel compiled for the
+ * order, 0 otherwise (the one-kernel form for any order where the plan
+ * gives real skies, else the two-kernel form), [9] projection tiles per wave,
  * [10] projection segments per workgroup, [11] fused sky workgroups per
  * CU requested (1-3, picked by the autotuner), [12] fused sky segments per
  * workgroup requested (0 for the precision's default, 1, 2 or 4) */
 void sphr_batch_info(const struct sphr_batch *, int info[13]);
 
-/* Select the sky stage's form: 1 (default) the fused kernel where it is
- * compiled for the batch's order, 0 the two-kernel form (a_lm and ring
- * sums, then the phi DFT as a GEMM).  Both give the same results to
+/* Select the sky stage's form: 1 (default) one kernel (the fused one where
+ * it is compiled for the batch's order, else its form for any order where
+ * the plan gives real skies), 0 the two-kernel
+ * form (a_lm and ring sums, then the phi DFT as a GEMM).  Both give the same results to
  * rounding. */
 void sphr_batch_set_fused(struct sphr_batch *, int on);
 /* Fused sky kernel's persistent workgroups per CU: 1 (default), 2 (the

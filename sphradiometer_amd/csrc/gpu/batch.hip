@@ -43,13 +43,14 @@ struct sphr_batch {
 	int sky_nsub;			/* fused sky segments per workgroup, 0 (default), 1, 2 or 4 (autotuned) */
 	int ksplit_opt[4], nsplit_opt[4];	/* K-split candidates: 1, 2, 4 x CUs workgroups, 64 per split */
 	int shape;			/* the projection shape index in use (sphr_batch_set_shape) */
+	int real;			/* the plan gives real skies (checked) */
 	int lag_ok, lag;		/* lag-domain route built / in use */
 	size_t m_bytes;			/* its table's bytes */
 	int xc_forms, xc_form;		/* its kernel forms (bit f - 1 for form f), the one in use (autotuned) */
 	struct xproj_geom g;
 	struct xcorr_geom xg;
 	struct synth_dev syn;
-	void *W, *R, *tw, *spec, *partial, *F, *M, *twW;
+	void *W, *R, *tw, *spec, *partial, *F, *M, *twW, *Wany;
 	int *col_bl;
 	int2 *lm;
 	int profile;
@@ -87,9 +88,14 @@ static int build_tables(struct sphr_batch *bt, const struct sphr_net_desc *d)
 	T *tw = (T *) malloc(2 * (size_t) N * sizeof(T));
 	double *twd = (double *) malloc(2 * (size_t) N * sizeof(double));
 	int rc = -1;
+	/* real skies: every projected column real (no imaginary column of W)
+	 * and rotation rows with R_l,-m = (-1)^m conj R_lm */
+	bt->real = 1;
+	const double rtol = sizeof(T) == 4 ? 1e-9 : 1e-12;	/* the rotation rows' recursion loses digits with l */
 	if(!W || !R || !tw || !twd)
 		goto done;
 	for(int b = 0; b < nb; b++) {
+		double big = 0.0, imag = 0.0;
 		const int Lb = d->Lb[b], c0 = bt->g.col_start[b];
 		const double *dp = d->dp[b];		/* N x (Lb+1) complex */
 		for(int f = 0; f < Nh; f++) {
@@ -102,6 +108,9 @@ static int build_tables(struct sphr_batch *bt, const struct sphr_net_desc *d)
 				/* G = a + b, H = i (a - b) */
 				const double gr = ar + br, gi = ai + bi;
 				const double hr = -(ai - bi), hi = ar - br;
+				/* (bins 0 and N/2 of real data have no imaginary part) */
+				big = fmax(big, fabs(gr));
+				imag = fmax(imag, self ? fabs(gi) : fmax(fabs(gi), fabs(hi)));
 				W[(size_t) (2 * f) * CT + c0 + 2 * l] = (T) (gr / N);
 				W[(size_t) (2 * f) * CT + c0 + 2 * l + 1] = (T) (gi / N);
 				W[(size_t) (2 * f + 1) * CT + c0 + 2 * l] = (T) (hr / N);
@@ -112,10 +121,16 @@ static int build_tables(struct sphr_batch *bt, const struct sphr_net_desc *d)
 		 * baselines (correlator.c:1004) */
 		T *Rb = R + 2 * ncoef * b;
 		Rb[0] = (T) (1.0 / nb);
+		if(!(imag <= 1e-12 * big))
+			bt->real = 0;
 		for(int l = 1; l <= Lb; l++)
 			for(int mp = -l; mp <= l; mp++) {
 				const size_t src = block_offset_h(l) + (size_t) (2 * l + 1) * (mp + l) + l;
 				const int dst = lm_offset(L, l, mp);
+				const size_t mir = block_offset_h(l) + (size_t) (2 * l + 1) * (l - mp) + l;
+				const double sg = (mp & 1) ? -1.0 : 1.0;
+				if(!(fabs(d->blocks[b][2 * src] - sg * d->blocks[b][2 * mir]) <= rtol) || !(fabs(d->blocks[b][2 * src + 1] + sg * d->blocks[b][2 * mir + 1]) <= rtol))
+					bt->real = 0;
 				Rb[2 * dst] = (T) (d->blocks[b][2 * src] / nb);
 				Rb[2 * dst + 1] = (T) (d->blocks[b][2 * src + 1] / nb);
 			}
@@ -271,7 +286,7 @@ extern "C" void sphr_batch_free(struct sphr_batch *bt)
 {
 	if(!bt)
 		return;
-	void *ptrs[] = { bt->W, bt->R, bt->tw, bt->spec, bt->partial, bt->col_bl, bt->lm, bt->F, bt->M, bt->twW };
+	void *ptrs[] = { bt->W, bt->R, bt->tw, bt->spec, bt->partial, bt->col_bl, bt->lm, bt->F, bt->M, bt->twW, bt->Wany };
 	for(unsigned i = 0; i < sizeof(ptrs) / sizeof(ptrs[0]); i++)
 		if(ptrs[i])
 			hipFree(ptrs[i]);
@@ -383,6 +398,14 @@ extern "C" struct sphr_batch *sphr_batch_create(const struct sphr_net_desc *d, u
 		goto fail;
 	if(synth_tables_build(bt->L, &bt->syn))
 		goto fail;
+	if(bt->real) {
+		hipStream_t st = sphr_rt_stream();
+		const size_t bytes = precision == SPHR_MIXED ? sky_any_table_bytes<float>(bt->L) : sky_any_table_bytes<double>(bt->L);
+		if(sphr_rt_check(hipMalloc(&bt->Wany, bytes), "hipMalloc")
+		   || (precision == SPHR_MIXED ? sky_any_table<float>(bt->L, bt->syn.twp, (float *) bt->Wany, st) : sky_any_table<double>(bt->L, bt->syn.twp, (double *) bt->Wany, st))
+		   || sphr_rt_check(hipStreamSynchronize(st), "sky table"))
+			goto fail;
+	}
 	if(sphr_rt_check(hipMalloc(&bt->spec, (size_t) bt->D * max_segments * bt->Nh * 2 * esz), "hipMalloc spectra")
 	   || sphr_rt_check(hipMalloc(&bt->partial, (size_t) bt->nsplit_opt[3] * max_segments * CT * esz), "hipMalloc partials")
 	   || sphr_rt_check(hipMalloc(&bt->F, (size_t) max_segments * 2 * (bt->L + 1) * (2 * bt->L + 1) * 2 * esz), "hipMalloc ring sums"))
@@ -422,10 +445,18 @@ static int run_t(struct sphr_batch *bt, void *spec, void *partial, void *F, cons
 			hipEventRecord(ev[2], st);
 	}
 	const int nsplit = bt->lag ? 1 : bt->nsplit;
-	/* the fused sky kernel at the orders it is compiled for; else a_lm
-	 * and ring sums, then the phi DFT as a GEMM; the one-kernel form when
-	 * the coefficients do not fit the LDS budget */
-	if(bt->fused && launch_sky_fused<T>((const T *) partial, nsplit, S, &bt->g, (const cplx<T> *) bt->R, bt->lm, gmst, &bt->syn.g, &bt->syn.tb, (cplx<T> *) alm, (cplx<T> *) map, st, bt->sky_occ, bt->sky_nsub) == 0) {
+	/* the fused sky kernel at the orders it is compiled for, its form for
+	 * any order where the plan gives real skies; else a_lm and ring sums,
+	 * then the phi DFT as a GEMM; the one-kernel form when the
+	 * coefficients do not fit the LDS budget */
+	/* (at the fused kernel's orders few segments would run faster here,
+	 * 24.9 against 28.1 us at two sites and 16 segments, but its forms
+	 * give the same bits and this kernel's sums run in another order) */
+	const bool any = bt->fused && bt->real && !sky_fused_order(bt->L);
+	if(any && launch_sky_any<T>((const T *) partial, nsplit, S, &bt->g, (const cplx<T> *) bt->R, bt->lm, gmst, bt->L, &bt->syn.tb, (const T *) bt->Wany, (cplx<T> *) alm, (cplx<T> *) map, st) == 0) {
+		if(ev)
+			hipEventRecord(ev[3], st);
+	} else if(bt->fused && launch_sky_fused<T>((const T *) partial, nsplit, S, &bt->g, (const cplx<T> *) bt->R, bt->lm, gmst, &bt->syn.g, &bt->syn.tb, (cplx<T> *) alm, (cplx<T> *) map, st, bt->sky_occ, bt->sky_nsub) == 0) {
 		if(ev)
 			hipEventRecord(ev[3], st);
 	} else if((F || !map) && launch_sky_lf<T>((const T *) partial, nsplit, S, &bt->g, (const cplx<T> *) bt->R, bt->lm, gmst, &bt->syn.g, &bt->syn.tb, (cplx<T> *) alm, map ? (cplx<T> *) F : (cplx<T> *) NULL, st) == 0) {

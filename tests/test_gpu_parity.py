@@ -494,3 +494,52 @@ def test_batch_full_size_three_site_properties(three_site):
     err = np.linalg.norm(almm - alm, axis=1) / np.linalg.norm(alm, axis=1)
     print("mixed a_lm rel err: max %.3g median %.3g; map %.3g" % (err.max(), np.median(err), rel(mpm, mp)), flush=True)
     assert err.max() < TOL_MIXED
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L,nseg", [(1, 1), (2, 3), (7, 2), (8, 130), (15, 3), (16, 5), (24, 7), (31, 2), (31, 128), (33, 600), (47, 3), (48, 2), (64, 2), (90, 2)])
+def test_gpu_sky_any_order_matches_two_kernel_form(L, nseg):
+    """the one-kernel sky stage for any order against the two-kernel form:
+    edges of its ring groups (8), point tiles (16) and column groups, every
+    split of a segment over workgroups, a GMST per segment, a_lm alone"""
+    net = S.Network(inject.positions("ABC"), 512, 1.0 / 4096, L)
+    rng = np.random.default_rng(L + nseg)
+    ts, gm = rng.standard_normal((3, nseg, 512)), rng.uniform(0, 6, nseg)
+    d_ts, d_g = S.DeviceBuffer.from_numpy(ts), S.DeviceBuffer.from_numpy(gm)
+    n, nc = 2 * L + 2, (L + 1) ** 2
+    for prec, cdt, tol in ((S.FP64, np.complex128, 1e-12), (S.MIXED, np.complex64, 3e-6)):
+        print(f"sky any order L={L} segments={nseg} precision={prec}", flush=True)
+        b = S.Batch(net, L, prec, max_segments=nseg)
+        out = []
+        for fused in (True, False):
+            b.set_fused(fused)
+            d_a, d_m = S.DeviceBuffer(nseg * nc * np.dtype(cdt).itemsize), S.DeviceBuffer(nseg * n * n * np.dtype(cdt).itemsize)
+            b.run(d_ts.ptr, nseg, d_a.ptr, d_m.ptr, d_gmst=d_g.ptr)
+            S.synchronize()
+            out.append((d_a.to_numpy(cdt, (nseg, nc)), d_m.to_numpy(cdt, (nseg, n, n))))
+        assert rel(out[0][0], out[1][0]) < tol and rel(out[0][1], out[1][1]) < tol, (rel(out[0][0], out[1][0]), rel(out[0][1], out[1][1]))
+        b.set_fused(True)
+        b.run(d_ts.ptr, nseg, d_a.ptr, None, d_gmst=d_g.ptr)
+        S.synchronize()
+        assert rel(d_a.to_numpy(cdt, (nseg, nc)), out[1][0]) < tol
+
+
+@pytest.mark.gpu
+def test_gpu_sky_of_a_plan_that_is_not_real():
+    """a delay product scaled by a complex number gives complex skies: the
+    stages for real skies are not taken, the imaginary parts stay"""
+    L, nseg = 20, 4
+    net = S.Network(inject.positions("ABC"), 512, 1.0 / 4096, L)
+    S.array_view(net.baseline_plan(1).contents.delay_product)[:] *= 0.6 + 0.8j
+    rng = np.random.default_rng(2)
+    d_ts = S.DeviceBuffer.from_numpy(rng.standard_normal((3, nseg, 512)))
+    b = S.Batch(net, L, S.FP64, max_segments=nseg)
+    maps = []
+    for fused in (True, False):
+        b.set_fused(fused)
+        d_a, d_m = S.DeviceBuffer(nseg * (L + 1) ** 2 * 16), S.DeviceBuffer(nseg * (2 * L + 2) ** 2 * 16)
+        b.run(d_ts.ptr, nseg, d_a.ptr, d_m.ptr)
+        S.synchronize()
+        maps.append(d_m.to_numpy(np.complex128, (nseg, 2 * L + 2, 2 * L + 2)))
+    assert np.linalg.norm(maps[1].imag) > 0.1 * np.linalg.norm(maps[1].real)
+    assert rel(maps[0], maps[1]) < 1e-13
