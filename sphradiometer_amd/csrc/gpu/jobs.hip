@@ -45,6 +45,7 @@ struct jb_bl {
 	double r_dt, theta, phi, inv_nb, scale;	/* scale = 1 / N^2 */
 	long off_nt, off_nq;		/* node arrays (x then w) in the chunk's node buffer */
 	long off_Pt, off_Pq, off_C, off_T, off_K, off_Y, off_F;	/* chunk workspace (doubles) */
+	int ldq;			/* row stride of Pq */
 	long off_M, off_R, off_c, off_pw;	/* persistent: M (T), R (cplx T), c (T), power slot */
 };
 
@@ -89,16 +90,21 @@ __device__ inline double sinc_pi(double x)
 }
 
 /*
- * Per baseline, over the first half of each (mirror-symmetric) rule:
- * Pbar_l0 at the tap nodes (Pt[j][l], j < nt/2, l <= a) and at the
- * product nodes (Pq[q][l], q < (nq+1)/2, l <= max(a, Lt)); the delay
- * table of the tap nodes: y_j = r_dt cos(acos x_j) (the delay of node j
- * in samples, projection.c:99-107), g_j = sin(pi y_j) nt (2 pi w_j / nt)
- * / pi and the weight 2 pi w_j / nt; the product-rule weights.
- * Y = [y | g | weight] (nt/2 each) then (nq+1)/2 product weights.
+ * Legendre tables over the first half of each (mirror-symmetric) rule:
+ * Pbar_l0 at the tap nodes (Pt[j][l], j < nt/2, l <= a) and at the product
+ * nodes (Pq[q][l], q < (nq+1)/2).  They depend on the rule alone, and the
+ * baselines of a chunk (about two thousand) have a few hundred rules between
+ * them, so each is made once per chunk and shared: 13 GB of tables for
+ * 20,430 baselines were 2.4, 5.7 -> 1.1 ms per plan, and the products'
+ * right operands stay in the caches.  One workgroup per table.
  */
+struct pg_table {
+	long off_x, off;	/* nodes; the table in the workspace */
+	int n, lmax, ld;	/* rows (nodes of the first half), orders 0..lmax, row stride */
+};
+
 #define PG_TL 8		/* orders per staged block of the table rows */
-__global__ void __launch_bounds__(256) k_pg_tables(const struct jb_bl *__restrict__ bl, int b0, const double *__restrict__ nodes, const double *__restrict__ lc, double *__restrict__ ws)
+__global__ void __launch_bounds__(256) k_pg_tables(const struct pg_table *__restrict__ tab, const double *__restrict__ nodes, const double *__restrict__ lc, double *__restrict__ ws)
 {
 	/* each wave's 64 rows, PG_TL orders at a time: a lane runs its node's
 	 * normalised Legendre recurrence
@@ -108,15 +114,54 @@ __global__ void __launch_bounds__(256) k_pg_tables(const struct jb_bl *__restric
 	 * orders per row (a row per lane written straight out put 64 rows'
 	 * cache lines in every store) */
 	__shared__ double tile[4][64][PG_TL + 1];
-	const struct jb_bl &B = bl[b0 + blockIdx.x];
-	const int lq = B.a > B.Lt ? B.a : B.Lt;
-	const int nth = B.nt / 2, nqh = (B.nq + 1) / 2, nn = nth + nqh;
+	const struct pg_table &B = tab[blockIdx.x];
 	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-	for(int base = 0; base < nn; base += 256) {
+	for(int base = 0; base < B.n; base += 256) {
 		const int i = base + threadIdx.x;
-		double x = 0.0;
+		const double x = i < B.n ? nodes[B.off_x + i] : 0.0;
+		/* Pbar_l0(x) for l = 0..lmax (every lane, the same bound) */
+		double p0 = 0.28209479177387814347, p1 = lc[2] * x * p0;
+		for(int l0 = 0; l0 <= B.lmax; l0 += PG_TL) {
+#pragma unroll
+			for(int c = 0; c < PG_TL; c++) {
+				const int l = l0 + c;
+				double v = 0.0;
+				if(l == 0)
+					v = p0;
+				else if(l == 1)
+					v = p1;
+				else if(l <= B.lmax) {
+					v = lc[2 * l] * x * p1 - lc[2 * l + 1] * p0;
+					p0 = p1;
+					p1 = v;
+				}
+				tile[wave][lane][c] = v;
+			}
+			__syncthreads();
+#pragma unroll
+			for(int k = 0; k < 8; k++) {
+				const int r = (lane >> 3) + 8 * k, c = lane & 7, nd = base + 64 * wave + r, l = l0 + c;
+				if(nd < B.n && l <= B.lmax)
+					ws[B.off + (size_t) nd * B.ld + l] = tile[wave][r][c];
+			}
+			__syncthreads();
+		}
+	}
+}
+
+/*
+ * The delay table of a baseline's tap nodes: y_j = r_dt cos(acos x_j) (the
+ * delay of node j in samples, projection.c:99-107), g_j = sin(pi y_j) nt
+ * (2 pi w_j / nt) / pi and the weight 2 pi w_j / nt; the product-rule
+ * weights.  Y = [y | g | weight] (nt/2 each) then (nq+1)/2 product weights.
+ */
+__global__ void __launch_bounds__(256) k_pg_nodes(const struct jb_bl *__restrict__ bl, int b0, const double *__restrict__ nodes, double *__restrict__ ws)
+{
+	const struct jb_bl &B = bl[b0 + blockIdx.x];
+	const int nth = B.nt / 2, nqh = (B.nq + 1) / 2;
+	for(int i = threadIdx.x; i < nth + nqh; i += 256) {
 		if(i < nth) {
-			x = nodes[B.off_nt + i];
+			const double x = nodes[B.off_nt + i];
 			const double y = B.r_dt * cos(acos(x));
 			const double ww = nodes[B.off_nt + B.nt + i] * (2. * M_PI / B.nt);
 			/* sin(pi y) = (-1)^n sin(pi (y - n)), n = rint(y): y - n is
@@ -128,40 +173,9 @@ __global__ void __launch_bounds__(256) k_pg_tables(const struct jb_bl *__restric
 			ws[B.off_Y + i] = y;
 			ws[B.off_Y + nth + i] = sy / M_PI * (double) B.nt * ww;
 			ws[B.off_Y + 2 * nth + i] = ww;
-		} else if(i < nn) {
+		} else {
 			const int q = i - nth;
-			x = nodes[B.off_nq + q];
 			ws[B.off_Y + 3 * nth + q] = nodes[B.off_nq + B.nq + q];
-		}
-		/* Pbar_l0(x) for l = 0..lq (every lane, the same bound) */
-		double p0 = 0.28209479177387814347, p1 = lc[2] * x * p0;
-		for(int l0 = 0; l0 <= lq; l0 += PG_TL) {
-#pragma unroll
-			for(int c = 0; c < PG_TL; c++) {
-				const int l = l0 + c;
-				double v = 0.0;
-				if(l == 0)
-					v = p0;
-				else if(l == 1)
-					v = p1;
-				else if(l <= lq) {
-					v = lc[2 * l] * x * p1 - lc[2 * l + 1] * p0;
-					p0 = p1;
-					p1 = v;
-				}
-				tile[wave][lane][c] = v;
-			}
-			__syncthreads();
-#pragma unroll
-			for(int k = 0; k < 8; k++) {
-				const int r = (lane >> 3) + 8 * k, c = lane & 7, nd = base + 64 * wave + r, l = l0 + c;
-				if(nd < nth) {
-					if(l <= B.a)
-						ws[B.off_Pt + (size_t) nd * (B.a + 1) + l] = tile[wave][r][c];
-				} else if(nd < nn && l <= lq)
-					ws[B.off_Pq + (size_t) (nd - nth) * (lq + 1) + l] = tile[wave][r][c];
-			}
-			__syncthreads();
 		}
 	}
 }
@@ -229,13 +243,45 @@ __global__ void k_pg_lag(const struct jb_bl *__restrict__ bl, int b0, double *__
 	ws[B.off_K + e] = acc;
 }
 
+/* tile -> baseline of the chunk for its four grouped launches (a binary
+ * search of the prefix sums in every workgroup was eleven dependent loads,
+ * 55.8 -> 54.7 ms for 4096 jobs):
+ * grid (baselines, 4), launch k's tiles from start[k nb + b] on, its map at
+ * map + base[k] */
+struct pg_bases {
+	long v[4];
+	int tot[4];
+};
+
+__global__ void k_pg_map(const int *__restrict__ start, int nb, struct pg_bases base, int *__restrict__ map)
+{
+	const int b = blockIdx.x, k = blockIdx.y;
+	const int t0 = start[k * nb + b], t1 = b + 1 < nb ? start[k * nb + b + 1] : base.tot[k];
+	for(int t = t0 + threadIdx.x; t < t1; t += blockDim.x)
+		map[base.v[k] + t] = b;
+}
+
+/* workgroup -> tile: contiguous ranges of tiles per XCD (workgroups go to
+ * the eight XCDs in turn, each with its own L2), so that the tiles of one
+ * baseline share its operands in one L2 (all plan products 57.4 -> 55.9 ms
+ * per plan and run of 4096 jobs) */
+__device__ inline int pg_tile_of(int id, int n)
+{
+	const int n8 = n & ~7;
+	return id < n8 ? (id & 7) * (n8 >> 3) + (id >> 3) : id;
+}
+
 /*
  * The plan's three products as one grouped float64 GEMM on MFMA
  * (v_mfma_f64_16x16x4f64) over all baselines of a chunk: workgroup = a
  * 64 x 64 tile of one baseline's product (4 waves of 32 x 32), K in
  * chunks of 16 staged in LDS through registers (the next chunk's loads in
- * flight during this chunk's MFMAs).  The workgroup finds its baseline
- * in the chunk's tile prefix sums.
+ * flight during this chunk's MFMAs).  Bound by the latency of that staging
+ * (a second LDS buffer leaves fewer workgroups per CU and is slower, 59.1
+ * against 57.4 ms): clamped loads in place of bounds branches took all of
+ * 4096 jobs from 64.7 to 60.4 ms, the swizzle (padded rows put the staging
+ * stores on few banks) to 57.4; the three products of a chunk of ~2,000
+ * baselines are 1.41 + 1.00 + 0.52 ms.
  *
  * Both quadrature rules are mirror-symmetric: node n-1-j is -x_j with the
  * same weight, and Pbar_l0(-x) = (-1)^l Pbar_l0(x).  Each product folds
@@ -257,31 +303,33 @@ enum { PG_TAPS, PG_SYNTH, PG_M };
 #define PG_TILE 64
 #define PG_KC 16
 
+__device__ inline int pg_swz(int k)
+{
+	return ((k & 1) << 4) | (k >> 1 << 1);
+}
+
 template <int MODE, typename TO>
-__global__ void __launch_bounds__(256) k_pg_gemm(const struct jb_bl *__restrict__ bl, int b0, int nb, const int *__restrict__ tile_start, double *__restrict__ ws, TO *__restrict__ Mout)
+__global__ void __launch_bounds__(256) k_pg_gemm(const struct jb_bl *__restrict__ bl, int b0, const int *__restrict__ tile_start, const int *__restrict__ tile_bl, double *__restrict__ ws, TO *__restrict__ Mout)
 {
 	typedef double v4 __attribute__((ext_vector_type(4)));
 	constexpr int NA = MODE == PG_SYNTH ? 1 : 2;	/* A tiles: pair sum and difference */
-	__shared__ double sA[NA][PG_KC][PG_TILE + 4];	/* [k][row] */
-	__shared__ double sB[PG_KC][PG_TILE + 4];	/* [k][col] */
-	/* this workgroup's baseline: the last with tile_start <= blockIdx.x */
-	int lo = 0, hi = nb - 1;
-	while(lo < hi) {
-		const int mid = (lo + hi + 1) >> 1;
-		if(tile_start[mid] <= (int) blockIdx.x)
-			lo = mid;
-		else
-			hi = mid - 1;
-	}
+	/* [k][row] and [k][col], column c of k at c ^ pg_swz(k): the staging
+	 * stores (16 k x 2 rows per half wave) and the operand reads (2 k x 16
+	 * rows) then fall on distinct banks */
+	__shared__ double sA[NA][PG_KC][PG_TILE];
+	__shared__ double sB[PG_KC][PG_TILE];
+	const int tile = pg_tile_of(blockIdx.x, gridDim.x);
+	const int lo = tile_bl[tile];
 	const struct jb_bl &B = bl[b0 + lo];
 	const int nqh = (B.nq + 1) / 2;
 	const int M = MODE == PG_M ? B.lags : B.np;
 	const int K = MODE == PG_TAPS ? B.nt / 2 : MODE == PG_SYNTH ? B.a + 1 : nqh;
 	const int ncol = MODE == PG_TAPS ? B.a + 1 : MODE == PG_SYNTH ? nqh : B.Lt + 1;
-	const int tiles_m = (M + PG_TILE - 1) / PG_TILE;
-	const int local = blockIdx.x - tile_start[lo];
-	const int m0 = (local % tiles_m) * PG_TILE, n0 = (local / tiles_m) * PG_TILE;
-	const int lq = B.a > B.Lt ? B.a : B.Lt;
+	/* the column tiles of a row panel side by side: the left operand, the
+	 * larger, is read from HBM once */
+	const int tiles_n = (ncol + PG_TILE - 1) / PG_TILE;
+	const int local = tile - tile_start[lo];
+	const int m0 = (local / tiles_n) * PG_TILE, n0 = (local % tiles_n) * PG_TILE;
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 	const int li = lane & 15, lk = lane >> 4;
 	const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
@@ -291,57 +339,65 @@ __global__ void __launch_bounds__(256) k_pg_gemm(const struct jb_bl *__restrict_
 	/* K chunk entry -> l (synthesis: 8 even l, then 8 odd l) */
 	auto kl = [&](int k0, int k) -> int { return MODE == PG_SYNTH ? k0 + (k < 8 ? 2 * k : 2 * (k - 8) + 1) : k0 + k; };
 	const int nth = B.nt / 2;
-	const double *Y = ws + B.off_Y;
+	/* each thread stages 4 rows x one k of A and either 4 k x one column of
+	 * B or, where B's rows are its columns (the synthesis), like A.  Loads
+	 * are clamped into the operands instead of skipped (a branch around a
+	 * load waits for all of them): rows and columns past the ends are not
+	 * stored, past the last k the B value is zero */
+	const int ka = tid % PG_KC, ia = tid / PG_KC, jb = tid % PG_TILE, kb4 = tid / PG_TILE;
+	const double *pa[4], *pm[4], *pb[4];
+#pragma unroll
+	for(int r = 0; r < 4; r++) {
+		const int i = m0 + ia + 16 * r < M ? m0 + ia + 16 * r : M - 1;
+		pa[r] = MODE == PG_TAPS ? ws + B.off_F + 2 * (size_t) i * nth : MODE == PG_SYNTH ? ws + B.off_C + (size_t) i * (B.a + 1) : ws + B.off_K + (size_t) i * nqh;
+		pm[r] = MODE == PG_M ? ws + B.off_K + (size_t) (B.lags - 1 - i) * nqh : NULL;
+		if(MODE == PG_SYNTH) {
+			const int j = n0 + ia + 16 * r < ncol ? n0 + ia + 16 * r : ncol - 1;
+			pb[r] = ws + B.off_Pq + (size_t) j * B.ldq;
+		}
+	}
+	const int jcol = MODE == PG_SYNTH || col(jb) < ncol ? col(jb) : ncol - 1;
+	const double *pB = MODE == PG_TAPS ? ws + B.off_Pt + jcol : ws + B.off_Pq + jcol;
+	const size_t ldB = MODE == PG_TAPS ? B.a + 1 : B.ldq;
+	const double *Yw = ws + B.off_Y + 3 * (size_t) nth;
 	double ra[NA][4], rb[4];
 	auto load = [&](int k0) {
+		const int k = kl(k0, ka), kc = k < K ? k : K - 1;
 #pragma unroll
 		for(int r = 0; r < 4; r++) {
-			const int e = tid + 256 * r;
-			const int i = m0 + e / PG_KC, k = kl(k0, e % PG_KC);
-			double v0 = 0.0, v1 = 0.0;
-			if(i < M && k < K) {
-				if(MODE == PG_TAPS) {
-					const double2 f = *reinterpret_cast<const double2 *>(ws + B.off_F + 2 * ((size_t) i * nth + k));
-					v0 = f.x;
-					v1 = f.y;
-				}
-				else if(MODE == PG_SYNTH)
-					v0 = ws[B.off_C + (size_t) i * (B.a + 1) + k];
-				else {
-					const double kp = ws[B.off_K + (size_t) i * nqh + k];
-					if(2 * k == B.nq - 1)
-						v0 = kp;
-					else {
-						const double km = ws[B.off_K + (size_t) (B.lags - 1 - i) * nqh + k];
-						v0 = kp + km;
-						v1 = kp - km;
-					}
-				}
+			if(MODE == PG_TAPS) {
+				const double2 f = *reinterpret_cast<const double2 *>(pa[r] + 2 * (size_t) kc);
+				ra[0][r] = f.x;
+				ra[NA - 1][r] = f.y;
+			} else if(MODE == PG_SYNTH)
+				ra[0][r] = pa[r][kc];
+			else {
+				const double kp = pa[r][kc], km = pm[r][kc];
+				const bool mid = 2 * kc == B.nq - 1;	/* the middle node once */
+				ra[0][r] = mid ? kp : kp + km;
+				ra[NA - 1][r] = mid ? 0.0 : kp - km;
 			}
-			ra[0][r] = v0;
-			if(NA == 2)
-				ra[NA - 1][r] = v1;
-			const int kb = kl(k0, e / PG_TILE), j = col(e % PG_TILE);
-			double vb = 0.0;
-			if(kb < K && j < ncol) {
-				if(MODE == PG_TAPS)
-					vb = ws[B.off_Pt + (size_t) kb * (B.a + 1) + j];
-				else if(MODE == PG_SYNTH)
-					vb = ws[B.off_Pq + (size_t) j * (lq + 1) + kb];
-				else
-					vb = (2. * M_PI * Y[3 * nth + kb]) * ws[B.off_Pq + (size_t) kb * (lq + 1) + j];
+			if(MODE == PG_SYNTH)
+				rb[r] = k < K ? pb[r][kc] : 0.0;
+			else {
+				const int kb = k0 + kb4 + 4 * r, kbc = kb < K ? kb : K - 1;
+				double v = pB[kbc * ldB];
+				if(MODE == PG_M)
+					v *= 2. * M_PI * Yw[kbc];
+				rb[r] = kb < K ? v : 0.0;
 			}
-			rb[r] = vb;
 		}
 	};
 	auto store = [&]() {
 #pragma unroll
 		for(int r = 0; r < 4; r++) {
-			const int e = tid + 256 * r;
 #pragma unroll
 			for(int h = 0; h < NA; h++)
-				sA[h][e % PG_KC][e / PG_KC] = ra[h][r];
-			sB[e / PG_TILE][e % PG_TILE] = rb[r];
+				sA[h][ka][(ia + 16 * r) ^ pg_swz(ka)] = ra[h][r];
+			if(MODE == PG_SYNTH)
+				sB[ka][(ia + 16 * r) ^ pg_swz(ka)] = rb[r];
+			else
+				sB[kb4 + 4 * r][jb ^ pg_swz(kb4 + 4 * r)] = rb[r];
 		}
 	};
 	v4 acc[2][2][2];	/* [parity of l (synthesis)][row block][column block] */
@@ -361,13 +417,14 @@ __global__ void __launch_bounds__(256) k_pg_gemm(const struct jb_bl *__restrict_
 #pragma unroll
 		for(int ks = 0; ks < PG_KC; ks += 4) {
 			const int p = MODE == PG_SYNTH && ks >= 8 ? 1 : 0;
+			const int sw = pg_swz(ks + lk);
 			double af[2], bf[2];
 #pragma unroll
 			for(int a = 0; a < 2; a++)
-				af[a] = sA[sel][ks + lk][wm + 16 * a + li];
+				af[a] = sA[sel][ks + lk][(wm + 16 * a + li) ^ sw];
 #pragma unroll
 			for(int b = 0; b < 2; b++)
-				bf[b] = sB[ks + lk][wn + 16 * b + li];
+				bf[b] = sB[ks + lk][(wn + 16 * b + li) ^ sw];
 #pragma unroll
 			for(int a = 0; a < 2; a++)
 #pragma unroll
@@ -422,19 +479,13 @@ __host__ __device__ inline size_t pg_lag_lds(int np, int lq)
 	return (size_t) ((np + PG_LPA) + (PG_LR - 1 + np + PG_LPB)) * lq * sizeof(double);
 }
 
-__global__ void __launch_bounds__(256) k_pg_lag2(const struct jb_bl *__restrict__ bl, int b0, int nb, const int *__restrict__ qblk_start, int lq, double *__restrict__ ws)
+__global__ void __launch_bounds__(256) k_pg_lag2(const struct jb_bl *__restrict__ bl, int b0, const int *__restrict__ qblk_start, const int *__restrict__ qblk_bl, int lq, double *__restrict__ ws)
 {
 	extern __shared__ double lg_sm[];
-	int lo = 0, hi = nb - 1;
-	while(lo < hi) {
-		const int mid = (lo + hi + 1) >> 1;
-		if(qblk_start[mid] <= (int) blockIdx.x)
-			lo = mid;
-		else
-			hi = mid - 1;
-	}
+	const int tile = pg_tile_of(blockIdx.x, gridDim.x);
+	const int lo = qblk_bl[tile];
 	const struct jb_bl &B = bl[b0 + lo];
-	const int q0 = (blockIdx.x - qblk_start[lo]) * lq;
+	const int q0 = (tile - qblk_start[lo]) * lq;
 	const int np = B.np, nq = B.nq;
 	const int na = np + PG_LPA, nbr = PG_LR - 1 + np + PG_LPB;
 	double *Ta = lg_sm;			/* [na][lq]: T[i][q0 + c] */
@@ -713,10 +764,15 @@ static int generate_plans(struct sphr_jobs *J, hipStream_t st, int (*host_work)(
 	const int nbl = J->n_bl;
 	double *ws = NULL, *nodes = NULL, *hnodes = NULL;
 	int *d_ts = NULL, *h_ts = NULL;	/* per chunk: tile prefix sums of its four plan launches */
+	int *d_map = NULL;	/* their tiles' baselines, one chunk at a time */
+	long map_max = 0;
 	long *rule_t = NULL, *rule_q = NULL;
+	struct pg_table *tabs = NULL, *d_tabs = NULL;
+	int *lq_of = NULL, *seen_t = NULL, *seen_q = NULL, ntab = 0;	/* per rule: largest order, its table in the chunk at hand */
 	struct pg_chunk {
 		int b0, b1, lq, lag_tiled, np_max, lags_nq_max;
 		long f_max;	/* most taps pairs of a baseline */
+		int t0, nt;	/* its Legendre tables */
 		long tot[4];
 	} *ch = NULL;
 	int nch = 0, rc = -1;
@@ -731,7 +787,11 @@ static int generate_plans(struct sphr_jobs *J, hipStream_t st, int (*host_work)(
 	rule_q = (long *) malloc((nq_max + 1) * sizeof(long));
 	ch = (struct pg_chunk *) calloc(nbl, sizeof(*ch));
 	h_ts = (int *) malloc((size_t) 4 * nbl * sizeof(int));
-	if(!rule_t || !rule_q || !ch || !h_ts) {
+	lq_of = (int *) calloc(nq_max + 1, sizeof(int));
+	seen_t = (int *) malloc((a_max + 1) * sizeof(int));
+	seen_q = (int *) malloc((nq_max + 1) * sizeof(int));
+	tabs = (struct pg_table *) malloc(2 * (size_t) nbl * sizeof(*tabs));
+	if(!rule_t || !rule_q || !ch || !h_ts || !lq_of || !seen_t || !seen_q || !tabs) {
 		sphr_set_error("sphr_jobs_new: out of memory");
 		goto done;
 	}
@@ -759,6 +819,8 @@ static int generate_plans(struct sphr_jobs *J, hipStream_t st, int (*host_work)(
 		for(int b = 0; b < nbl; b++) {
 			const int lq = J->bl[b].a > J->bl[b].Lt ? J->bl[b].a : J->bl[b].Lt;
 			lq_max = lq > lq_max ? lq : lq_max;
+			int &lo = lq_of[J->bl[b].nq];
+			lo = lq > lo ? lq : lo;
 		}
 		lc_off = nsz;
 		lc_n = lq_max + 1;
@@ -815,17 +877,35 @@ static int generate_plans(struct sphr_jobs *J, hipStream_t st, int (*host_work)(
 		int b1 = b0;
 		C.np_max = C.lags_nq_max = 0;
 		C.f_max = 0;
+		for(int i = 0; i <= a_max; i++)
+			seen_t[i] = -1;
+		for(int i = 0; i <= nq_max; i++)
+			seen_q[i] = -1;
+		C.t0 = ntab;
 		while(b1 < nbl) {
 			struct jb_bl &B = J->bl[b1];
-			const int lq = B.a > B.Lt ? B.a : B.Lt;
-			const int nth = B.nt / 2, nqh = (B.nq + 1) / 2;
-			const size_t need = (size_t) nth * (B.a + 1) + (size_t) nqh * (lq + 1) + (size_t) B.np * (B.a + 1) + (size_t) B.np * B.nq + (size_t) B.lags * nqh + 3 * (size_t) nth + nqh
+			const int nth = B.nt / 2, nqh = (B.nq + 1) / 2, ldq = lq_of[B.nq] + 1;
+			/* the Legendre tables, where no baseline of the chunk has
+			 * made them needed yet */
+			const size_t n_t = seen_t[B.a] < 0 ? (size_t) nth * (B.a + 1) : 0, n_q = seen_q[B.nq] < 0 ? (size_t) nqh * ldq : 0;
+			const size_t need = n_t + n_q + (size_t) B.np * (B.a + 1) + (size_t) B.np * B.nq + (size_t) B.lags * nqh + 3 * (size_t) nth + nqh
 					    + 2 * (size_t) B.np * nth + 1;
 			if(b1 > b0 && (wsz + need) * sizeof(double) > budget)
 				break;
-			B.off_Pt = wsz;
-			B.off_Pq = B.off_Pt + (long) nth * (B.a + 1);
-			B.off_C = B.off_Pq + (long) nqh * (lq + 1);
+			if(n_t) {
+				const struct pg_table t = { B.off_nt, (long) wsz, nth, B.a, B.a + 1 };
+				seen_t[B.a] = ntab;
+				tabs[ntab++] = t;
+			}
+			if(n_q) {
+				const struct pg_table t = { B.off_nq, (long) (wsz + n_t), nqh, ldq - 1, ldq };
+				seen_q[B.nq] = ntab;
+				tabs[ntab++] = t;
+			}
+			B.off_Pt = tabs[seen_t[B.a]].off;
+			B.off_Pq = tabs[seen_q[B.nq]].off;
+			B.ldq = ldq;
+			B.off_C = (long) (wsz + n_t + n_q);
 			B.off_T = B.off_C + (long) B.np * (B.a + 1);
 			B.off_K = B.off_T + (long) B.np * B.nq;
 			B.off_Y = B.off_K + (long) B.lags * nqh;
@@ -841,6 +921,7 @@ static int generate_plans(struct sphr_jobs *J, hipStream_t st, int (*host_work)(
 		}
 		C.b0 = b0;
 		C.b1 = b1;
+		C.nt = ntab - C.t0;
 		wsz_max = wsz > wsz_max ? wsz : wsz_max;
 		/* lag tile: the widest column block whose two LDS column blocks
 		 * stay within 48 KiB (four workgroups per CU); past 160 KiB at
@@ -871,10 +952,15 @@ static int generate_plans(struct sphr_jobs *J, hipStream_t st, int (*host_work)(
 				sphr_set_error("sphr_jobs_new: plan chunk too large");
 				goto done;
 			}
+		const long mt = C.tot[0] + C.tot[1] + C.tot[2] + C.tot[3];
+		map_max = mt > map_max ? mt : map_max;
 		b0 = b1;
 	}
 	if(sphr_rt_check(hipMalloc(&ws, wsz_max * sizeof(double)), "hipMalloc") || sphr_rt_check(hipMalloc(&nodes, nsz * sizeof(double)), "hipMalloc")
 	   || sphr_rt_check(hipMalloc(&d_ts, (size_t) 4 * nbl * sizeof(int)), "hipMalloc")
+	   || sphr_rt_check(hipMalloc(&d_map, map_max * sizeof(int)), "hipMalloc")
+	   || sphr_rt_check(hipMalloc(&d_tabs, ntab * sizeof(*tabs)), "hipMalloc")
+	   || sphr_rt_check(hipMemcpyAsync(d_tabs, tabs, ntab * sizeof(*tabs), hipMemcpyHostToDevice, st), "hipMemcpy")
 	   || sphr_rt_check(hipMemcpyAsync(nodes, hnodes, nsz * sizeof(double), hipMemcpyHostToDevice, st), "hipMemcpy")
 	   || sphr_rt_check(hipMemcpyAsync(J->d_bl, J->bl, (size_t) nbl * sizeof(struct jb_bl), hipMemcpyHostToDevice, st), "hipMemcpy")
 	   || sphr_rt_check(hipMemcpyAsync(d_ts, h_ts, (size_t) 4 * nbl * sizeof(int), hipMemcpyHostToDevice, st), "hipMemcpy"))
@@ -883,15 +969,24 @@ static int generate_plans(struct sphr_jobs *J, hipStream_t st, int (*host_work)(
 		const struct pg_chunk &C = ch[c];
 		const int b0 = C.b0, nb = C.b1 - C.b0;
 		const int *ts = d_ts + 4 * (size_t) b0;
-		hipLaunchKernelGGL(k_pg_tables, dim3(nb), dim3(256), 0, st, J->d_bl, b0, nodes, nodes + lc_off, ws);
+		struct pg_bases pb;
+		long at = 0;
+		for(int k = 0; k < 4; k++) {
+			pb.v[k] = at;
+			pb.tot[k] = (int) C.tot[k];
+			at += C.tot[k];
+		}
+		hipLaunchKernelGGL(k_pg_map, dim3(nb, 4), dim3(64), 0, st, ts, nb, pb, d_map);
+		hipLaunchKernelGGL(k_pg_tables, dim3(C.nt), dim3(256), 0, st, d_tabs + C.t0, nodes, nodes + lc_off, ws);
+		hipLaunchKernelGGL(k_pg_nodes, dim3(nb), dim3(256), 0, st, J->d_bl, b0, nodes, ws);
 		hipLaunchKernelGGL(k_pg_fpairs, dim3((unsigned) ((C.f_max + PG_FB - 1) / PG_FB), nb), dim3(256), 0, st, J->d_bl, b0, ws);
-		hipLaunchKernelGGL((k_pg_gemm<PG_TAPS, double>), dim3(C.tot[0]), dim3(256), 0, st, J->d_bl, b0, nb, ts, ws, (double *) NULL);
-		hipLaunchKernelGGL((k_pg_gemm<PG_SYNTH, double>), dim3(C.tot[1]), dim3(256), 0, st, J->d_bl, b0, nb, ts + nb, ws, (double *) NULL);
+		hipLaunchKernelGGL((k_pg_gemm<PG_TAPS, double>), dim3(C.tot[0]), dim3(256), 0, st, J->d_bl, b0, ts, d_map + pb.v[0], ws, (double *) NULL);
+		hipLaunchKernelGGL((k_pg_gemm<PG_SYNTH, double>), dim3(C.tot[1]), dim3(256), 0, st, J->d_bl, b0, ts + nb, d_map + pb.v[1], ws, (double *) NULL);
 		if(C.lag_tiled)
-			hipLaunchKernelGGL(k_pg_lag2, dim3(C.tot[3]), dim3(256), pg_lag_lds(C.np_max, C.lq), st, J->d_bl, b0, nb, ts + 3 * nb, C.lq, ws);
+			hipLaunchKernelGGL(k_pg_lag2, dim3(C.tot[3]), dim3(256), pg_lag_lds(C.np_max, C.lq), st, J->d_bl, b0, ts + 3 * nb, d_map + pb.v[3], C.lq, ws);
 		else
 			hipLaunchKernelGGL(k_pg_lag, dim3((C.lags_nq_max + 255) / 256, nb), dim3(256), 0, st, J->d_bl, b0, ws);
-		hipLaunchKernelGGL((k_pg_gemm<PG_M, T>), dim3(C.tot[2]), dim3(256), 0, st, J->d_bl, b0, nb, ts + 2 * nb, ws, (T *) J->M);
+		hipLaunchKernelGGL((k_pg_gemm<PG_M, T>), dim3(C.tot[2]), dim3(256), 0, st, J->d_bl, b0, ts + 2 * nb, d_map + pb.v[2], ws, (T *) J->M);
 		hipLaunchKernelGGL((k_pg_rot<T>), dim3(nb), dim3(128), 0, st, J->d_bl, b0, (cplx<T> *) J->R);
 		if(sphr_rt_check(hipGetLastError(), "plan kernels"))
 			goto done;
@@ -912,6 +1007,14 @@ done:
 		hipFree(nodes);
 	if(d_ts)
 		hipFree(d_ts);
+	if(d_map)
+		hipFree(d_map);
+	if(d_tabs)
+		hipFree(d_tabs);
+	free(lq_of);
+	free(seen_t);
+	free(seen_q);
+	free(tabs);
 	free(hnodes);
 	free(h_ts);
 	free(rule_t);

@@ -210,3 +210,45 @@ def test_gpu_jobs_tuned_tiles_match_oracle(top_case, prec):
         J.set_lag_tile(sc, nt)
         print("lag tile", sc, nt, flush=True)
         _check_jobs(J, jobs, want, d_in, cdt, tol)
+
+
+def shared_rule_jobs(sep):
+    """Jobs of one pair of sites (separation sep in Earth radii) over the
+    orders: they share the tap rule; orders 2k and 2k + 1 also share the
+    product rule, whose table has to reach the larger of the two.  Orders
+    62..65 straddle a 64-wide tile of the plan products."""
+    r = inject.EARTH_RADIUS_SPHERE / inject.C_SI
+    pos = r * np.array([[0.0, 0.0, 1.0], [0.0, math.sin(sep), math.cos(sep)]])
+    rng = np.random.default_rng(5)
+    jobs = [{"positions": pos, "N": 512, "l_max": L} for L in (1, 2, 3, 18, 19, 62, 63, 64, 65)]
+    data = [rng.standard_normal((2, 512)).astype(np.float32) for _ in jobs]
+    return jobs, data
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sep", [0.05, 0.3, 1.2])
+@pytest.mark.parametrize("prec,cdt,tol", [(S.FP64, np.complex128, 1e-12), (S.MIXED, np.complex64, 1e-5)])
+def test_gpu_jobs_sharing_rules(oracle, sep, prec, cdt, tol):
+    """Every job's sky is bit for bit the one it has alone (its tables then
+    reach its own order only, and its tiles are in another order); up to
+    order 19 it is the oracle's.  (Above, rounding of the
+    polar rotation, a recursion over the orders on both sides, passes 1e-12
+    for some directions.)"""
+    jobs, data = shared_rule_jobs(sep)
+
+    def run(js, ds):
+        J = S.Jobs(js, DT, precision=prec)
+        n = J.info()["alm_elems"]
+        d_in = S.DeviceBuffer.from_numpy(np.concatenate([d.ravel() for d in ds]))
+        d_alm = S.DeviceBuffer(n * np.dtype(cdt).itemsize)
+        d_map = S.DeviceBuffer(J.info()["map_elems"] * np.dtype(cdt).itemsize)
+        J.run(d_in.ptr, d_alm.ptr, d_map.ptr)
+        S.synchronize()
+        alm = d_alm.to_numpy(cdt, (n,))
+        return [alm[o:o + (j["l_max"] + 1) ** 2] for o, j in zip(J.off_alm, js)]
+
+    for j, d, a in zip(jobs, data, run(jobs, data)):
+        assert np.array_equal(a, run([j], [d])[0]), j["l_max"]
+        if j["l_max"] <= 19:
+            want, _ = oracle.Network(j["positions"], j["N"], DT, j["l_max"]).segment(d.astype(np.float64), j["l_max"])
+            assert rel(a, want) < tol, j["l_max"]
