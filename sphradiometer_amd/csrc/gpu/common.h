@@ -47,9 +47,8 @@ __host__ __device__ inline int lm_offset(int L, int l, int m)
 	return base + l - (m < 0 ? -m : m);
 }
 
-/* the order m of coefficient idx in a series of order L (closed form of
- * lm_decode's m: the block of idx from the quadratic of the block starts,
- * then corrected by whole blocks) */
+/* the order m of coefficient idx in a series of order L: the block of idx
+ * from the quadratic of the block starts, then corrected by whole blocks */
 __host__ __device__ inline int lm_order(int L, int idx)
 {
 	const int L1 = L + 1;
@@ -79,24 +78,13 @@ __host__ __device__ inline int lm_order(int L, int idx)
 /* inverse of lm_offset: decode index -> (l, m) */
 __host__ __device__ inline void lm_decode(int L, int idx, int *l, int *m)
 {
-	const int L1 = L + 1;
-	const int npos = L1 * (L1 + 1) / 2;
-	if(idx < npos) {
-		int mm = 0;
-		while(L1 * (mm + 1) - (mm + 1) * mm / 2 <= idx)
-			mm++;
-		*m = mm;
-		*l = idx - (L1 * mm - mm * (mm - 1) / 2) + mm;
-	} else {
-		/* blocks m = -L .. -1 follow */
-		int rem = idx - npos;
-		int mm = -L;
-		while(rem >= L1 + mm) {
-			rem -= L1 + mm;
-			mm++;
-		}
-		*m = mm;
-		*l = rem - mm;
+	const int mm = lm_order(L, idx);
+	*m = mm;
+	if(mm >= 0)
+		*l = idx - ((L + 1) * mm - mm * (mm - 1) / 2) + mm;
+	else {
+		const int k = mm + L;
+		*l = idx - (L + 1) * (L + 2) / 2 - k * (k + 1) / 2 - mm;
 	}
 }
 

@@ -57,15 +57,38 @@ struct td_plan {
 	double *d_powc;			/* power_1d as P + 1 complex (imaginary parts 0) */
 	double *d_rows;			/* (P + 1)^2 complex: D^l_{0 m'} of the rotation plan */
 	size_t cap_out, cap_sv, cap_edge;
-	double *d_sv;			/* window differences on their support: values, then offsets */
-	double *d_edge;			/* first row and column of C */
+	double *d_sv;			/* a call's window differences on their support, baseline by baseline */
+	double *d_edge;			/* first row and column of C, by chunk */
 	double *d_out;			/* rotated series (or a network's partial sums) */
 	/* a network's series and windows (kept on its first plan) */
-	size_t cap_nts, cap_nws;
-	double *d_nts, *d_nws;
+	size_t cap_nts, cap_nws, cap_npow;
+	double *d_nts, *d_nws, *d_npow;	/* npow: every baseline's power */
 };
 
 namespace {
+
+/*
+ * One baseline of a call.  The baselines of a network go through each
+ * kernel together, blockIdx.z the baseline (at most TD_SET per launch): the
+ * launches of one baseline leave the chip nearly idle, and one after the
+ * other with a copy of each window's differences between them they were
+ * 300 of the 780 us of three baselines over 65536 samples; together 50.
+ */
+#define TD_SET 8
+struct td_item {
+	const double *a, *b;	/* the series */
+	const double *w;	/* the window, or NULL where sv describes it */
+	const double *sv;	/* its nnz first differences: values, offsets, running sums */
+	const double *Ta, *Tb, *WP;
+	double *part, *edge, *C, *U, *pow;
+	int sparse, nnz, nt, np, nq, P;
+	int nk, nz, tpz, tiles;	/* correlation: terms, K splits, terms per split, tiles per side */
+	int nch, spc;		/* first row and column: chunks, samples per chunk */
+};
+
+struct td_set {
+	struct td_item it[TD_SET];
+};
 
 /*
  * partial[z][k][k'] = sum_{t in split z} w[t] a[s_t + k] b[s_t + k'],
@@ -84,8 +107,13 @@ namespace {
 /* output samples per K split */
 #define TD_TSPLIT 1024
 
-__global__ void __launch_bounds__(256) k_td_corr(const double *__restrict__ a, const double *__restrict__ b, const double *__restrict__ w, const double *__restrict__ sidx, int na, int nt, int np, int tpz, int tiles, double *__restrict__ part)
+__global__ void __launch_bounds__(256) k_td_corr(const struct td_set set, int na)
 {
+	const struct td_item &I = set.it[blockIdx.z];
+	const int tiles = I.tiles, np = I.np, nt = I.nk, tpz = I.tpz;
+	if((int) blockIdx.x >= tiles * tiles * I.nz)
+		return;
+	const double *__restrict__ a = I.a, *__restrict__ b = I.b, *__restrict__ w = I.sparse ? I.sv : I.w, *__restrict__ sidx = I.sparse ? I.sv + I.nnz : NULL;
 	typedef double v4 __attribute__((ext_vector_type(4)));
 	__shared__ double sA[TD_KC][TD_TILE + 4];	/* [t][k] */
 	__shared__ double sB[TD_KC][TD_TILE + 4];	/* [t][k'] */
@@ -144,7 +172,8 @@ __global__ void __launch_bounds__(256) k_td_corr(const double *__restrict__ a, c
 		}
 		__syncthreads();
 	}
-	double *P = part + (size_t) z * np * np;
+	/* a single split is C itself */
+	double *P = I.nz == 1 ? I.C : I.part + (size_t) z * np * np;
 #pragma unroll
 	for(int i = 0; i < 2; i++)
 #pragma unroll
@@ -161,81 +190,142 @@ __global__ void __launch_bounds__(256) k_td_corr(const double *__restrict__ a, c
 		}
 }
 
-/* C = sum_z partial[z] */
-__global__ void k_td_reduce(const double *__restrict__ part, int nz, long n, double *__restrict__ C)
+/* C = sum_z partial[z] where there are several */
+__global__ void k_td_reduce(const struct td_set set)
 {
-	const long i = (long) blockIdx.x * blockDim.x + threadIdx.x;
-	if(i >= n)
+	const struct td_item &I = set.it[blockIdx.z];
+	const long i = (long) blockIdx.x * blockDim.x + threadIdx.x, n = (long) I.np * I.np;
+	if(i >= n || I.nz == 1)
 		return;
 	double s = 0.0;
-	for(int z = 0; z < nz; z++)
-		s += part[(size_t) z * n + i];
-	C[i] = s;
+#pragma unroll 4
+	for(int z = 0; z < I.nz; z++)
+		s += I.part[(size_t) z * n + i];
+	I.C[i] = s;
 }
 
-/* part[c][j] = sum_{t in chunk c} w[t] a[t] b[t + j] and part[c][np + j]
- * = sum_{t in chunk c} w[t] a[t + j] b[t], j < np (the first row and
- * column of C, summed over the chunks by k_td_reduce): TD_EC samples per
- * workgroup, staged in LDS with the np - 1 samples after them, each
- * thread one or more j of both */
-#define TD_EC 1024
+/*
+ * part[c][j] = sum_{t in chunk c} w[t] a[t] b[t + j] and part[c][np + j] =
+ * sum_{t in chunk c} w[t] a[t + j] b[t], j < np (the first row and column
+ * of C, summed over the chunks by k_td_diag).  A workgroup takes a chunk
+ * and TD_EJ offsets j, TD_EC samples at a time through LDS: each wave a
+ * quarter of the samples, each lane four consecutive j, whose 2 x 4 shifted
+ * samples slide through its registers, two LDS reads for eight
+ * multiply-adds (with one j per thread the reads bounded it: three
+ * baselines over 65536 samples 81 + 48 us with the sum over the chunks,
+ * now 13, and the sum 4 of k_td_diag's 9).  The shifted samples lie with one double of padding after every
+ * four (lanes four apart then read different banks).  The window is rebuilt
+ * where it is staged from its differences: w[t] = -sum_{s <= t} v[s].
+ */
+#define TD_EC 256
+#define TD_EJ 256
+/* most chunks of a baseline: a longer series has longer chunks */
+#define TD_NCH_MAX 1024
 #define TD_EDGE_NP_MAX 1024
-__global__ void __launch_bounds__(256) k_td_edge(const double *__restrict__ a, const double *__restrict__ b, const double *__restrict__ w, int nt, int n, int np, double *__restrict__ part)
+__global__ void __launch_bounds__(256) k_td_edge(const struct td_set set, int n)
 {
-	__shared__ double wa[TD_EC], wb[TD_EC], ya[TD_EC + TD_EDGE_NP_MAX], yb[TD_EC + TD_EDGE_NP_MAX];
-	const int t0 = blockIdx.x * TD_EC;
-	for(int t = threadIdx.x; t < TD_EC; t += 256) {
-		const bool ok = t0 + t < nt;
-		wa[t] = ok ? w[t0 + t] * a[t0 + t] : 0.0;
-		wb[t] = ok ? w[t0 + t] * b[t0 + t] : 0.0;
+	constexpr int NY = TD_EC + TD_EJ + 4;
+	__shared__ double wa[TD_EC], wb[TD_EC], ya[NY + NY / 4], yb[NY + NY / 4], red[2][4][TD_EJ];
+	const struct td_item &I = set.it[blockIdx.z];
+	const int nt = I.nt, np = I.np, nnz = I.nnz, j0 = blockIdx.y * TD_EJ;
+	if(!I.sparse || (int) blockIdx.x >= I.nch || j0 >= np)
+		return;
+	const double *__restrict__ a = I.a, *__restrict__ b = I.b, *__restrict__ sidx = I.sv + nnz, *__restrict__ cum = I.sv + 2 * (size_t) nnz;
+	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+	const int c0 = blockIdx.x * I.spc, c1 = c0 + I.spc < nt ? c0 + I.spc : nt;
+	double r[4] = { 0.0, 0.0, 0.0, 0.0 }, c[4] = { 0.0, 0.0, 0.0, 0.0 };
+	for(int t0 = c0; t0 < c1; t0 += TD_EC) {
+		__syncthreads();
+		for(int i = tid; i < NY; i += 256) {
+			const int t = t0 + j0 + i;
+			ya[i + (i >> 2)] = t < n ? a[t] : 0.0;
+			yb[i + (i >> 2)] = t < n ? b[t] : 0.0;
+		}
+		{
+			const int t = t0 + tid;
+			double x = 0.0, y = 0.0;
+			if(t < c1) {
+				int lo = 0, hi = nnz;
+				while(lo < hi) {
+					const int mid = (lo + hi) >> 1;
+					if(sidx[mid] <= (double) t)
+						lo = mid + 1;
+					else
+						hi = mid;
+				}
+				const double w = lo ? -cum[lo - 1] : 0.0;
+				x = w * a[t];
+				y = w * b[t];
+			}
+			wa[tid] = x;
+			wb[tid] = y;
+		}
+		__syncthreads();
+		/* samples t0 + s, s = 64 wave + ..: y index 4 lane + s + (0..3) */
+		const int s0 = 64 * wave, y0 = 5 * lane + (s0 + (s0 >> 2));
+		double va[8], vb[8];
+#pragma unroll
+		for(int i = 0; i < 4; i++) {
+			va[i] = ya[y0 + i];
+			vb[i] = yb[y0 + i];
+		}
+#pragma unroll 4
+		for(int s = 0; s < 64; s += 4) {
+#pragma unroll
+			for(int i = 0; i < 4; i++) {
+				va[4 + i] = ya[y0 + s / 4 * 5 + 5 + i];
+				vb[4 + i] = yb[y0 + s / 4 * 5 + 5 + i];
+			}
+#pragma unroll
+			for(int u = 0; u < 4; u++) {
+				const double x = wa[s0 + s + u], y = wb[s0 + s + u];
+#pragma unroll
+				for(int i = 0; i < 4; i++) {
+					r[i] = fma(x, vb[u + i], r[i]);
+					c[i] = fma(y, va[u + i], c[i]);
+				}
+			}
+#pragma unroll
+			for(int i = 0; i < 4; i++) {
+				va[i] = va[4 + i];
+				vb[i] = vb[4 + i];
+			}
+		}
 	}
-	for(int t = threadIdx.x; t < TD_EC + np - 1; t += 256) {
-		const bool ok = t0 + t < n;
-		ya[t] = ok ? a[t0 + t] : 0.0;
-		yb[t] = ok ? b[t0 + t] : 0.0;
+#pragma unroll
+	for(int i = 0; i < 4; i++) {
+		red[0][wave][4 * lane + i] = r[i];
+		red[1][wave][4 * lane + i] = c[i];
 	}
 	__syncthreads();
-	for(int jj = threadIdx.x; jj < np; jj += 256) {
-		double r = 0.0, c = 0.0;
-		for(int t = 0; t < TD_EC; t++) {
-			r = fma(wa[t], yb[t + jj], r);
-			c = fma(wb[t], ya[t + jj], c);
-		}
-		part[(size_t) blockIdx.x * 2 * np + jj] = r;
-		part[(size_t) blockIdx.x * 2 * np + np + jj] = c;
+	if(j0 + tid < np) {
+		double *o = I.edge + (size_t) blockIdx.x * 2 * np + j0 + tid;
+		o[0] = (red[0][0][tid] + red[0][1][tid]) + (red[0][2][tid] + red[0][3][tid]);
+		o[np] = (red[1][0][tid] + red[1][1][tid]) + (red[1][2][tid] + red[1][3][tid]);
 	}
 }
 
-/* w[t] = -sum_{s <= t} v[s], t < nt: the window rebuilt from its first
- * differences on their support (offsets sidx, running sums cum), so a
- * flat window need not be copied to the device */
-__global__ void k_td_wfill(const double *__restrict__ sidx, const double *__restrict__ cum, int nnz, int nt, double *__restrict__ w)
+/* C from its first row and column (the chunk sums in edge) and the diagonal
+ * differences D (in C on entry): C[k + 1][k' + 1] = C[k][k'] + D[k][k'].
+ * One wave per diagonal k' - k: the lanes sum the chunks of its first
+ * element, each lane sums a segment of D, a scan over the lanes gives each
+ * segment's starting value, and the lanes then write their segments. */
+__global__ void __launch_bounds__(256) k_td_diag(const struct td_set set)
 {
-	const int t = blockIdx.x * blockDim.x + threadIdx.x;
-	if(t >= nt)
-		return;
-	int lo = 0, hi = nnz;
-	while(lo < hi) {
-		const int mid = (lo + hi) >> 1;
-		if(sidx[mid] <= (double) t)
-			lo = mid + 1;
-		else
-			hi = mid;
-	}
-	w[t] = lo ? -cum[lo - 1] : 0.0;
-}
-
-/* C from its first row and column (edge) and the diagonal differences D
- * (in X on entry, C on return): C[k + 1][k' + 1] = C[k][k'] + D[k][k'].
- * One wave per diagonal k' - k: each lane sums a segment of D, a scan
- * over the lanes gives each segment's starting value, and the lanes then
- * write their segments. */
-__global__ void __launch_bounds__(256) k_td_diag(const double *__restrict__ edge, int np, double *__restrict__ X)
-{
+	const struct td_item &I = set.it[blockIdx.z];
+	const int np = I.np;
 	const int lane = threadIdx.x & 63;
 	const int d = (int) (blockIdx.x * 4 + (threadIdx.x >> 6)) - (np - 1);
-	if(d > np - 1)
+	if(!I.sparse || d > np - 1)
 		return;
+	double *__restrict__ X = I.C;
+	const double *__restrict__ edge = I.edge + (d >= 0 ? d : np - d);
+	double e0 = 0.0;
+#pragma unroll 4
+	for(int c = lane; c < I.nch; c += 64)
+		e0 += edge[(size_t) c * 2 * np];
+	for(int o = 32; o; o >>= 1)
+		e0 += __shfl_xor(e0, o);
 	const int k0 = d >= 0 ? 0 : -d, kp0 = d >= 0 ? d : 0;
 	const int len = np - (d >= 0 ? d : -d);
 	const int seg = (len + 63) / 64, b0 = lane * seg, b1 = b0 + seg < len ? b0 + seg : len;
@@ -250,7 +340,7 @@ __global__ void __launch_bounds__(256) k_td_diag(const double *__restrict__ edge
 		if(lane >= o)
 			incl += u;
 	}
-	double c = (d >= 0 ? edge[d] : edge[np - d]) + (incl - sum);
+	double c = e0 + (incl - sum);
 	for(int e = b0; e < b1; e++) {
 		const double x = X[base + e * step];
 		X[base + e * step] = c;
@@ -258,81 +348,96 @@ __global__ void __launch_bounds__(256) k_td_diag(const double *__restrict__ edge
 	}
 }
 
-/* Upart[kb][q] = sum_{k in block kb} Ta[k][q] sum_k' C[k][k'] Tb[k'][q]:
- * Y = C Tb and its bilinear form with Ta in one pass, for 16 k (block kb)
- * by 64 q per workgroup; each wave takes 4 k, each lane one q.  The 16 C
- * rows go through LDS in chunks of TD_YU_KC (every lane of a wave reads
- * the same element: a broadcast), the Tb row reads are coalesced over q. */
-#define TD_YU_KC 256
+/*
+ * Upart[kb][q] = sum_{k in block kb} Ta[k][q] sum_k' C[k][k'] Tb[k'][q]:
+ * Y = C Tb and its bilinear form with Ta in one pass, 16 k (block kb) by
+ * 16 q per workgroup on v_mfma_f64_16x16x4f64, each of the four waves a
+ * quarter of the k', their Y never added up: the form is linear in Y.
+ * Bound by the latency of its operand loads (L2): many small tiles, eight
+ * loads in flight per lane; one thread per (4 k, q) was a chain of 175
+ * loads, 25 us a baseline at 233 taps and 351 nodes, now 11 for three.
+ * Loads are clamped into the matrices, terms past the end multiply by 0.
+ */
 /* the product rule's node count that k_td_pw's LDS holds */
 #define TD_NQ_MAX 7680
-__global__ void __launch_bounds__(256) k_td_yu(const double *__restrict__ C, const double *__restrict__ Ta, const double *__restrict__ Tb, int np, int nq, double *__restrict__ Upart)
+__global__ void __launch_bounds__(256) k_td_yu(const struct td_set set)
 {
-	__shared__ double Cs[16][TD_YU_KC];
-	__shared__ double red[4][64];
-	const int qi = threadIdx.x & 63, kw = threadIdx.x >> 6;
-	const int q = blockIdx.x * 64 + qi, kb = blockIdx.y, k0 = kb * 16 + kw * 4;
-	double y0 = 0.0, y1 = 0.0, y2 = 0.0, y3 = 0.0;
-	for(int c0 = 0; c0 < np; c0 += TD_YU_KC) {
-		const int nc = np - c0 < TD_YU_KC ? np - c0 : TD_YU_KC;
-		__syncthreads();
-		for(int e = threadIdx.x; e < 16 * TD_YU_KC; e += 256) {
-			const int r = e / TD_YU_KC, c = e % TD_YU_KC, k = kb * 16 + r;
-			Cs[r][c] = (k < np && c < nc) ? C[(size_t) k * np + c0 + c] : 0.0;
+	typedef double v4 __attribute__((ext_vector_type(4)));
+	__shared__ double red[4][16];
+	const struct td_item &I = set.it[blockIdx.z];
+	const int np = I.np, nq = I.nq, q0 = blockIdx.x * 16, kb = blockIdx.y, k0 = kb * 16;
+	if(q0 >= nq || k0 >= np)
+		return;
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, lk = lane >> 4;
+	const int q = q0 + li < nq ? q0 + li : nq - 1, ka = k0 + li < np ? k0 + li : np - 1;
+	const int per = (np + 15) / 16 * 4, cb = wave * per, ce = cb + per < np ? cb + per : np;
+	const double *__restrict__ A = I.C + (size_t) ka * np, *__restrict__ B = I.Tb + q;
+	v4 acc = (v4) 0;
+	for(int c0 = cb; c0 < ce; c0 += 16) {
+		double af[4], bf[4];
+#pragma unroll
+		for(int i = 0; i < 4; i++) {
+			const int c = c0 + 4 * i + lk, cc = c < ce ? c : ce - 1;
+			af[i] = A[cc];
+			bf[i] = B[(size_t) cc * nq];
+			af[i] = c < ce ? af[i] : 0.0;
+			bf[i] = c < ce ? bf[i] : 0.0;
 		}
-		__syncthreads();
-		if(q < nq) {
-			const double *tb = Tb + (size_t) c0 * nq + q;
-#pragma unroll 4
-			for(int c = 0; c < nc; c++) {
-				const double b = tb[(size_t) c * nq];
-				y0 = fma(Cs[kw * 4 + 0][c], b, y0);
-				y1 = fma(Cs[kw * 4 + 1][c], b, y1);
-				y2 = fma(Cs[kw * 4 + 2][c], b, y2);
-				y3 = fma(Cs[kw * 4 + 3][c], b, y3);
-			}
-		}
+#pragma unroll
+		for(int i = 0; i < 4; i++)
+			acc = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i], bf[i], acc, 0, 0, 0);
 	}
 	double u = 0.0;
-	if(q < nq) {
-		const double y[4] = { y0, y1, y2, y3 };
-		for(int j = 0; j < 4; j++)
-			if(k0 + j < np)
-				u = fma(Ta[(size_t) (k0 + j) * nq + q], y[j], u);
+#pragma unroll
+	for(int e = 0; e < 4; e++) {
+		const int k = k0 + lk + 4 * e;
+		const double t = I.Ta[(size_t) (k < np ? k : np - 1) * nq + q];
+		u = k < np ? fma(t, acc[e], u) : u;
 	}
-	red[kw][qi] = u;
+	u += __shfl_xor(u, 16);
+	u += __shfl_xor(u, 32);
+	if(lk == 0)
+		red[wave][li] = u;
 	__syncthreads();
-	if(kw == 0 && q < nq)
-		Upart[(size_t) kb * nq + q] = (red[0][qi] + red[1][qi]) + (red[2][qi] + red[3][qi]);
+	if(threadIdx.x < 16 && q0 + li < nq)
+		I.U[(size_t) kb * nq + q] = (red[0][li] + red[1][li]) + (red[2][li] + red[3][li]);
 }
 
 /* power[d] = sum_q U_q WP[q][d] with U_q = sum_kb Upart[kb][q] (stored as
  * the complex power[d] + 0 i): 16 d per workgroup, the q sum split 16
- * ways; every workgroup first sums U into LDS (nq doubles, dynamic) */
-__global__ void __launch_bounds__(256) k_td_pw(const double *__restrict__ Upart, int nkb, const double *__restrict__ WP, int nq, int P, double *__restrict__ power)
+ * ways; every workgroup first sums U into LDS (nq doubles, dynamic).  Both
+ * sums are chains of L2 loads, four in flight (14.5 us a baseline, now 8.6
+ * for three). */
+__global__ void __launch_bounds__(256) k_td_pw(const struct td_set set)
 {
 	extern __shared__ double Us[];
 	__shared__ double red[16][16];
+	const struct td_item &I = set.it[blockIdx.z];
+	const int nq = I.nq, P = I.P, nkb = (I.np + 15) / 16;
+	if((int) blockIdx.x * 16 > P)
+		return;
+	const double *__restrict__ Upart = I.U, *__restrict__ WP = I.WP;
 	for(int q = threadIdx.x; q < nq; q += 256) {
 		double u = 0.0;
+#pragma unroll 4
 		for(int kb = 0; kb < nkb; kb++)
 			u += Upart[(size_t) kb * nq + q];
 		Us[q] = u;
 	}
 	__syncthreads();
-	const int di = threadIdx.x & 15, qs = threadIdx.x >> 4, d = blockIdx.x * 16 + di;
+	const int di = threadIdx.x & 15, qs = threadIdx.x >> 4, d = blockIdx.x * 16 + di, dc = d <= P ? d : P;
 	double s = 0.0;
-	if(d <= P)
-		for(int q = qs; q < nq; q += 16)
-			s = fma(Us[q], WP[(size_t) q * (P + 1) + d], s);
+#pragma unroll 4
+	for(int q = qs; q < nq; q += 16)
+		s = fma(Us[q], WP[(size_t) q * (P + 1) + dc], s);
 	red[qs][di] = s;
 	__syncthreads();
 	if(qs == 0 && d <= P) {
 		double t = 0.0;
 		for(int g = 0; g < 16; g++)
 			t += red[g][di];
-		power[2 * d] = t;
-		power[2 * d + 1] = 0.0;
+		I.pow[2 * d] = t;
+		I.pow[2 * d + 1] = 0.0;
 	}
 }
 
@@ -342,7 +447,7 @@ __global__ void __launch_bounds__(256) k_td_pw(const double *__restrict__ Upart,
 
 static void td_dev_free(struct td_plan *p)
 {
-	double *b[] = { p->d_Ta, p->d_Tb, p->d_WP, p->d_a, p->d_b, p->d_w, p->d_part, p->d_C, p->d_U, p->d_powc, p->d_rows, p->d_out, p->d_sv, p->d_edge, p->d_nts, p->d_nws };
+	double *b[] = { p->d_Ta, p->d_Tb, p->d_WP, p->d_a, p->d_b, p->d_w, p->d_part, p->d_C, p->d_U, p->d_powc, p->d_rows, p->d_out, p->d_sv, p->d_edge, p->d_nts, p->d_nws, p->d_npow };
 	for(unsigned i = 0; i < sizeof(b) / sizeof(b[0]); i++)
 		if(b[i])
 			(void) hipFree(b[i]);
@@ -475,18 +580,6 @@ static int grow(double **buf, size_t *cap, size_t need)
 	return 0;
 }
 
-/* the plan's power (complex, in d_powc) from device copies of the series
- * a, b (n samples) and window w (n - 2 transient; hw: the same window in
- * host memory, or NULL); launches only.  nnz is td_window_nnz of the
- * window: when it is not -1 the window is not read from w but rebuilt
- * there (w is then a device buffer of nt doubles to fill).
- *
- * With v[s] = w[s - 1] - w[s] for s = 0..nt (w = 0 outside [0, nt)),
- * C[k + 1][k' + 1] - C[k][k'] = sum_s v[s] a[s + k] b[s + k'] exactly.  For
- * windows that are constant over most of the series (the square and
- * Tukey windows of the reference's stitching) v has few nonzeros: the
- * correlation kernel then runs over that support only, and C follows from
- * its first row and column along the diagonals. */
 /* the number of nonzero first differences of the host window hw (nt
  * samples) when the flat-window route applies to a plan of np taps, else
  * -1 */
@@ -501,72 +594,137 @@ static int td_window_nnz(const double *hw, int nt, int np)
 	return nnz;
 }
 
-static int td_power_dev(const double *a, const double *b, double *w, const double *hw, int nnz, int n, struct td_plan *p)
+/* one baseline of td_power_dev: its plan, device copies of its series,
+ * its window in host memory and, where nnz (td_window_nnz) is -1, on the
+ * device; pow takes P + 1 complex values */
+struct td_call {
+	struct td_plan *p;
+	const double *a, *b, *hw, *w;
+	double *pow;
+	int nnz;
+};
+
+/*
+ * The powers of m baselines over n samples.
+ *
+ * With v[s] = w[s - 1] - w[s] for s = 0..nt (w = 0 outside [0, nt)),
+ * C[k + 1][k' + 1] - C[k][k'] = sum_s v[s] a[s + k] b[s + k'] exactly.  For
+ * windows that are constant over most of the series (the square and
+ * Tukey windows of the reference's stitching) v has few nonzeros: the
+ * correlation kernel then runs over that support only, and C follows from
+ * its first row and column along the diagonals.  The differences of all
+ * windows go to the device in one copy, into owner's buffer; the kernels
+ * then run back to back.
+ */
+static int td_power_dev(struct td_call *call, int m, int n, struct td_plan *owner)
 {
-	const int np = p->np, nq = p->nq, nt = n - 2 * p->pub.transient;
 	hipStream_t st = sphr_rt_stream();
-	const int sparse = nnz >= 0;
-	const double *cw = w, *sidx = NULL;
-	int nk = nt;
-	if(sparse) {
-		/* values, offsets and running sums of the window's differences */
-		double *hv = (double *) malloc(3 * (size_t) (nnz > 0 ? nnz : 1) * sizeof(double));
+	size_t nsv = 0;
+	for(int k = 0; k < m; k++)
+		nsv += call[k].nnz > 0 ? 3 * (size_t) call[k].nnz : 0;
+	if(grow(&owner->d_sv, &owner->cap_sv, nsv ? nsv : 1))
+		return -1;
+	if(nsv) {
+		/* values, offsets and running sums of each window's differences */
+		double *hv = (double *) malloc(nsv * sizeof(double)), *v = hv;
 		if(!hv)
 			return -1;
-		double run = 0.0;
-		for(int s = 0, e = 0; s <= nt; s++) {
-			const double v = (s > 0 ? hw[s - 1] : 0.0) - (s < nt ? hw[s] : 0.0);
-			if(v != 0.0) {
-				run += v;
-				hv[e] = v;
-				hv[nnz + e] = (double) s;
-				hv[2 * nnz + e++] = run;
+		for(int k = 0; k < m; k++) {
+			const double *hw = call[k].hw;
+			const int nt = n - 2 * call[k].p->pub.transient, nnz = call[k].nnz;
+			if(nnz <= 0)
+				continue;
+			double run = 0.0;
+			for(int s = 0, e = 0; s <= nt; s++) {
+				const double x = (s > 0 ? hw[s - 1] : 0.0) - (s < nt ? hw[s] : 0.0);
+				if(x != 0.0) {
+					run += x;
+					v[e] = x;
+					v[nnz + e] = (double) s;
+					v[2 * nnz + e++] = run;
+				}
 			}
+			v += 3 * (size_t) nnz;
 		}
-		const int rc = grow(&p->d_sv, &p->cap_sv, 3 * (size_t) (nnz > 0 ? nnz : 1)) || (nnz > 0 && sphr_memcpy_htod(p->d_sv, hv, 3 * (size_t) nnz * sizeof(double)));
+		const int rc = sphr_memcpy_htod(owner->d_sv, hv, nsv * sizeof(double));
 		free(hv);
-		if(rc || grow(&p->d_edge, &p->cap_edge, 2 * (size_t) np))
+		if(rc)
 			return -1;
-		cw = p->d_sv;
-		sidx = p->d_sv + nnz;
-		nk = nnz;
-		/* the window itself, for the first row and column */
-		hipLaunchKernelGGL(k_td_wfill, dim3((nt + 255) / 256), dim3(256), 0, st, sidx, p->d_sv + 2 * nnz, nnz, nt, w);
 	}
-	/* K splits of about TD_TSPLIT terms, enough workgroups on a short
-	 * series; on a long one at most eight workgroups per CU's worth of
-	 * splits, each then longer, so the partial sums (nz np^2 doubles)
-	 * stay bounded whatever the stream's length */
-	const int tiles = (np + TD_TILE - 1) / TD_TILE;
-	int nz = (nk + TD_TSPLIT - 1) / TD_TSPLIT;
-	const int nz_max = 8 * (sphr_rt_cus() > 0 ? sphr_rt_cus() : 256) / (tiles * tiles);
-	if(nz > nz_max)
-		nz = nz_max;
-	if(nz < 1)
-		nz = 1;
-	const int tpz = ((nk + nz - 1) / nz + TD_KC - 1) / TD_KC * TD_KC;
-	nz = nk > 0 ? (nk + tpz - 1) / tpz : 1;
-	/* d_part holds the K-split partials of C, then (sparse windows) the
-	 * chunk sums of its first row and column: sized once for both, before
-	 * any launch */
-	const int nch = (nt + TD_EC - 1) / TD_EC;
-	const size_t need = (size_t) nz * np * np > (size_t) nch * 2 * np ? (size_t) nz * np * np : (size_t) nch * 2 * np;
-	if(grow(&p->d_part, &p->cap_part, need))
-		return -1;
-	if(nk > 0)
-		hipLaunchKernelGGL(k_td_corr, dim3(tiles * tiles * nz), dim3(256), 0, st, a, b, cw, sidx, n, nk, np, tpz, tiles, p->d_part);
-	else
-		(void) hipMemsetAsync(p->d_part, 0, (size_t) np * np * sizeof(double), st);
-	const long nc = (long) np * np;
-	hipLaunchKernelGGL(k_td_reduce, dim3((nc + 255) / 256), dim3(256), 0, st, p->d_part, nk > 0 ? nz : 1, nc, p->d_C);
-	if(sparse) {
-		hipLaunchKernelGGL(k_td_edge, dim3(nch), dim3(256), 0, st, a, b, w, nt, n, np, p->d_part);
-		hipLaunchKernelGGL(k_td_reduce, dim3((2 * np + 255) / 256), dim3(256), 0, st, p->d_part, nch, (long) 2 * np, p->d_edge);
-		hipLaunchKernelGGL(k_td_diag, dim3((2 * np - 1 + 3) / 4), dim3(256), 0, st, p->d_edge, np, p->d_C);
+	const double *sv = owner->d_sv;
+	for(int k0 = 0; k0 < m; k0 += TD_SET) {
+		const int g = m - k0 < TD_SET ? m - k0 : TD_SET;
+		struct td_set set;
+		memset(&set, 0, sizeof(set));
+		unsigned corr = 0, red = 0, nch = 0, jb = 0, diag = 0, qb = 0, kb = 0, db = 0;
+		size_t lds = 0;
+		for(int k = 0; k < g; k++) {
+			const struct td_call *c = call + k0 + k;
+			struct td_plan *p = c->p;
+			struct td_item *I = &set.it[k];
+			const int np = p->np;
+			I->a = c->a;
+			I->b = c->b;
+			I->w = c->w;
+			I->sparse = c->nnz >= 0;
+			I->nnz = I->sparse ? c->nnz : 0;
+			I->sv = sv;
+			sv += 3 * (size_t) I->nnz;
+			I->nt = n - 2 * p->pub.transient;
+			I->np = np;
+			I->nq = p->nq;
+			I->P = p->P;
+			I->nk = I->sparse ? I->nnz : I->nt;
+			/* K splits of about TD_TSPLIT terms, enough workgroups on a
+			 * short series; on a long one at most eight workgroups per
+			 * CU's worth of splits, each then longer, so the partial sums
+			 * (nz np^2 doubles) stay bounded whatever the stream's
+			 * length */
+			I->tiles = (np + TD_TILE - 1) / TD_TILE;
+			int nz = (I->nk + TD_TSPLIT - 1) / TD_TSPLIT;
+			const int nz_max = 8 * (sphr_rt_cus() > 0 ? sphr_rt_cus() : 256) / (I->tiles * I->tiles);
+			if(nz > nz_max)
+				nz = nz_max;
+			if(nz < 1)
+				nz = 1;
+			I->tpz = ((I->nk + nz - 1) / nz + TD_KC - 1) / TD_KC * TD_KC;
+			I->nz = I->nk > 0 ? (I->nk + I->tpz - 1) / I->tpz : 1;
+			I->spc = ((I->nt + TD_NCH_MAX - 1) / TD_NCH_MAX + TD_EC - 1) / TD_EC * TD_EC;
+			I->nch = I->sparse ? (I->nt + I->spc - 1) / I->spc : 0;
+			if(grow(&p->d_part, &p->cap_part, I->nz > 1 ? (size_t) I->nz * np * np : 1) || grow(&p->d_edge, &p->cap_edge, (size_t) (I->nch ? I->nch : 1) * 2 * np))
+				return -1;
+			I->part = p->d_part;
+			I->edge = p->d_edge;
+			I->C = p->d_C;
+			I->U = p->d_U;
+			I->pow = c->pow;
+			I->Ta = p->d_Ta;
+			I->Tb = p->d_Tb;
+			I->WP = p->d_WP;
+			auto most = [](unsigned &x, unsigned y) { x = y > x ? y : x; };
+			most(corr, (unsigned) (I->tiles * I->tiles * I->nz));
+			if(I->nz > 1)
+				most(red, (unsigned) (((long) np * np + 255) / 256));
+			if(I->sparse) {
+				most(nch, (unsigned) I->nch);
+				most(jb, (unsigned) ((np + TD_EJ - 1) / TD_EJ));
+				most(diag, (unsigned) ((2 * np - 1 + 3) / 4));
+			}
+			most(qb, (unsigned) ((p->nq + 15) / 16));
+			most(kb, (unsigned) ((np + 15) / 16));
+			most(db, (unsigned) ((p->P + 16) / 16));
+			lds = (size_t) p->nq * sizeof(double) > lds ? (size_t) p->nq * sizeof(double) : lds;
+		}
+		hipLaunchKernelGGL(k_td_corr, dim3(corr, 1, g), dim3(256), 0, st, set, n);
+		if(red)
+			hipLaunchKernelGGL(k_td_reduce, dim3(red, 1, g), dim3(256), 0, st, set);
+		if(nch)
+			hipLaunchKernelGGL(k_td_edge, dim3(nch, jb, g), dim3(256), 0, st, set, n);
+		if(diag)
+			hipLaunchKernelGGL(k_td_diag, dim3(diag, 1, g), dim3(256), 0, st, set);
+		hipLaunchKernelGGL(k_td_yu, dim3(qb, kb, g), dim3(256), 0, st, set);
+		hipLaunchKernelGGL(k_td_pw, dim3(db, 1, g), dim3(256), lds, st, set);
 	}
-	const int nkb = (np + 15) / 16;
-	hipLaunchKernelGGL(k_td_yu, dim3((nq + 63) / 64, nkb), dim3(256), 0, st, p->d_C, p->d_Ta, p->d_Tb, np, nq, p->d_U);
-	hipLaunchKernelGGL(k_td_pw, dim3((p->P + 16) / 16), dim3(256), (size_t) nq * sizeof(double), st, p->d_U, nkb, p->d_WP, nq, p->P, p->d_powc);
 	return sphr_rt_check(hipGetLastError(), "time-domain correlator") ? -1 : 0;
 }
 
@@ -582,18 +740,15 @@ static int td_power_1d(const double *ta, const double *tb, const double *window,
 	if(sphr_memcpy_htod(p->d_a, ta, (size_t) n * sizeof(double)) || sphr_memcpy_htod(p->d_b, tb, (size_t) n * sizeof(double))
 	   || (nt > 0 && nnz < 0 && sphr_memcpy_htod(p->d_w, window, (size_t) nt * sizeof(double))))
 		return -1;
-	return td_power_dev(p->d_a, p->d_b, p->d_w, window, nnz, n, p);
+	struct td_call c = { p, p->d_a, p->d_b, window, p->d_w, p->d_powc, nnz };
+	return td_power_dev(&c, 1, n, p);
 }
 
-/* power_1d of the plan set from the device power; buf holds 2 (P + 1)
- * doubles */
-static int td_fetch_power(struct td_plan *p, double *buf)
+/* power_1d of the plan set from its P + 1 complex values */
+static void td_set_power(struct td_plan *p, const double *v)
 {
-	if(sphr_memcpy_dtoh(buf, p->d_powc, 2 * (size_t) (p->P + 1) * sizeof(double)))
-		return -1;
 	for(int d = 0; d <= p->P; d++)
-		sh_series_set(p->pub.power_1d, d, 0, buf[2 * d]);
-	return 0;
+		sh_series_set(p->pub.power_1d, d, 0, v[2 * d]);
 }
 
 /* correlator_baseline_integrate_power_td (correlator.c:648-673) */
@@ -620,7 +775,11 @@ extern "C" struct sh_series *correlator_baseline_integrate_power_td(const double
 			sphr_set_error("rotation launch failed");
 	}
 	if(!rc)
-		rc = td_fetch_power(p, buf) || sphr_memcpy_dtoh(power_2d->coeff, p->d_out, 2 * nsky * sizeof(double));
+		rc = sphr_memcpy_dtoh(buf, p->d_powc, 2 * (size_t) (P + 1) * sizeof(double));
+	if(!rc)
+		td_set_power(p, buf);
+	if(!rc)
+		rc = sphr_memcpy_dtoh(power_2d->coeff, p->d_out, 2 * nsky * sizeof(double));
 	pthread_mutex_unlock(&sphr_dropin_lock);
 	free(buf);
 	if(rc) {
@@ -678,8 +837,10 @@ extern "C" struct sh_series *correlator_network_integrate_power_td(struct sh_ser
 	const int nb = plan->baselines->n_baselines;
 	const int n_inst = instrument_array_len(plan->baselines->baselines[0]->instruments);
 	int tmax = 0, Pmax = 0;
+	size_t npow = 0;
 	for(int k = 0; k < nb; k++) {
 		const struct td_plan *p = (const struct td_plan *) plan->plans[k];
+		npow += 2 * (size_t) (p->P + 1);
 		tmax = p->pub.transient > tmax ? p->pub.transient : tmax;
 		Pmax = p->P > Pmax ? p->P : Pmax;
 	}
@@ -689,43 +850,44 @@ extern "C" struct sh_series *correlator_network_integrate_power_td(struct sh_ser
 	const int L = (int) sky->l_max;
 	const size_t nsky = (size_t) (L + 1) * (L + 1);
 	const int nchunk = (nb + SPHR_MAX_BASELINES - 1) / SPHR_MAX_BASELINES;
-	double *buf = (double *) malloc(2 * (size_t) (Pmax + 1) * sizeof(double));
+	double *buf = (double *) malloc(npow * sizeof(double));
+	struct td_call *call = (struct td_call *) calloc(nb, sizeof(*call));
 	double *part = nchunk > 1 ? (double *) malloc(2 * nsky * sizeof(double)) : NULL;
 	struct td_plan *p0 = (struct td_plan *) plan->plans[0];
-	int rc = !buf || (nchunk > 1 && !part);
+	int rc = !buf || !call || (nchunk > 1 && !part);
 	pthread_mutex_lock(&sphr_dropin_lock);
 	if(!rc)
-		rc = grow(&p0->d_nts, &p0->cap_nts, (size_t) n_inst * tseries_length) || grow(&p0->d_nws, &p0->cap_nws, (size_t) nb * tseries_length);
+		rc = grow(&p0->d_nts, &p0->cap_nts, (size_t) n_inst * tseries_length) || grow(&p0->d_nws, &p0->cap_nws, (size_t) nb * tseries_length)
+		     || grow(&p0->d_npow, &p0->cap_npow, npow);
 	double *dts = p0->d_nts, *dws = p0->d_nws;
 	for(int i = 0; i < n_inst && !rc; i++)
 		rc = sphr_memcpy_htod(dts + (size_t) i * tseries_length, tseries[i], (size_t) tseries_length * sizeof(double));
 	/* windows flat over most of the series are rebuilt on the device from
 	 * their differences; the others are copied */
-	int nnzs[SPHR_MAX_BASELINES];
-	for(int k = 0; k < nb && !rc; k++) {
-		const int nt = tseries_length - 2 * plan->plans[k]->transient;
-		const int nnz = td_window_nnz(windows[k], nt, ((const struct td_plan *) plan->plans[k])->np);
-		if(k < SPHR_MAX_BASELINES)
-			nnzs[k] = nnz;
-		rc = nt > 0 && (k >= SPHR_MAX_BASELINES || nnz < 0) && sphr_memcpy_htod(dws + (size_t) k * tseries_length, windows[k], (size_t) nt * sizeof(double));
-	}
+	size_t at = 0;
 	int k = 0;
 	for(int i = 1; i < n_inst && !rc; i++)
-		for(int j = 0; j < i && !rc; j++, k++)
-			rc = td_power_dev(dts + (size_t) i * tseries_length, dts + (size_t) j * tseries_length, dws + (size_t) k * tseries_length, windows[k],
-					  k < SPHR_MAX_BASELINES ? nnzs[k] : -1, tseries_length, (struct td_plan *) plan->plans[k]);
-	for(k = 0; k < nb && !rc; k++)
-		rc = td_fetch_power((struct td_plan *) plan->plans[k], buf);
-	if(!rc && (sky->polar || L < Pmax))
-		rc = -1;
+		for(int j = 0; j < i && !rc; j++, k++) {
+			struct td_plan *p = (struct td_plan *) plan->plans[k];
+			const int nt = tseries_length - 2 * p->pub.transient;
+			const int nnz = td_window_nnz(windows[k], nt, p->np);
+			const struct td_call c = { p, dts + (size_t) i * tseries_length, dts + (size_t) j * tseries_length, windows[k], dws + (size_t) k * tseries_length, p0->d_npow + at, nnz };
+			call[k] = c;
+			at += 2 * (size_t) (p->P + 1);
+			rc = nt > 0 && nnz < 0 && sphr_memcpy_htod(dws + (size_t) k * tseries_length, windows[k], (size_t) nt * sizeof(double));
+		}
 	if(!rc)
+		rc = td_power_dev(call, k, tseries_length, p0);
+	/* the sky is refused after the powers are set */
+	const int refused = sky->polar || L < Pmax;
+	if(!rc && !refused)
 		rc = grow(&p0->d_out, &p0->cap_out, 2 * nsky * nchunk);
-	for(int c = 0; c < nchunk && !rc; c++) {
+	for(int c = 0; c < nchunk && !rc && !refused; c++) {
 		const cplx<double> *pw[SPHR_MAX_BASELINES], *bk[SPHR_MAX_BASELINES];
 		int Lb[SPHR_MAX_BASELINES], pol[SPHR_MAX_BASELINES], m = 0;
 		for(k = c * SPHR_MAX_BASELINES; k < nb && m < SPHR_MAX_BASELINES; k++, m++) {
 			const struct td_plan *p = (const struct td_plan *) plan->plans[k];
-			pw[m] = (const cplx<double> *) p->d_powc;
+			pw[m] = (const cplx<double> *) call[k].pow;
 			bk[m] = (const cplx<double> *) p->d_rows;
 			Lb[m] = p->P;
 			pol[m] = 1;
@@ -733,6 +895,14 @@ extern "C" struct sh_series *correlator_network_integrate_power_td(struct sh_ser
 		rc = launch_rotsum(m, pw, Lb, pol, bk, L, 1.0 / nb, (cplx<double> *) p0->d_out + nsky * c, sphr_rt_stream());
 		if(rc)
 			sphr_set_error("rotation launch failed");
+	}
+	if(!rc)
+		rc = sphr_memcpy_dtoh(buf, p0->d_npow, npow * sizeof(double));
+	if(!rc) {
+		const double *v = buf;
+		for(k = 0; k < nb; v += 2 * (size_t) (((struct td_plan *) plan->plans[k])->P + 1), k++)
+			td_set_power((struct td_plan *) plan->plans[k], v);
+		rc = refused ? -1 : 0;
 	}
 	for(int c = 0; c < nchunk && !rc; c++) {
 		double *dst = c ? part : (double *) sky->coeff;
@@ -742,6 +912,7 @@ extern "C" struct sh_series *correlator_network_integrate_power_td(struct sh_ser
 	}
 	pthread_mutex_unlock(&sphr_dropin_lock);
 	free(buf);
+	free(call);
 	free(part);
 	if(rc) {
 		sh_series_zero(sky);

@@ -240,3 +240,73 @@ def test_gpu_td_long_stream_bounded_splits():
     p_2 = _integrate(plan, a[s:], b[s:], w[s:])
     assert rel(p_1 + p_2, p_full) < 1e-11, rel(p_1 + p_2, p_full)
     S.lib().correlator_plan_td_free(plan)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rate,extra", [(4096, 2), (4096, 255), (4096, 256), (4096, 257), (4096, 1024 * 256 + 300), (65536, 700)])
+def test_gpu_td_window_route_edges(rate, extra):
+    """The window-difference route at the edges of its chunks (256 samples,
+    longer ones past 1024 chunks) and of its blocks of 256 taps (367 taps
+    at 65536 samples/s): a window w of few steps gives the sum of the
+    calls with r and w - r, r random, which take the full correlation (the
+    power is linear in the window; three summation orders agree to 1e-11)."""
+    print("td window edges", rate, extra, flush=True)
+    net = _Net(POS[:2])
+    plan = S.lib().correlator_plan_td_new(net.baseline(0), 1.0 / rate)
+    tr = plan.contents.transient
+    assert (2 * tr + 1 > 256) == (rate > 4096)
+    rng = np.random.default_rng(extra)
+    a, b = rng.standard_normal(extra + 2 * tr), rng.standard_normal(extra + 2 * tr)
+    r = rng.uniform(0.5, 1.0, extra) / extra
+    step = np.where(np.arange(extra) < extra // 2, 2.0, 0.5) / extra
+    last = np.zeros(extra)
+    last[-1] = 1.0
+    for w in (np.full(extra, 1.0 / extra), step, last):
+        got, p0, p1 = _integrate(plan, a, b, w), _integrate(plan, a, b, r), _integrate(plan, a, b, w - r)
+        assert rel(got, p0 + p1) < 1e-11 * (1 + np.linalg.norm(p0) / np.linalg.norm(got))
+    # an all-zero window has no differences: the power is exactly zero
+    assert not np.any(_integrate(plan, a, b, np.zeros(extra)))
+    S.lib().correlator_plan_td_free(plan)
+
+
+@pytest.mark.gpu
+def test_gpu_td_network_groups():
+    """ten baselines (more than one launch holds), flat and random windows
+    mixed: every baseline's power is bit for bit that of its own call, the
+    sky their average"""
+    print("td network of five", flush=True)
+    rng = np.random.default_rng(9)
+    v = rng.standard_normal((5, 3))
+    pos = np.linalg.norm(POS[0]) * v / np.linalg.norm(v, axis=1, keepdims=True)
+    net = _Net(pos)
+    L = S.lib()
+    plan = L.correlator_network_plan_td_new(net.bl, DT)
+    assert plan, S.last_error()
+    trs = [plan.contents.plans[k].contents.transient for k in range(10)]
+    lmax = max(plan.contents.plans[k].contents.power_1d.contents.l_max for k in range(10))
+    n = 2 * max(trs) + 900
+    ts = rng.standard_normal((5, n))
+    wins = [_window(L, ("square", "random", "tukey")[k % 3], n - 2 * t, rng) for k, t in enumerate(trs)]
+    tp = (ctypes.c_void_p * 5)(*[ts[i].ctypes.data for i in range(5)])
+    wp = (ctypes.c_void_p * 10)(*[w.ctypes.data for w in wins])
+    sky = L.sh_series_new(lmax, 0)
+    assert L.correlator_network_integrate_power_td(sky, tp, n, wp, plan), S.last_error()
+    powers = [S.coeff_view(plan.contents.plans[k].contents.power_1d).copy() for k in range(10)]
+    k = 0
+    mean = np.zeros((lmax + 1) ** 2, np.complex128)
+    for i in range(1, 5):
+        for j in range(i):
+            r = L.correlator_baseline_integrate_power_td(ts[i].ctypes.data, ts[j].ctypes.data, wins[k].ctypes.data, n, plan.contents.plans[k])
+            assert r, S.last_error()
+            assert np.array_equal(S.coeff_view(plan.contents.plans[k].contents.power_1d), powers[k]), k
+            got, lb, at = S.coeff_view(r), r.contents.l_max, 0
+            for m in list(range(lb + 1)) + list(range(-lb, 0)):
+                o = (lmax + 1) * m - m * (m - 1) // 2 if m >= 0 else (lmax + 1) * (lmax + 1 + m) + m * (m - 1) // 2
+                w = lb + 1 - abs(m)
+                mean[o:o + w] += got[at:at + w] / 10
+                at += w
+            L.sh_series_free(r)
+            k += 1
+    assert rel(S.coeff_view(sky), mean) < 1e-13
+    L.sh_series_free(sky)
+    L.correlator_network_plan_td_free(plan)
