@@ -581,17 +581,66 @@ static int grow(double **buf, size_t *cap, size_t need)
 }
 
 /* the number of nonzero first differences of the host window hw (nt
- * samples) when the flat-window route applies to a plan of np taps, else
- * -1 */
-static int td_window_nnz(const double *hw, int nt, int np)
+ * samples) when the flat-window route applies to a plan of np taps, their
+ * offsets in off (room for nt / 2 + 1), else -1.  A flat window is read at
+ * the speed of memory: 64 samples are compared without a branch, and only
+ * blocks with a difference are gone through. */
+static int td_window_nnz(const double *hw, int nt, int np, int *off)
 {
 	if(!hw || nt < 2 || np < 2 || np > TD_EDGE_NP_MAX)
 		return -1;
+	const int most = nt / 2;
 	int nnz = 0;
-	for(int s = 0; s <= nt; s++)
-		if((s > 0 ? hw[s - 1] : 0.0) - (s < nt ? hw[s] : 0.0) != 0.0 && 2 * ++nnz > nt)
+	if(hw[0] != 0.0)
+		off[nnz++] = 0;
+	for(int s0 = 1; s0 < nt; s0 += 64) {
+		const int s1 = s0 + 64 < nt ? s0 + 64 : nt;
+		int any = 0;
+		for(int s = s0; s < s1; s++)
+			any += hw[s - 1] - hw[s] != 0.0;
+		if(!any)
+			continue;
+		if(nnz + any > most)
 			return -1;
+		for(int s = s0; s < s1; s++)
+			if(hw[s - 1] - hw[s] != 0.0)
+				off[nnz++] = s;
+	}
+	if(hw[nt - 1] != 0.0) {
+		if(nnz + 1 > most)
+			return -1;
+		off[nnz++] = nt;
+	}
 	return nnz;
+}
+
+/* host memory on its way to the device: through a pinned buffer where the
+ * call fits in one of TD_PIN_MAX bytes (the copies then run behind the
+ * host's work: with the scan above 451 -> 274 us for 16 s of three sites),
+ * otherwise copied directly.  The buffer belongs to the
+ * runtime, is used under the drop-in lock and is free again once the call
+ * has waited for its stream. */
+#define TD_PIN_MAX ((size_t) 16 << 20)
+struct td_stage {
+	char *p;
+	size_t at, cap;
+};
+
+static struct td_stage td_stage_new(size_t bytes)
+{
+	struct td_stage g = { bytes <= TD_PIN_MAX ? (char *) sphr_rt_pinned(0, bytes) : NULL, 0, bytes };
+	return g;
+}
+
+static int td_upload(struct td_stage *g, double *dst, const double *src, size_t n)
+{
+	const size_t bytes = n * sizeof(double);
+	if(!g->p || g->at + bytes > g->cap)
+		return sphr_memcpy_htod(dst, src, bytes);
+	memcpy(g->p + g->at, src, bytes);
+	const int rc = sphr_rt_check(hipMemcpyAsync(dst, g->p + g->at, bytes, hipMemcpyHostToDevice, sphr_rt_stream()), "hipMemcpy HtoD");
+	g->at += bytes;
+	return rc ? -1 : 0;
 }
 
 /* one baseline of td_power_dev: its plan, device copies of its series,
@@ -602,6 +651,7 @@ struct td_call {
 	const double *a, *b, *hw, *w;
 	double *pow;
 	int nnz;
+	const int *off;		/* the differences' offsets */
 };
 
 /*
@@ -616,7 +666,7 @@ struct td_call {
  * windows go to the device in one copy, into owner's buffer; the kernels
  * then run back to back.
  */
-static int td_power_dev(struct td_call *call, int m, int n, struct td_plan *owner)
+static int td_power_dev(struct td_call *call, int m, int n, struct td_plan *owner, struct td_stage *stage)
 {
 	hipStream_t st = sphr_rt_stream();
 	size_t nsv = 0;
@@ -635,18 +685,17 @@ static int td_power_dev(struct td_call *call, int m, int n, struct td_plan *owne
 			if(nnz <= 0)
 				continue;
 			double run = 0.0;
-			for(int s = 0, e = 0; s <= nt; s++) {
+			for(int e = 0; e < nnz; e++) {
+				const int s = call[k].off[e];
 				const double x = (s > 0 ? hw[s - 1] : 0.0) - (s < nt ? hw[s] : 0.0);
-				if(x != 0.0) {
-					run += x;
-					v[e] = x;
-					v[nnz + e] = (double) s;
-					v[2 * nnz + e++] = run;
-				}
+				run += x;
+				v[e] = x;
+				v[nnz + e] = (double) s;
+				v[2 * nnz + e] = run;
 			}
 			v += 3 * (size_t) nnz;
 		}
-		const int rc = sphr_memcpy_htod(owner->d_sv, hv, nsv * sizeof(double));
+		const int rc = td_upload(stage, owner->d_sv, hv, nsv);
 		free(hv);
 		if(rc)
 			return -1;
@@ -736,12 +785,17 @@ static int td_power_1d(const double *ta, const double *tb, const double *window,
 	if(grow(&p->d_a, &cap_a, (size_t) n) || grow(&p->d_b, &cap_b, (size_t) n) || grow(&p->d_w, &cap_w, (size_t) (nt > 0 ? nt : 1)))
 		return -1;
 	p->cap_n = cap_a < cap_b ? (cap_a < cap_w ? cap_a : cap_w) : (cap_b < cap_w ? cap_b : cap_w);
-	const int nnz = td_window_nnz(window, nt, p->np);
-	if(sphr_memcpy_htod(p->d_a, ta, (size_t) n * sizeof(double)) || sphr_memcpy_htod(p->d_b, tb, (size_t) n * sizeof(double))
-	   || (nt > 0 && nnz < 0 && sphr_memcpy_htod(p->d_w, window, (size_t) nt * sizeof(double))))
+	int *off = (int *) malloc(((size_t) (nt > 0 ? nt : 0) / 2 + 1) * sizeof(int));
+	if(!off)
 		return -1;
-	struct td_call c = { p, p->d_a, p->d_b, window, p->d_w, p->d_powc, nnz };
-	return td_power_dev(&c, 1, n, p);
+	const int nnz = td_window_nnz(window, nt, p->np, off);
+	struct td_stage stage = td_stage_new((2 * (size_t) n + (nnz < 0 ? (size_t) nt : 3 * (size_t) nnz)) * sizeof(double));
+	int rc = td_upload(&stage, p->d_a, ta, (size_t) n) || td_upload(&stage, p->d_b, tb, (size_t) n) || (nt > 0 && nnz < 0 && td_upload(&stage, p->d_w, window, (size_t) nt));
+	struct td_call c = { p, p->d_a, p->d_b, window, p->d_w, p->d_powc, nnz, off };
+	if(!rc)
+		rc = td_power_dev(&c, 1, n, p, &stage);
+	free(off);
+	return rc ? -1 : 0;
 }
 
 /* power_1d of the plan set from its P + 1 complex values */
@@ -780,6 +834,8 @@ extern "C" struct sh_series *correlator_baseline_integrate_power_td(const double
 		td_set_power(p, buf);
 	if(!rc)
 		rc = sphr_memcpy_dtoh(power_2d->coeff, p->d_out, 2 * nsky * sizeof(double));
+	if(rc)
+		(void) hipStreamSynchronize(sphr_rt_stream());
 	pthread_mutex_unlock(&sphr_dropin_lock);
 	free(buf);
 	if(rc) {
@@ -824,6 +880,48 @@ extern "C" void correlator_network_plan_td_free(struct correlator_network_plan_t
 	free(plan);
 }
 
+/* the powers (npow doubles, to buf and the plans) and n doubles of the sky:
+ * through pinned memory the second half arrives as the host empties the
+ * first (16 s of three sites, order 351: 274 us a call; thirds 282, quarters
+ * 292, each copy starting 25 us after the last) */
+#define TD_PARTS 2
+static int td_fetch(struct correlator_network_plan_td *plan, struct td_plan *p0, double *buf, size_t npow, double *sky, size_t n)
+{
+	hipStream_t st = sphr_rt_stream();
+	const size_t bytes = (npow + n) * sizeof(double);
+	double *h = bytes <= TD_PIN_MAX ? (double *) sphr_rt_pinned(1, bytes) : NULL;
+	hipEvent_t ev[TD_PARTS] = { 0 };
+	int rc = 0, np = 0;
+	if(!h)
+		rc = sphr_memcpy_dtoh(buf, p0->d_npow, npow * sizeof(double)) || (n && sphr_memcpy_dtoh(sky, p0->d_out, n * sizeof(double)));
+	else {
+		np = n ? TD_PARTS : 1;
+		rc = sphr_rt_check(hipMemcpyAsync(h, p0->d_npow, npow * sizeof(double), hipMemcpyDeviceToHost, st), "hipMemcpy DtoH") ? -1 : 0;
+		for(int i = 0; i < np && !rc; i++) {
+			const size_t a = n * i / np, b = n * (i + 1) / np;
+			rc = (b > a && sphr_rt_check(hipMemcpyAsync(h + npow + a, p0->d_out + a, (b - a) * sizeof(double), hipMemcpyDeviceToHost, st), "hipMemcpy DtoH"))
+			     || sphr_rt_check(hipEventCreateWithFlags(&ev[i], hipEventDisableTiming), "hipEventCreate") || sphr_rt_check(hipEventRecord(ev[i], st), "hipEventRecord");
+		}
+		for(int i = 0; i < np && !rc; i++) {
+			const size_t a = n * i / np, b = n * (i + 1) / np;
+			rc = sphr_rt_check(hipEventSynchronize(ev[i]), "hipEventSynchronize");
+			if(!rc && i == 0)
+				memcpy(buf, h, npow * sizeof(double));
+			if(!rc)
+				memcpy(sky + a, h + npow + a, (b - a) * sizeof(double));
+		}
+		for(int i = 0; i < np; i++)
+			if(ev[i])
+				(void) hipEventDestroy(ev[i]);
+	}
+	if(rc)
+		return -1;
+	const double *v = buf;
+	for(int k = 0; k < plan->baselines->n_baselines; v += 2 * (size_t) (((struct td_plan *) plan->plans[k])->P + 1), k++)
+		td_set_power((struct td_plan *) plan->plans[k], v);
+	return 0;
+}
+
 /* correlator_network_integrate_power_td (correlator.c:967-984).  The
  * series go to the device once for all baselines, in the first plan's
  * buffers; each baseline's power stays on the device, and one k_rotsum
@@ -860,24 +958,35 @@ extern "C" struct sh_series *correlator_network_integrate_power_td(struct sh_ser
 		rc = grow(&p0->d_nts, &p0->cap_nts, (size_t) n_inst * tseries_length) || grow(&p0->d_nws, &p0->cap_nws, (size_t) nb * tseries_length)
 		     || grow(&p0->d_npow, &p0->cap_npow, npow);
 	double *dts = p0->d_nts, *dws = p0->d_nws;
-	for(int i = 0; i < n_inst && !rc; i++)
-		rc = sphr_memcpy_htod(dts + (size_t) i * tseries_length, tseries[i], (size_t) tseries_length * sizeof(double));
 	/* windows flat over most of the series are rebuilt on the device from
 	 * their differences; the others are copied */
-	size_t at = 0;
+	const size_t ostr = (size_t) tseries_length / 2 + 1;
+	int *off = rc ? NULL : (int *) malloc(nb * ostr * sizeof(int));
+	size_t at = 0, up = (size_t) n_inst * tseries_length;
 	int k = 0;
+	if(!rc && !off)
+		rc = -1;
 	for(int i = 1; i < n_inst && !rc; i++)
-		for(int j = 0; j < i && !rc; j++, k++) {
+		for(int j = 0; j < i; j++, k++) {
 			struct td_plan *p = (struct td_plan *) plan->plans[k];
 			const int nt = tseries_length - 2 * p->pub.transient;
-			const int nnz = td_window_nnz(windows[k], nt, p->np);
-			const struct td_call c = { p, dts + (size_t) i * tseries_length, dts + (size_t) j * tseries_length, windows[k], dws + (size_t) k * tseries_length, p0->d_npow + at, nnz };
+			const int nnz = td_window_nnz(windows[k], nt, p->np, off + k * ostr);
+			const struct td_call c = { p, dts + (size_t) i * tseries_length, dts + (size_t) j * tseries_length, windows[k], dws + (size_t) k * tseries_length, p0->d_npow + at, nnz, off + k * ostr };
 			call[k] = c;
 			at += 2 * (size_t) (p->P + 1);
-			rc = nt > 0 && nnz < 0 && sphr_memcpy_htod(dws + (size_t) k * tseries_length, windows[k], (size_t) nt * sizeof(double));
+			up += nnz < 0 ? (size_t) nt : 3 * (size_t) nnz;
 		}
+	struct td_stage stage = { NULL, 0, 0 };
 	if(!rc)
-		rc = td_power_dev(call, k, tseries_length, p0);
+		stage = td_stage_new(up * sizeof(double));
+	for(int i = 0; i < n_inst && !rc; i++)
+		rc = td_upload(&stage, dts + (size_t) i * tseries_length, tseries[i], (size_t) tseries_length);
+	for(int c = 0; c < k && !rc; c++) {
+		const int nt = tseries_length - 2 * call[c].p->pub.transient;
+		rc = nt > 0 && call[c].nnz < 0 && td_upload(&stage, dws + (size_t) c * tseries_length, windows[c], (size_t) nt);
+	}
+	if(!rc)
+		rc = td_power_dev(call, k, tseries_length, p0, &stage);
 	/* the sky is refused after the powers are set */
 	const int refused = sky->polar || L < Pmax;
 	if(!rc && !refused)
@@ -897,21 +1006,19 @@ extern "C" struct sh_series *correlator_network_integrate_power_td(struct sh_ser
 			sphr_set_error("rotation launch failed");
 	}
 	if(!rc)
-		rc = sphr_memcpy_dtoh(buf, p0->d_npow, npow * sizeof(double));
-	if(!rc) {
-		const double *v = buf;
-		for(k = 0; k < nb; v += 2 * (size_t) (((struct td_plan *) plan->plans[k])->P + 1), k++)
-			td_set_power((struct td_plan *) plan->plans[k], v);
-		rc = refused ? -1 : 0;
-	}
-	for(int c = 0; c < nchunk && !rc; c++) {
-		double *dst = c ? part : (double *) sky->coeff;
-		rc = sphr_memcpy_dtoh(dst, p0->d_out + 2 * nsky * c, 2 * nsky * sizeof(double));
-		for(size_t i = 0; c && !rc && i < 2 * nsky; i++)
+		rc = td_fetch(plan, p0, buf, npow, (double *) sky->coeff, refused ? 0 : 2 * nsky);
+	if(!rc && refused)
+		rc = -1;
+	for(int c = 1; c < nchunk && !rc; c++) {
+		rc = sphr_memcpy_dtoh(part, p0->d_out + 2 * nsky * c, 2 * nsky * sizeof(double));
+		for(size_t i = 0; !rc && i < 2 * nsky; i++)
 			((double *) sky->coeff)[i] += part[i];
 	}
+	if(rc)
+		(void) hipStreamSynchronize(sphr_rt_stream());
 	pthread_mutex_unlock(&sphr_dropin_lock);
 	free(buf);
+	free(off);
 	free(call);
 	free(part);
 	if(rc) {

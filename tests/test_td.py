@@ -243,10 +243,10 @@ def test_gpu_td_long_stream_bounded_splits():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rate,extra", [(4096, 2), (4096, 255), (4096, 256), (4096, 257), (4096, 1024 * 256 + 300), (65536, 700)])
+@pytest.mark.parametrize("rate,extra", [(4096, 2), (4096, 255), (4096, 256), (4096, 257), (4096, 1024 * 256 + 300), (4096, 1200000), (65536, 700)])
 def test_gpu_td_window_route_edges(rate, extra):
     """The window-difference route at the edges of its chunks (256 samples,
-    longer ones past 1024 chunks) and of its blocks of 256 taps (367 taps
+    longer ones past 1024 chunks; the last past the pinned buffer) and of its blocks of 256 taps (367 taps
     at 65536 samples/s): a window w of few steps gives the sum of the
     calls with r and w - r, r random, which take the full correlation (the
     power is linear in the window; three summation orders agree to 1e-11)."""
