@@ -283,27 +283,36 @@ int launch_fft_single(const double *in, int real_input, int N, const cplx<double
 }
 
 /* direct DFT for lengths that are not powers of two; exact twiddle index
- * (j k mod N) into the length-N table */
-__global__ void k_dft_direct(const double *__restrict__ in, int real_input, int N, const cplx<double> *__restrict__ tw, cplx<double> *__restrict__ out)
+ * (j k mod N) into the length-N table.  One wave per frequency, the samples
+ * over its lanes: a frequency per thread was a chain of N loads in N / 256
+ * workgroups (the segment pipeline of three sites: 564 -> 180 us at 1025
+ * samples, 1673 -> 256 at 3000). */
+__global__ void __launch_bounds__(NT) k_dft_direct(const double *__restrict__ in, int real_input, int N, const cplx<double> *__restrict__ tw, cplx<double> *__restrict__ out)
 {
-	const int k = blockIdx.x * blockDim.x + threadIdx.x;
+	const int k = blockIdx.x * (NT / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
 	if(k >= N)
 		return;
 	cplx<double> acc = mk(0.0, 0.0);
-	long t = 0;
-	for(int j = 0; j < N; j++) {
-		const cplx<double> v = real_input ? mk(in[j], 0.0) : mk(in[2 * j], in[2 * j + 1]);
+	const int step = (int) (64L * k % N);
+	int t = (int) ((long) lane * k % N);
+#pragma unroll 4
+	for(int j = lane; j < N; j += 64) {
+		const cplx<double> v = real_input ? mk(in[j], 0.0) : mk(in[2 * (size_t) j], in[2 * (size_t) j + 1]);
 		cfma(acc, v, tw[t]);
-		t += k;
-		if(t >= N)
-			t -= N;
+		t += step;
+		t = t >= N ? t - N : t;
 	}
-	out[k] = acc;
+	for(int o = 32; o; o >>= 1) {
+		acc.re += __shfl_xor(acc.re, o);
+		acc.im += __shfl_xor(acc.im, o);
+	}
+	if(lane == 0)
+		out[k] = acc;
 }
 
 int launch_dft_direct(const double *in, int real_input, int N, const cplx<double> *tw, cplx<double> *out, hipStream_t st)
 {
-	hipLaunchKernelGGL(k_dft_direct, dim3((N + NT - 1) / NT), dim3(NT), 0, st, in, real_input, N, tw, out);
+	hipLaunchKernelGGL(k_dft_direct, dim3((N + NT / 64 - 1) / (NT / 64)), dim3(NT), 0, st, in, real_input, N, tw, out);
 	return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

@@ -543,3 +543,17 @@ def test_gpu_sky_of_a_plan_that_is_not_real():
         maps.append(d_m.to_numpy(np.complex128, (nseg, 2 * L + 2, 2 * L + 2)))
     assert np.linalg.norm(maps[1].imag) > 0.1 * np.linalg.norm(maps[1].real)
     assert rel(maps[0], maps[1]) < 1e-13
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [3, 63, 65, 257, 1000, 1025])
+@pytest.mark.parametrize("cplx", [False, True])
+def test_gpu_direct_dft_lengths(n, cplx):
+    """Transforms of lengths that are not powers of two, a wave per
+    frequency: at the edges of its 64 lanes, against numpy; a sum of n
+    products carries at most n roundings of each."""
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal(n) + (1j * rng.standard_normal(n) if cplx else 0)
+    got = (S.ctseries_to_fseries if cplx else S.tseries_to_fseries)(x)
+    want = np.fft.fft(x)
+    assert np.max(np.abs(got - want)) < 4 * n * 2.2e-16 * np.sum(np.abs(x))
