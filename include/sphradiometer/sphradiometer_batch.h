@@ -122,7 +122,7 @@ void sphr_loc_info(const struct sphr_loc *, int info[8]);
  * HEALPix maps of many series on the GPU (the pixel-domain output of
  * sh_series_healpix.cc:247-286 and healpix.py:141-171, and the posterior
  * of RapidLocalization.py:498-530).  A plan holds the Legendre tables of
- * order l_max for nside (any nside up to 1024; sphr_healpix_nside gives the
+ * order l_max for nside (any nside up to 4096; sphr_healpix_nside gives the
  * reference's lmax2nside rule).  Layouts (device, row-major):
  *   alm   [n][(l_max+1)^2] complex (float64 pairs for SPHR_FP64, float32
  *         pairs for SPHR_MIXED), the reference coefficient order

@@ -38,7 +38,7 @@
 #include "runtime.h"
 
 #define HP_NT 256
-#define HP_NSIDE_MAX 4096	/* the per-ring form keeps 4 nside twiddles in LDS */
+#define HP_NSIDE_MAX 4096	/* the per-ring form keeps nside twiddles in LDS */
 
 struct sphr_healpix {
 	int L, nside, precision;
@@ -441,101 +441,122 @@ __global__ void k_hm_pixels(struct hm_geom g, T *__restrict__ W)
 	}
 }
 
-/* orders and resolutions without tables: workgroup = one ring x
- * HP_SPW series, the coefficients read from global memory, the ring's
- * twiddles in LDS at exact integer indices (m j mod nphi) */
+/*
+ * Without the tables: workgroup = one ring x HP_SPW series, the coefficients
+ * read from global memory.  The quarter turn shares the pixels' phases as in
+ * k_healpix_mm: with m j = q nphi / 4 + r, exp(2 pi i m j / nphi) is i^q
+ * exp(2 pi i r / nphi), so LDS holds a quarter of the ring's twiddles, at
+ * exact integer indices, and a thread sums the pixels j + k nphi / 4
+ * (k = 0..3) of a series from one read of each m's twiddle and (A, B).
+ * nside twiddles fit beside the (A, B) of any order up to 1500 at nside 4096
+ * (a whole ring's did not in float64).  Bound by the recurrences, which every
+ * ring repeats: one float64 series of order 120 at nside 512 260 us with
+ * whole rings, 205 so; of order 50 at nside 1024 417, 165.
+ */
 template <typename T>
 __global__ void __launch_bounds__(HP_NT) k_healpix_ring(const cplx<T> *__restrict__ alm, int n, int L, int nside, const double *__restrict__ cf, const double *__restrict__ cm, T *__restrict__ map)
 {
 	extern __shared__ __align__(16) unsigned char hp_sm[];
-	const int ring = blockIdx.x + 1, s0 = blockIdx.y * HP_SPW;
+	const int ring = blockIdx.x + 1, s0 = blockIdx.y * HP_SPW, ns = n - s0 < HP_SPW ? n - s0 : HP_SPW;
 	double z, st, phi0;
 	int nphi;
 	long start;
 	hp_ring(nside, ring, &z, &st, &nphi, &start, &phi0);
 	const long npix = 12L * nside * nside;
-	const int ncoef = (L + 1) * (L + 1);
-	T *AB = reinterpret_cast<T *>(hp_sm);				/* [HP_SPW][L + 1][2] */
-	T *tw = AB + 2 * HP_SPW * (L + 1);				/* [nphi][2]: cos, sin */
-	for(int k = threadIdx.x; k < nphi; k += HP_NT) {
+	const int ncoef = (L + 1) * (L + 1), n4 = nphi / 4;
+	cplx<T> *AB = reinterpret_cast<cplx<T> *>(hp_sm);		/* [HP_SPW][L + 1]: (A, B) */
+	cplx<T> *tw = AB + HP_SPW * (L + 1);				/* [n4]: cos, sin */
+	for(int k = threadIdx.x; k < n4; k += HP_NT) {
 		double sn, cs;
 		sincospi(2. * k / nphi, &sn, &cs);
-		tw[2 * k] = (T) cs;
-		tw[2 * k + 1] = (T) sn;
+		tw[k] = mk((T) cs, (T) sn);
 	}
 	/* Legendre sums: thread (series, |m|) */
-	for(int t = threadIdx.x; t < HP_SPW * (L + 1); t += HP_NT) {
-		const int sl = t / (L + 1), m = t - sl * (L + 1), s = s0 + sl;
-		double ar = 0., bi = 0.;
-		if(s < n) {
-			const cplx<T> *a = alm + (size_t) s * ncoef;
-			/* Pbar_mm = cm[m] sin^m theta by repeated products */
-			double p2 = cm[m];
-			for(int k = 0; k < m; k++)
-				p2 *= st;
-			const cplx<T> *ap = a + lm_offset(L, m, m);
-			const cplx<T> *an = m ? a + lm_offset(L, m, -m) : ap;
-			double fpr = (double) ap[0].re * p2, fpi = (double) ap[0].im * p2;
-			double fnr = (double) an[0].re * p2, fni = (double) an[0].im * p2;
-			const double *c = cf + 2 * lm_offset(L, m, m);
-			double p1 = 0.;
-			if(m < L) {
-				p1 = c[2] * z * p2;
-				fpr = fma((double) ap[1].re, p1, fpr);
-				fpi = fma((double) ap[1].im, p1, fpi);
-				fnr = fma((double) an[1].re, p1, fnr);
-				fni = fma((double) an[1].im, p1, fni);
-			}
-			for(int l = m + 2; l <= L; l++) {
-				const int d = l - m;
-				const double p = c[2 * d] * z * p1 - c[2 * d + 1] * p2;
-				fpr = fma((double) ap[d].re, p, fpr);
-				fpi = fma((double) ap[d].im, p, fpi);
-				fnr = fma((double) an[d].re, p, fnr);
-				fni = fma((double) an[d].im, p, fni);
-				p2 = p1;
-				p1 = p;
-			}
-			/* Pbar_l,-m = (-1)^m Pbar_lm; G_+-m = F_+-m exp(+-i m phi_0) */
-			if(m & 1) {
-				fnr = -fnr;
-				fni = -fni;
-			}
-			double sn, cs;
-			sincos(m * phi0, &sn, &cs);
-			const double gpr = fpr * cs - fpi * sn, gpi = fpr * sn + fpi * cs;
-			const double gnr = fnr * cs + fni * sn, gni = -fnr * sn + fni * cs;
-			if(m) {
-				ar = gpr + gnr;
-				bi = gpi - gni;
-			} else {
-				ar = gpr;
-				bi = 0.;
-			}
+	for(int t = threadIdx.x; t < ns * (L + 1); t += HP_NT) {
+		const int sl = t / (L + 1), m = t - sl * (L + 1);
+		const cplx<T> *a = alm + (size_t) (s0 + sl) * ncoef;
+		/* Pbar_mm = cm[m] sin^m theta by repeated products */
+		double p2 = cm[m];
+		for(int k = 0; k < m; k++)
+			p2 *= st;
+		const cplx<T> *ap = a + lm_offset(L, m, m);
+		const cplx<T> *an = m ? a + lm_offset(L, m, -m) : ap;
+		double fpr = (double) ap[0].re * p2, fpi = (double) ap[0].im * p2;
+		double fnr = (double) an[0].re * p2, fni = (double) an[0].im * p2;
+		const double *c = cf + 2 * lm_offset(L, m, m);
+		double p1 = 0.;
+		if(m < L) {
+			p1 = c[2] * z * p2;
+			fpr = fma((double) ap[1].re, p1, fpr);
+			fpi = fma((double) ap[1].im, p1, fpi);
+			fnr = fma((double) an[1].re, p1, fnr);
+			fni = fma((double) an[1].im, p1, fni);
 		}
-		AB[2 * t] = (T) ar;
-		AB[2 * t + 1] = (T) bi;
+		for(int l = m + 2; l <= L; l++) {
+			const int d = l - m;
+			const double p = c[2 * d] * z * p1 - c[2 * d + 1] * p2;
+			fpr = fma((double) ap[d].re, p, fpr);
+			fpi = fma((double) ap[d].im, p, fpi);
+			fnr = fma((double) an[d].re, p, fnr);
+			fni = fma((double) an[d].im, p, fni);
+			p2 = p1;
+			p1 = p;
+		}
+		/* Pbar_l,-m = (-1)^m Pbar_lm; G_+-m = F_+-m exp(+-i m phi_0) */
+		if(m & 1) {
+			fnr = -fnr;
+			fni = -fni;
+		}
+		double sn, cs;
+		sincos(m * phi0, &sn, &cs);
+		const double gpr = fpr * cs - fpi * sn, gpi = fpr * sn + fpi * cs;
+		const double gnr = fnr * cs + fni * sn, gni = -fnr * sn + fni * cs;
+		AB[t] = m ? mk((T) (gpr + gnr), (T) (gpi - gni)) : mk((T) gpr, (T) 0);
 	}
 	__syncthreads();
-	/* pixels: thread (series, j) */
-	for(int t = threadIdx.x; t < HP_SPW * nphi; t += HP_NT) {
-		const int sl = t / nphi, j = t - sl * nphi, s = s0 + sl;
-		if(s >= n)
-			continue;
-		const T *ab = AB + 2 * sl * (L + 1);
-		T v0 = ab[0], v1 = 0;
-		int k = j;	/* m j mod nphi for m = 1 */
-		for(int m = 1; m <= L; m++) {
-			const T c = tw[2 * k], sn = tw[2 * k + 1];
-			if(m & 1)
-				v1 = fma(ab[2 * m], c, fma(-ab[2 * m + 1], sn, v1));
-			else
-				v0 = fma(ab[2 * m], c, fma(-ab[2 * m + 1], sn, v0));
-			k += j;
-			if(k >= nphi)
-				k -= nphi;
+	/* pixels: thread (series, j).  C_m = A_m cos m phi - B_m sin m phi and
+	 * D_m = A_m sin m phi + B_m cos m phi; S_k, T_k their sums over m = k
+	 * mod 4 */
+	for(int t = threadIdx.x; t < ns * n4; t += HP_NT) {
+		const int sl = t / n4, j = t - sl * n4;
+		const cplx<T> *ab = AB + sl * (L + 1);
+		T S0 = ab[0].re, S1 = 0, S2 = 0, S3 = 0, T1 = 0, T3 = 0;
+		int r = j, q = 0;	/* m j = q n4 + r, q mod 4 */
+		auto term = [&](int m, int k) {
+			const cplx<T> e = tw[r], c = ab[m];
+			const T x = q & 1 ? e.im : e.re, y = q & 1 ? e.re : e.im;
+			const T cs = q == 1 || q == 2 ? -x : x, sn = q & 2 ? -y : y;
+			if(k == 0)
+				S0 = fma(c.re, cs, fma(-c.im, sn, S0));
+			else if(k == 2)
+				S2 = fma(c.re, cs, fma(-c.im, sn, S2));
+			else if(k == 1) {
+				S1 = fma(c.re, cs, fma(-c.im, sn, S1));
+				T1 = fma(c.re, sn, fma(c.im, cs, T1));
+			} else {
+				S3 = fma(c.re, cs, fma(-c.im, sn, S3));
+				T3 = fma(c.re, sn, fma(c.im, cs, T3));
+			}
+			r += j;
+			if(r >= n4) {
+				r -= n4;
+				q = (q + 1) & 3;
+			}
+		};
+		int m = 1;
+		for(; m + 3 <= L; m += 4) {
+			term(m, 1);
+			term(m + 1, 2);
+			term(m + 2, 3);
+			term(m + 3, 0);
 		}
-		map[(size_t) s * npix + start + j] = v0 + v1;
+		for(; m <= L; m++)
+			term(m, m & 3);
+		T *o = map + (size_t) (s0 + sl) * npix + start + j;
+		o[0] = (S0 + S2) + (S1 + S3);
+		o[n4] = (S0 - S2) - (T1 - T3);
+		o[2 * n4] = (S0 + S2) - (S1 + S3);
+		o[3 * n4] = (S0 - S2) + (T1 - T3);
 	}
 }
 
@@ -826,16 +847,23 @@ extern "C" int sphr_healpix_maps(const struct sphr_healpix *h, const void *alm, 
 			hipLaunchKernelGGL(k_healpix_mm<double>, dim3(grid), dim3(HM_NT), lds, st, (const cplx<double> *) alm, g, (const double *) h->W, (double *) map);
 	} else {
 		/* one workgroup per (ring, HP_SPW series) */
-		const size_t lr = (2 * HP_SPW * (size_t) (h->L + 1) + 2 * 4 * (size_t) h->nside) * esz;
+		const size_t lr = 2 * (HP_SPW * (size_t) (h->L + 1) + (size_t) h->nside) * esz;
 		if(lr > 160 * 1024) {
 			sphr_set_error("sphr_healpix_maps: l_max %d with nside %d needs %zu bytes of LDS", h->L, h->nside, lr);
 			return -1;
 		}
+		/* where a workgroup's series pass an XCD's L2 (4 MB) and all of
+		 * them together the caches' share of it, LDS keeps the workgroups
+		 * per CU few, which then read less past it (64 float64 series of
+		 * order 400 at nside 256 99 -> 71 ms; with few series more
+		 * workgroups are faster, one of order 300 631 against 724 us) */
+		const size_t one = (size_t) (h->L + 1) * (h->L + 1) * 2 * esz;
+		const size_t lds = HP_SPW * one > (size_t) 4 << 20 && n * one > (size_t) 64 << 20 && lr < 42 * 1024 ? 42 * 1024 : lr;
 		const dim3 grid(4 * h->nside - 1, (n + HP_SPW - 1) / HP_SPW);
 		if(h->precision == SPHR_MIXED)
-			hipLaunchKernelGGL(k_healpix_ring<float>, grid, dim3(HP_NT), lr, st, (const cplx<float> *) alm, n, h->L, h->nside, h->d_cf, h->d_cm, (float *) map);
+			hipLaunchKernelGGL(k_healpix_ring<float>, grid, dim3(HP_NT), lds, st, (const cplx<float> *) alm, n, h->L, h->nside, h->d_cf, h->d_cm, (float *) map);
 		else
-			hipLaunchKernelGGL(k_healpix_ring<double>, grid, dim3(HP_NT), lr, st, (const cplx<double> *) alm, n, h->L, h->nside, h->d_cf, h->d_cm, (double *) map);
+			hipLaunchKernelGGL(k_healpix_ring<double>, grid, dim3(HP_NT), lds, st, (const cplx<double> *) alm, n, h->L, h->nside, h->d_cf, h->d_cm, (double *) map);
 	}
 	return sphr_rt_check(hipGetLastError(), "k_healpix") ? -1 : 0;
 }

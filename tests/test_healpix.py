@@ -17,6 +17,7 @@ import os
 
 import numpy as np
 import pytest
+from scipy.special import sph_harm_y
 
 import sphradiometer_amd as S
 from sphradiometer_amd import healpix as H
@@ -254,6 +255,49 @@ def test_gpu_healpix_series_counts_and_tiles(oracle, L, nside, n):
         assert rel(m64[k], ref) < TOL64, (k, rel(m64[k], ref))
         ref32 = oracle.healpix_map(series[k].astype(np.complex64).astype(np.complex128), L, nside)
         assert rel(m32[k], ref32) < TOL_MIXED, (k, rel(m32[k], ref32))
+
+
+def _ring_values(c, L, nside, ring):
+    """(index of the first pixel, Re f at the centres) of one ring, by
+    direct summation"""
+    N, k = nside, min(ring, 4 * nside - ring)
+    # cap: 1 - cos theta = k^2 / (3 N^2) (acos of z would lose eps / theta)
+    theta = 2 * math.asin(k / (N * math.sqrt(6.0))) if k < N else math.acos(4.0 / 3.0 - 2.0 * k / (3.0 * N))
+    theta = math.pi - theta if ring > 2 * N else theta
+    n = 4 * min(k, N)
+    start = 2 * ring * (ring - 1) if ring < N else 2 * N * (N - 1) + (ring - N) * 4 * N if ring <= 3 * N else 12 * N * N - 2 * k * (k + 1)
+    phi = (np.arange(n) + (0.0 if k >= N and (ring + N) & 1 else 0.5)) * (2 * math.pi / n)
+    out, at = np.zeros(n), 0
+    for m in list(range(L + 1)) + list(range(-L, 0)):
+        for l in range(abs(m), L + 1):
+            out += (c[at] * sph_harm_y(l, m, theta, phi)).real
+            at += 1
+    return start, out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L,nside,n", [(0, 4096, 1), (1, 4096, 1), (2, 3000, 2), (3, 4096, 1), (4, 2300, 5), (8, 4096, 1)])
+def test_gpu_healpix_largest_nside(L, nside, n):
+    """the per-ring form at the largest nside, every remainder of l_max by
+    4 and a count of series that is not a multiple of its four: rings of
+    both caps, at their edges and the equator, of the first and the last
+    series"""
+    print("healpix largest nside L", L, "nside", nside, "n", n, flush=True)
+    rng = np.random.default_rng(nside + L)
+    series = [rand_series(rng, L) for _ in range(n)]
+    for prec, tol in ((S.FP64, TOL64), (S.MIXED, TOL_MIXED)):
+        cdt, rdt = (np.complex128, np.float64) if prec == S.FP64 else (np.complex64, np.float32)
+        hp = S.Healpix(L, nside, prec)
+        d_alm = S.DeviceBuffer.from_numpy(np.array(series).astype(cdt))
+        d_map = S.DeviceBuffer(n * hp.npix * np.dtype(rdt).itemsize)
+        hp.maps(d_alm.ptr, n, d_map.ptr)
+        S.synchronize()
+        for k in sorted({0, n - 1}):
+            for ring in (1, 2, 3, nside - 1, nside, nside + 1, 2 * nside, 3 * nside, 3 * nside + 1, 4 * nside - 1):
+                start, ref = _ring_values(np.array(series[k]).astype(cdt).astype(np.complex128), L, nside, ring)
+                got = d_map.to_numpy(rdt, ref.shape, offset=(k * hp.npix + start) * np.dtype(rdt).itemsize)
+                assert rel(got, ref) < tol, (prec, k, ring, rel(got, ref))
+        d_map.free()
 
 
 @pytest.mark.gpu
