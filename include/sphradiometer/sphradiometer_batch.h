@@ -139,6 +139,11 @@ struct sphr_healpix *sphr_healpix_new(unsigned l_max, int nside, int precision);
 void sphr_healpix_free(struct sphr_healpix *);
 long sphr_healpix_npix(const struct sphr_healpix *);
 int sphr_healpix_maps(const struct sphr_healpix *, const void *alm, int n, void *map, void *stream);
+/* The kernel that sphr_healpix_maps runs for n series: 1 products with the
+ * plan's tables, 0 recurrences per ring (a few series, or a plan whose
+ * tables would be too large); -1 for bad arguments.  Same results to
+ * rounding. */
+int sphr_healpix_form(const struct sphr_healpix *, int n);
 int sphr_healpix_posterior(const struct sphr_healpix *, const void *maps, int n_events, void *prob, void *stream);
 
 /*

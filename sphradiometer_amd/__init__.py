@@ -275,6 +275,7 @@ _PROTOS = {
     "sphr_healpix_free": (None, [c_void_p]),
     "sphr_healpix_npix": (ctypes.c_long, [c_void_p]),
     "sphr_healpix_maps": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p]),
+    "sphr_healpix_form": (c_int, [c_void_p, c_int]),
     "sphr_healpix_posterior": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p]),
     "sphr_loc_info": (None, [c_void_p, P(c_int)]),
 }
@@ -732,6 +733,11 @@ class Healpix:
         """d_alm [n][(l_max+1)^2] complex -> d_map [n][npix] real (device)."""
         if lib().sphr_healpix_maps(self.h, d_alm, n, d_map, stream):
             raise RuntimeError("sphr_healpix_maps failed: " + last_error())
+
+    def form(self, n):
+        """The kernel of maps() for n series (sphr_healpix_form): 1 products
+        with the plan's tables, 0 recurrences per ring."""
+        return lib().sphr_healpix_form(self.h, int(n))
 
     def posterior(self, d_maps, n_events, d_prob, stream=None):
         """d_maps [2][n_events][npix] -> d_prob [n_events][npix] (device)."""

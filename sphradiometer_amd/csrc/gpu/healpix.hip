@@ -21,9 +21,9 @@
  *   f(phi) = sum_m A_m cos(m phi) - B_m sin(m phi),  A_m + i B_m = F_m,
  * so a map is two contractions with tables that all series share: the
  * Legendre values of the rings and the cosines of the pixels.  k_healpix_mm
- * runs both on MFMA, eight series per workgroup (see there); orders and
- * resolutions whose tables would be too large run k_healpix_ring, which
- * forms them by recurrence.
+ * runs both on MFMA, eight series per workgroup (see there); a few series,
+ * and orders and resolutions whose tables would be too large, run
+ * k_healpix_ring, which forms them by recurrence.
  */
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -44,7 +44,7 @@ struct sphr_healpix {
 	int L, nside, precision;
 	double *d_cf;	/* [nal][2]: alpha_lm, alpha_lm / alpha_{l-1,m} at the (l, m >= 0) slots */
 	double *d_cm;	/* [L + 1]: Pbar_mm(cos theta) = cm[m] sin^m theta */
-	/* the tables of k_healpix_mm, NULL where k_healpix_ring runs */
+	/* the tables of k_healpix_mm, NULL (and rc 0) where k_healpix_ring always runs */
 	double *P;	/* Legendre values */
 	void *W;	/* cosines and sines of the pixels */
 	int *off;	/* [L + 1] first step of an order, then [2 nside + 1] first tile of a ring */
@@ -166,10 +166,13 @@ __global__ void __launch_bounds__(HM_NT) k_healpix_mm(const cplx<T> *__restrict_
 	typedef T vec4 __attribute__((ext_vector_type(4)));
 	extern __shared__ __align__(16) unsigned char hm_sm[];
 	T *AB = reinterpret_cast<T *>(hm_sm);	/* [rc][16][ld], then the waves' fetches */
-	/* the chunks of a group of series run on one XCD, side by side */
-	const int id = blockIdx.x, grp = id / (8 * g.chunks) * 8 + id % 8, chunk = id / 8 % g.chunks;
-	if(grp >= g.groups)
-		return;
+	/* workgroups go to the eight XCDs in turn: contiguous ranges of (group
+	 * of series, chunk) per XCD, so that a group's chunks share one L2 and
+	 * a single group still fills the chip (each group on one XCD left the
+	 * others idle below eight groups: eight float64 series of order 160 at
+	 * nside 128 638 -> 178 us, order 200 at nside 256 2597 -> 417) */
+	const int all = gridDim.x & ~7, id = (int) blockIdx.x < all ? (blockIdx.x & 7) * (all >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+	const int grp = id / g.chunks, chunk = id - grp * g.chunks;
 	const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 15, lq = lane >> 4;
 	const int L = g.L, L1 = L + 1, s0 = grp * HM_S, r0 = chunk * g.rc, N2 = 2 * g.nside;
 	/* the columns past the orders multiply zeros of the table: finite */
@@ -827,6 +830,28 @@ extern "C" long sphr_healpix_npix(const struct sphr_healpix *h)
 	return h ? 12L * h->nside * h->nside : -1;
 }
 
+/* which kernel for n series: both times in us from their sizes, fitted to 250
+ * measured shapes (orders 1-300, nside 1-512, 1-1024 series; the faster one
+ * is taken, or one within 15 % of it, at all but six).  k_healpix_mm makes
+ * eight series and sixteen rings at a time whatever it is asked for;
+ * k_healpix_ring's workgroups are independent, but each repeats the
+ * recurrences: one float64 series of order 120 at nside 64 takes 36 us there
+ * and 90 with the tables, nine 194 and 93. */
+static bool use_mm(const struct sphr_healpix *h, const struct hm_geom &g)
+{
+	if(!h->rc)
+		return false;
+	const double terms = (double) (h->L + 1) * (h->L + 1), rings = (double) g.n * h->nside;
+	const double rounds = ceil((double) g.groups * g.chunks / sphr_rt_cus());
+	const double groups = (h->k0 + h->k2 + 2 * h->k1) / 8, pixels = (h->precision == SPHR_MIXED ? 0.010 : 0.014) * (h->rc == 16 ? 2. : 1.);
+	return rounds * (5.5 + 0.0024 * terms + pixels * h->nside * groups) < 4.4 + rings * (2.2e-5 * terms + 6e-4);
+}
+
+extern "C" int sphr_healpix_form(const struct sphr_healpix *h, int n)
+{
+	return h && n > 0 ? use_mm(h, hm_geom_of(h, n)) : -1;
+}
+
 extern "C" int sphr_healpix_maps(const struct sphr_healpix *h, const void *alm, int n, void *map, void *stream)
 {
 	if(!h || !alm || !map || n < 0) {
@@ -837,9 +862,9 @@ extern "C" int sphr_healpix_maps(const struct sphr_healpix *h, const void *alm, 
 		return 0;
 	hipStream_t st = stream ? (hipStream_t) stream : sphr_rt_stream();
 	const size_t esz = h->precision == SPHR_MIXED ? sizeof(float) : sizeof(double);
-	if(h->rc) {
-		const struct hm_geom g = hm_geom_of(h, n);
-		const unsigned grid = (unsigned) ((g.groups + 7) / 8 * 8) * g.chunks;
+	const struct hm_geom g = hm_geom_of(h, n);
+	if(use_mm(h, g)) {
+		const unsigned grid = (unsigned) g.groups * g.chunks;
 		const size_t lds = (size_t) g.rc * g.rs * esz + HM_STAGE;
 		if(h->precision == SPHR_MIXED)
 			hipLaunchKernelGGL(k_healpix_mm<float>, dim3(grid), dim3(HM_NT), lds, st, (const cplx<float> *) alm, g, (const float *) h->W, (float *) map);

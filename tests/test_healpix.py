@@ -257,6 +257,39 @@ def test_gpu_healpix_series_counts_and_tiles(oracle, L, nside, n):
         assert rel(m32[k], ref32) < TOL_MIXED, (k, rel(m32[k], ref32))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("L,nside,n", [(1, 4, 4001), (2, 3, 8001), (3, 17, 1501), (7, 8, 700), (16, 9, 301), (25, 16, 100), (31, 20, 65), (50, 32, 41),
+                                       (63, 33, 23), (64, 16, 65), (100, 8, 63), (129, 40, 9), (200, 16, 25)])
+def test_gpu_healpix_table_products(oracle, L, nside, n):
+    """the products with the plan's tables where both precisions take them:
+    remainders of the groups of eight series, rings on both sides of the
+    16-pixel tiles and 16-ring chunks, every number of rings per workgroup,
+    workgroup counts that are not multiples of the eight XCDs; against the oracle
+    and, for the first series, the per-ring form of one series alone"""
+    rng = np.random.default_rng(3 * L + n)
+    pick = sorted({0, 1, 7, 8, n // 2, n - 1})
+    series = rng.standard_normal((n, (L + 1) ** 2)) + 1j * rng.standard_normal((n, (L + 1) ** 2))
+    for prec, tol in ((S.FP64, TOL64), (S.MIXED, TOL_MIXED)):
+        cdt, rdt = (np.complex128, np.float64) if prec == S.FP64 else (np.complex64, np.float32)
+        print("healpix table products L", L, "nside", nside, "n", n, "precision", prec, flush=True)
+        hp = S.Healpix(L, nside, prec)
+        assert hp.form(n) == 1 and hp.form(1) == 0
+        a = series.astype(cdt)
+        d_alm = S.DeviceBuffer.from_numpy(a)
+        d_map = S.DeviceBuffer(n * hp.npix * np.dtype(rdt).itemsize)
+        d_one = S.DeviceBuffer(hp.npix * np.dtype(rdt).itemsize)
+        hp.maps(d_alm.ptr, n, d_map.ptr)
+        hp.maps(d_alm.ptr, 1, d_one.ptr)
+        S.synchronize()
+        maps = d_map.to_numpy(rdt, (n, hp.npix))
+        assert np.all(np.isfinite(maps))
+        for k in pick:
+            ref = oracle.healpix_map(a[k].astype(np.complex128), L, nside)
+            assert rel(maps[k], ref) < tol, (k, rel(maps[k], ref))
+        one = d_one.to_numpy(rdt, (hp.npix,))
+        assert rel(one, maps[0]) < tol, rel(one, maps[0])
+
+
 def _ring_values(c, L, nside, ring):
     """(index of the first pixel, Re f at the centres) of one ring, by
     direct summation"""
