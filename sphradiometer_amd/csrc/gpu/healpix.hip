@@ -894,16 +894,23 @@ extern "C" int sphr_healpix_maps(const struct sphr_healpix *h, const void *alm, 
 }
 
 /* 1024 threads per event where the events are too few to fill the chip with
- * smaller workgroups (one per CU) */
+ * smaller workgroups (one per CU) and their maps long enough for them; one
+ * wave per event for many maps of at most 1024 pixels (5000 of 12 pixels
+ * 16.4 us with four waves, 9.0 so; 3000 of 768 21.9 and 20.1; one of 768 8.2
+ * with one wave, 5.2 with four) */
 template <typename T>
 static void launch_posterior(const T *maps, int E, long npix, T *prob, hipStream_t st)
 {
 	constexpr int V = 16 / sizeof(T);
 	const bool al = ((uintptr_t) maps | (uintptr_t) prob) % 16 == 0;
-	const bool few = E <= 2 * sphr_rt_cus();
-	if(few && al)
+	const bool small = npix <= 1024, few = E <= 2 * sphr_rt_cus();
+	if(small && !few && al)
+		hipLaunchKernelGGL((k_healpix_posterior<T, V, 64>), dim3(E), dim3(64), 0, st, maps, E, npix, prob);
+	else if(small && !few)
+		hipLaunchKernelGGL((k_healpix_posterior<T, 1, 64>), dim3(E), dim3(64), 0, st, maps, E, npix, prob);
+	else if(!small && few && al)
 		hipLaunchKernelGGL((k_healpix_posterior<T, V, 1024>), dim3(E), dim3(1024), 0, st, maps, E, npix, prob);
-	else if(few)
+	else if(!small && few)
 		hipLaunchKernelGGL((k_healpix_posterior<T, 1, 1024>), dim3(E), dim3(1024), 0, st, maps, E, npix, prob);
 	else if(al)
 		hipLaunchKernelGGL((k_healpix_posterior<T, V, 256>), dim3(E), dim3(256), 0, st, maps, E, npix, prob);

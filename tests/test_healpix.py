@@ -368,6 +368,29 @@ def test_gpu_posterior_special_values(prec, shift):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("nside", [1, 2, 9, 10])
+@pytest.mark.parametrize("E", [3, 1100])
+def test_gpu_posterior_of_small_maps(oracle, nside, E):
+    """maps on both sides of 1024 pixels, for few events and for many (one
+    wave, four and sixteen per event), aligned and not"""
+    rng = np.random.default_rng(nside + E)
+    for prec, rdt, tol in ((S.FP64, np.float64, TOL64), (S.MIXED, np.float32, TOL_MIXED)):
+        for shift in (0, 1):
+            print("posterior of small maps", nside, E, prec, shift, flush=True)
+            hp = S.Healpix(2, nside, prec)
+            m = (rng.standard_normal((2, E, hp.npix)) * 5).astype(rdt)
+            off = shift * m.itemsize
+            d_m, d_p = S.DeviceBuffer(m.nbytes + 16), S.DeviceBuffer(m.nbytes // 2 + 16)
+            d_m.upload(m, offset=off)
+            hp.posterior(d_m.ptr + off, E, d_p.ptr + off)
+            S.synchronize()
+            p = d_p.to_numpy(rdt, (E, hp.npix), offset=off)
+            for e in {0, 1, E // 2, E - 1}:
+                ref = oracle.healpix_posterior(m[0, e].astype(np.float64), m[1, e].astype(np.float64))
+                assert rel(p[e], ref) < tol, (prec, shift, e, rel(p[e], ref))
+
+
+@pytest.mark.gpu
 def test_gpu_write_healpix_map_file(tmp_path, oracle):
     rng = np.random.default_rng(11)
     for L, polar in ((13, False), (9, True)):
