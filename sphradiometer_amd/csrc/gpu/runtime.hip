@@ -138,6 +138,8 @@ int sphr_rt_check(hipError_t e, const char *what)
 {
 	if(e != hipSuccess) {
 		sphr_set_error("%s: %s", what, hipGetErrorString(e));
+		/* reported here: not again by the next call's check of its launches */
+		(void) hipGetLastError();
 		return -1;
 	}
 	return 0;

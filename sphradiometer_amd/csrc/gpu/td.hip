@@ -51,7 +51,7 @@ struct td_plan {
 	double *d_Ta, *d_Tb;		/* [np][nq]: tap projections at the product nodes */
 	double *d_WP;			/* [nq][P + 1]: 2 pi w_q Pbar_d0(x_q) */
 	/* per-call device buffers, grown as needed */
-	size_t cap_n, cap_part;
+	size_t cap_a, cap_b, cap_w, cap_part;
 	double *d_a, *d_b, *d_w, *d_part, *d_C;
 	double *d_U;			/* [ceil(np / 16)][nq]: partial bilinear forms */
 	double *d_powc;			/* power_1d as P + 1 complex (imaginary parts 0) */
@@ -574,6 +574,7 @@ static int grow(double **buf, size_t *cap, size_t need)
 	if(*buf)
 		(void) hipFree(*buf);
 	*buf = NULL;
+	*cap = 0;	/* also where the new buffer cannot be had */
 	if(sphr_rt_check(hipMalloc(buf, need * sizeof(double)), "hipMalloc"))
 		return -1;
 	*cap = need;
@@ -781,10 +782,8 @@ static int td_power_dev(struct td_call *call, int m, int n, struct td_plan *owne
 static int td_power_1d(const double *ta, const double *tb, const double *window, int n, struct td_plan *p)
 {
 	const int nt = n - 2 * p->pub.transient;
-	size_t cap_a = p->cap_n, cap_b = p->cap_n, cap_w = p->cap_n;
-	if(grow(&p->d_a, &cap_a, (size_t) n) || grow(&p->d_b, &cap_b, (size_t) n) || grow(&p->d_w, &cap_w, (size_t) (nt > 0 ? nt : 1)))
+	if(grow(&p->d_a, &p->cap_a, (size_t) n) || grow(&p->d_b, &p->cap_b, (size_t) n) || grow(&p->d_w, &p->cap_w, (size_t) (nt > 0 ? nt : 1)))
 		return -1;
-	p->cap_n = cap_a < cap_b ? (cap_a < cap_w ? cap_a : cap_w) : (cap_b < cap_w ? cap_b : cap_w);
 	int *off = (int *) malloc(((size_t) (nt > 0 ? nt : 0) / 2 + 1) * sizeof(int));
 	if(!off)
 		return -1;

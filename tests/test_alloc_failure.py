@@ -1,0 +1,97 @@
+"""Allocations that fail, on the CPU: the library's host code on a HIP
+runtime in host memory (tests/c/host_hip.c) that fails the n-th device
+allocation and checks every copy against the live ones.  Each test runs in
+a process of its own, where that runtime is loaded first."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def host_hip(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("host_hip") / "libhost_hip.so")
+    cc = os.environ.get("CC", "gcc")
+    r = subprocess.run([cc, "-std=gnu11", "-Wall", "-Wextra", "-Wno-unused-parameter", "-shared", "-fPIC", "-I/opt/rocm/include", "-o", out,
+                        os.path.join(ROOT, "tests", "c", "host_hip.c")], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stderr
+    return out
+
+
+def run(host_hip, body):
+    """body after the runtime and the package are loaded: H, S, lib"""
+    head = """
+        import ctypes, sys
+        H = ctypes.CDLL(%r, mode=ctypes.RTLD_GLOBAL)
+        H.host_hip_fail.argtypes = [ctypes.c_long]
+        for f in ("live", "allocs", "launches"):
+            getattr(H, "host_hip_" + f).restype = ctypes.c_long
+        sys.path.insert(0, %r)
+        import numpy as np
+        import sphradiometer_amd as S
+        from sphradiometer_amd import inject
+        lib = S.lib()
+        assert S.gpu_available(), S.last_error()
+    """ % (host_hip, ROOT)
+    r = subprocess.run([sys.executable, "-c", textwrap.dedent(head) + textwrap.dedent(body)], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+    return r.stdout
+
+
+TD = """
+    inst = lib.instrument_array_new(0)
+    for x, y, z in inject.positions("AB"):
+        lib.instrument_array_append(inst, lib.instrument_new(float(x), float(y), float(z), None))
+    plan = lib.correlator_network_plan_td_new(lib.correlator_network_baselines_new(inst), 1.0 / 512)
+    assert plan, S.last_error()
+    base = plan.contents.plans[0]
+    tr, P = base.contents.transient, base.contents.power_1d.contents.l_max
+    sky = lib.sh_series_new(P, 0)
+
+    def call(n, kind):
+        rng = np.random.default_rng(n)
+        x = [np.ascontiguousarray(rng.standard_normal(n)) for _ in range(2)]
+        nt = n - 2 * tr
+        w = np.ones(nt) if kind == "flat" else rng.uniform(0.5, 1.5, nt)
+        if network:
+            return bool(lib.correlator_network_integrate_power_td(sky, (ctypes.c_void_p * 2)(*[v.ctypes.data for v in x]), n, (ctypes.c_void_p * 1)(w.ctypes.data), plan))
+        s = lib.correlator_baseline_integrate_power_td(x[1].ctypes.data, x[0].ctypes.data, w.ctypes.data, n, base)
+        ok = bool(s)
+        if ok:
+            lib.sh_series_free(s)
+        return ok
+
+    small, n = 2 * tr + 500, 2 * tr + 500
+    assert call(small, "flat") and call(small, "random")
+    failed = 0
+    # every growth of every call fails once; the smaller calls after it run
+    # in whole buffers, and so does the larger one when memory is there
+    for kind in ("flat", "random"):
+        for k in range(1, 12):
+            n = 2 * n
+            H.host_hip_fail(k)
+            ok = call(n, kind)
+            H.host_hip_fail(0)
+            failed += not ok
+            assert call(small, "flat") and call(small, "random"), (kind, k)
+            assert call(n, kind), (kind, k)
+            n = n if n < 400000 else small
+            if n == small:
+                lib.correlator_network_plan_td_free(plan)
+                plan = lib.correlator_network_plan_td_new(lib.correlator_network_baselines_new(inst), 1.0 / 512)
+                base = plan.contents.plans[0]
+                assert call(small, "flat") and call(small, "random")
+    print("failed", failed)
+"""
+
+
+@pytest.mark.parametrize("network", [False, True])
+def test_td_buffers_after_a_failed_growth(host_hip, network):
+    """a growth that fails leaves no capacity behind for the buffer it
+    freed: later calls that fit the old capacity allocate again"""
+    out = run(host_hip, "    network = %r\n" % network + TD)
+    assert int(out.split()[-1]) >= 4, out
