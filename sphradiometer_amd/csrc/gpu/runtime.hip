@@ -107,6 +107,7 @@ void *sphr_rt_scratch(int slot, size_t bytes)
 		if(hipMalloc(&dev_slots[slot].p, want) != hipSuccess) {
 			dev_slots[slot].p = NULL;
 			sphr_set_error("hipMalloc of %zu bytes failed", want);
+			(void) hipGetLastError();	/* reported */
 			return NULL;
 		}
 		dev_slots[slot].n = want;
@@ -127,6 +128,7 @@ void *sphr_rt_pinned(int slot, size_t bytes)
 		if(hipHostMalloc(&host_slots[slot].p, want, hipHostMallocDefault) != hipSuccess) {
 			host_slots[slot].p = NULL;
 			sphr_set_error("hipHostMalloc of %zu bytes failed", want);
+			(void) hipGetLastError();	/* reported */
 			return NULL;
 		}
 		host_slots[slot].n = want;
@@ -172,6 +174,7 @@ extern "C" void *sphr_device_alloc(size_t bytes)
 		return NULL;
 	if(hipMalloc(&p, bytes ? bytes : 1) != hipSuccess) {
 		sphr_set_error("hipMalloc of %zu bytes failed", bytes);
+		(void) hipGetLastError();	/* reported */
 		return NULL;
 	}
 	return p;

@@ -18,10 +18,13 @@ static struct {
 	size_t n;
 } live[MAX_LIVE];
 static long n_live, n_allocs, fail_in, n_launches;
+static int fail_pinned;
 static hipError_t last;	/* kept until it is asked for */
 
 /* the n-th device allocation from now fails (0: none does) */
 void host_hip_fail(long n) { fail_in = n; }
+/* every pinned allocation fails while on */
+void host_hip_fail_pinned(int on) { fail_pinned = on; }
 long host_hip_live(void) { return n_live; }
 long host_hip_allocs(void) { return n_allocs; }
 long host_hip_launches(void) { return n_launches; }
@@ -117,7 +120,13 @@ const char *hipGetErrorString(hipError_t e) { return e == hipSuccess ? "no error
 hipError_t hipDeviceSynchronize(void) { return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t *st, unsigned flags) { (void) flags; *st = (hipStream_t) malloc(1); return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t st) { (void) st; return hipSuccess; }
-hipError_t hipHostMalloc(void **p, size_t n, unsigned flags) { (void) flags; *p = calloc(1, n); return *p ? hipSuccess : hipErrorOutOfMemory; }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned flags)
+{
+	(void) flags;
+	*p = fail_pinned ? NULL : calloc(1, n);
+	return *p ? hipSuccess : (last = hipErrorOutOfMemory);
+}
+
 hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned flags) { (void) flags; *e = (hipEvent_t) malloc(1); return hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t e) { free((void *) e); return hipSuccess; }

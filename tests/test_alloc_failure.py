@@ -42,7 +42,7 @@ def run(host_hip, body):
     return r.stdout
 
 
-TD = """
+TD_PLAN = """
     inst = lib.instrument_array_new(0)
     for x, y, z in inject.positions("AB"):
         lib.instrument_array_append(inst, lib.instrument_new(float(x), float(y), float(z), None))
@@ -65,6 +65,9 @@ TD = """
             lib.sh_series_free(s)
         return ok
 
+"""
+
+TD_GROWTH = """
     small, n = 2 * tr + 500, 2 * tr + 500
     assert call(small, "flat") and call(small, "random")
     failed = 0
@@ -93,5 +96,46 @@ TD = """
 def test_td_buffers_after_a_failed_growth(host_hip, network):
     """a growth that fails leaves no capacity behind for the buffer it
     freed: later calls that fit the old capacity allocate again"""
-    out = run(host_hip, "    network = %r\n" % network + TD)
+    out = run(host_hip, "    network = %r\n" % network + TD_PLAN + TD_GROWTH)
     assert int(out.split()[-1]) >= 4, out
+
+
+@pytest.mark.parametrize("network", [False, True])
+def test_td_without_pinned_memory(host_hip, network):
+    """without pinned memory the copies are made directly, and the calls
+    succeed, the first and those after it"""
+    run(host_hip, "    network = %r\n" % network + TD_PLAN + """
+    for on in (1, 0, 1):
+        H.host_hip_fail_pinned(on)
+        for n in (2 * tr + 3000 * (1 + on), 2 * tr + 400):
+            assert call(n, "flat") and call(n, "random"), (on, n, S.last_error())
+""")
+
+
+def test_device_alloc_after_a_failure(host_hip):
+    """an allocation that failed is reported once, by the call that asked"""
+    run(host_hip, """
+    H.host_hip_fail(1)
+    try:
+        S.DeviceBuffer(100)
+        raise SystemExit("no error")
+    except RuntimeError:
+        pass
+    x = np.zeros(100)
+    H.host_hip_fail(1)
+    f = None
+    try:
+        f = S.tseries_to_fseries(x)
+    except RuntimeError:
+        pass
+    a = S.DeviceBuffer.from_numpy(np.zeros(50, dtype=np.complex128))
+    h = S.Healpix(4, 4, S.FP64)
+    m = S.DeviceBuffer(h.npix * 8)
+    h.maps(a.ptr, 1, m.ptr)
+    H.host_hip_fail(1)
+    try:
+        S.DeviceBuffer(100)
+    except RuntimeError:
+        pass
+    h.maps(a.ptr, 1, m.ptr)
+""")
