@@ -712,9 +712,21 @@ static struct hm_geom hm_geom_of(const struct sphr_healpix *h, int n)
 	return g;
 }
 
+static void drop_mm(struct sphr_healpix *h)
+{
+	void *p[] = { h->P, h->W, h->off };
+	for(unsigned i = 0; i < sizeof(p) / sizeof(p[0]); i++)
+		if(p[i])
+			(void) hipFree(p[i]);
+	h->P = NULL;
+	h->W = NULL;
+	h->off = NULL;
+	h->rc = 0;
+}
+
 /* the tables of k_healpix_mm; left out, for the recurrences of
- * k_healpix_ring, where they would pass 512 MB or one ring's operand does
- * not fit in LDS */
+ * k_healpix_ring, where they would pass 512 MB, one ring's operand does not
+ * fit in LDS, or there is no memory for them */
 template <typename T>
 static int build_mm(struct sphr_healpix *h)
 {
@@ -752,9 +764,15 @@ static int build_mm(struct sphr_healpix *h)
 	h->rc = rc;
 	h->steps = (int) steps;
 	hipStream_t st = sphr_rt_stream();
-	int bad = sphr_rt_check(hipMalloc(&h->P, bP), "hipMalloc") || sphr_rt_check(hipMalloc(&h->W, bW), "hipMalloc")
-		  || sphr_rt_check(hipMalloc(&h->off, (L + 1 + 2 * (size_t) ns + 1) * sizeof(int)), "hipMalloc")
-		  || sphr_rt_check(hipMemcpy(h->off, off, (L + 1 + 2 * (size_t) ns + 1) * sizeof(int), hipMemcpyHostToDevice), "hipMemcpy");
+	int none = sphr_rt_check(hipMalloc(&h->P, bP), "hipMalloc") || sphr_rt_check(hipMalloc(&h->W, bW), "hipMalloc")
+		   || sphr_rt_check(hipMalloc(&h->off, (L + 1 + 2 * (size_t) ns + 1) * sizeof(int)), "hipMalloc");
+	if(none) {
+		/* the maps need no tables */
+		drop_mm(h);
+		free(off);
+		return 0;
+	}
+	const int bad = sphr_rt_check(hipMemcpy(h->off, off, (L + 1 + 2 * (size_t) ns + 1) * sizeof(int), hipMemcpyHostToDevice), "hipMemcpy");
 	free(off);
 	if(bad)
 		return -1;
@@ -818,10 +836,9 @@ extern "C" void sphr_healpix_free(struct sphr_healpix *h)
 {
 	if(!h)
 		return;
-	void *p[] = { h->d_cf, h->P, h->W, h->off };
-	for(unsigned i = 0; i < sizeof(p) / sizeof(p[0]); i++)
-		if(p[i])
-			hipFree(p[i]);
+	drop_mm(h);
+	if(h->d_cf)
+		hipFree(h->d_cf);
 	free(h);
 }
 

@@ -139,3 +139,33 @@ def test_device_alloc_after_a_failure(host_hip):
         pass
     h.maps(a.ptr, 1, m.ptr)
 """)
+
+
+def test_healpix_without_memory_for_tables(host_hip):
+    """the tables of the maps are optional: without memory for them the plan
+    runs the per-ring form; without memory for the coefficients there is no
+    plan; nothing is left allocated"""
+    run(host_hip, """
+    for prec in (S.FP64, S.MIXED):
+        start = H.host_hip_live()
+        n0 = H.host_hip_allocs()
+        h = S.Healpix(50, 32, prec)
+        n = H.host_hip_allocs() - n0
+        assert h.form(1000) == 1 and n == 4, n
+        del h
+        for k in range(1, n + 1):
+            H.host_hip_fail(k)
+            try:
+                h = S.Healpix(50, 32, prec)
+            except RuntimeError:
+                h = None
+            H.host_hip_fail(0)
+            assert (h is None) == (k == 1), k
+            if h:
+                assert h.form(1000) == 0
+                a, m = S.DeviceBuffer(51 ** 2 * 16), S.DeviceBuffer(h.npix * 8)
+                h.maps(a.ptr, 1, m.ptr)
+                a.free(), m.free()
+                del h
+            assert H.host_hip_live() == start, k
+    """)
