@@ -782,7 +782,8 @@ static int build_mm(struct sphr_healpix *h)
 	return sphr_rt_check(hipGetLastError(), "healpix tables") || sphr_rt_check(hipStreamSynchronize(st), "healpix tables") ? -1 : 0;
 }
 
-extern "C" struct sphr_healpix *sphr_healpix_new(unsigned l_max, int nside, int precision)
+/* with tables, or for few series without */
+static struct sphr_healpix *healpix_new(unsigned l_max, int nside, int precision, bool tables)
 {
 	if(sphr_gpu_ensure())
 		return NULL;
@@ -825,11 +826,16 @@ extern "C" struct sphr_healpix *sphr_healpix_new(unsigned l_max, int nside, int 
 	}
 	h->d_cm = h->d_cf + 2 * (size_t) nal;
 	free(hc);
-	if(precision == SPHR_MIXED ? build_mm<float>(h) : build_mm<double>(h)) {
+	if(tables && (precision == SPHR_MIXED ? build_mm<float>(h) : build_mm<double>(h))) {
 		sphr_healpix_free(h);
 		return NULL;
 	}
 	return h;
+}
+
+extern "C" struct sphr_healpix *sphr_healpix_new(unsigned l_max, int nside, int precision)
+{
+	return healpix_new(l_max, nside, precision, true);
 }
 
 extern "C" void sphr_healpix_free(struct sphr_healpix *h)
@@ -978,7 +984,7 @@ extern "C" int sh_series_write_healpix_map(const struct sh_series *series, const
 	for(int l = 0; l <= L; l++)
 		for(int m = series->polar ? 0 : -l; m <= (series->polar ? 0 : l); m++)
 			full[lm_offset(L, l, m)] = sh_series_get(series, l, m);
-	h = sphr_healpix_new(series->l_max, nside, SPHR_FP64);
+	h = healpix_new(series->l_max, nside, SPHR_FP64, false);
 	if(!h || sphr_rt_check(hipMalloc(&d_alm, ncoef * sizeof(*full)), "hipMalloc") || sphr_rt_check(hipMalloc(&d_map, npix * sizeof(double)), "hipMalloc")
 	   || sphr_memcpy_htod(d_alm, full, ncoef * sizeof(*full)) || sphr_healpix_maps(h, d_alm, 1, d_map, NULL)
 	   || sphr_memcpy_dtoh(hmap, d_map, npix * sizeof(double)))
