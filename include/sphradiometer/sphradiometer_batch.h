@@ -136,6 +136,9 @@ void sphr_loc_info(const struct sphr_loc *, int info[8]);
 struct sphr_healpix;
 int sphr_healpix_nside(unsigned l_max);
 struct sphr_healpix *sphr_healpix_new(unsigned l_max, int nside, int precision);
+/* the same without the tables that many series share: made faster, for a
+ * plan whose maps are few */
+struct sphr_healpix *sphr_healpix_new_few(unsigned l_max, int nside, int precision);
 void sphr_healpix_free(struct sphr_healpix *);
 long sphr_healpix_npix(const struct sphr_healpix *);
 int sphr_healpix_maps(const struct sphr_healpix *, const void *alm, int n, void *map, void *stream);

@@ -272,6 +272,7 @@ _PROTOS = {
     "sh_series_read_healpix_alm": (P(ShSeries), [ctypes.c_char_p]),
     "sphr_healpix_nside": (c_int, [c_uint]),
     "sphr_healpix_new": (c_void_p, [c_uint, c_int, c_int]),
+    "sphr_healpix_new_few": (c_void_p, [c_uint, c_int, c_int]),
     "sphr_healpix_free": (None, [c_void_p]),
     "sphr_healpix_npix": (ctypes.c_long, [c_void_p]),
     "sphr_healpix_maps": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p]),
@@ -718,13 +719,14 @@ class Localizer:
 class Healpix:
     """sphradiometer_batch.h sphr_healpix_*: RING-ordered HEALPix maps of
     many series on the GPU (Re f at the pixel centres), and the posterior
-    of the beta = +1 / -1 skies of localization events."""
+    of the beta = +1 / -1 skies of localization events.  few: no tables
+    (sphr_healpix_new_few), for a plan whose maps are few."""
 
-    def __init__(self, l_max, nside=None, precision=FP64):
+    def __init__(self, l_max, nside=None, precision=FP64, few=False):
         self.l_max = int(l_max)
         self.nside = int(nside) if nside is not None else lib().sphr_healpix_nside(self.l_max)
         self.precision = precision
-        self.h = lib().sphr_healpix_new(self.l_max, self.nside, precision)
+        self.h = (lib().sphr_healpix_new_few if few else lib().sphr_healpix_new)(self.l_max, self.nside, precision)
         if not self.h:
             raise RuntimeError("sphr_healpix_new failed: " + last_error())
         self.npix = lib().sphr_healpix_npix(self.h)

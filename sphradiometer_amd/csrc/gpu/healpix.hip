@@ -838,6 +838,11 @@ extern "C" struct sphr_healpix *sphr_healpix_new(unsigned l_max, int nside, int 
 	return healpix_new(l_max, nside, precision, true);
 }
 
+extern "C" struct sphr_healpix *sphr_healpix_new_few(unsigned l_max, int nside, int precision)
+{
+	return healpix_new(l_max, nside, precision, false);
+}
+
 extern "C" void sphr_healpix_free(struct sphr_healpix *h)
 {
 	if(!h)

@@ -113,7 +113,7 @@ def healpy_alm_to_map(alms, l_max, m_max):
     the map computed on the GPU in float64."""
     _check_mmax(l_max, m_max)
     nside = nside_for_map(l_max)
-    hp = Healpix(l_max, nside, FP64)
+    hp = Healpix(l_max, nside, FP64, few=True)
     full = _full_coefficients(alms, l_max, m_max)
     d_alm = DeviceBuffer.from_numpy(full)
     d_map = DeviceBuffer(hp.npix * 8)

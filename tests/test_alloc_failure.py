@@ -171,11 +171,15 @@ def test_healpix_without_memory_for_tables(host_hip):
     """)
 
 
-def test_one_map_to_a_file_makes_no_tables(host_hip, tmp_path):
-    """a plan used for one series holds the coefficients alone"""
+def test_one_map_makes_no_tables(host_hip, tmp_path):
+    """to a file and from healpy coefficients: a plan used for one series holds the coefficients alone"""
     run(host_hip, """
     s = S.series_from_numpy(np.ones(33 ** 2), 32, 0)
     start, n0 = H.host_hip_live(), H.host_hip_allocs()
     assert lib.sh_series_write_healpix_map(s, %r) == 0, S.last_error()
     assert H.host_hip_allocs() - n0 == 3 and H.host_hip_live() == start
+    from sphradiometer_amd import healpix
+    n0 = H.host_hip_allocs()
+    healpix.healpy_alm_to_map(np.ones(healpix.healpy_alm_length(32, 32)), 32, 32)
+    assert H.host_hip_allocs() - n0 == 3
     """ % os.path.join(str(tmp_path), "map.fits").encode())
