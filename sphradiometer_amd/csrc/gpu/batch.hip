@@ -50,7 +50,7 @@ struct sphr_batch {
 	struct xproj_geom g;
 	struct xcorr_geom xg;
 	struct synth_dev syn;
-	void *W, *R, *tw, *spec, *partial, *F, *M, *twW, *Wany;
+	void *W, *R, *Rs, *tw, *spec, *partial, *F, *M, *twW, *Wany;
 	int *col_bl;
 	int2 *lm;
 	int profile;
@@ -84,15 +84,20 @@ static int build_tables(struct sphr_batch *bt, const struct sphr_net_desc *d)
 	const int N = bt->N, Nh = bt->Nh, CT = bt->g.CT, K2 = bt->g.K2, L = bt->L, nb = bt->nb;
 	const size_t ncoef = (size_t) (L + 1) * (L + 1);
 	T *W = (T *) calloc((size_t) K2 * CT, sizeof(T));
-	T *R = (T *) calloc(2 * ncoef * nb, sizeof(T));
+	const size_t nal = (size_t) (L + 1) * (L + 2) / 2;
+	T *R = (T *) calloc(2 * ncoef * nb, sizeof(T)), *Rs = (T *) calloc(2 * nal * nb, sizeof(T));
 	T *tw = (T *) malloc(2 * (size_t) N * sizeof(T));
 	double *twd = (double *) malloc(2 * (size_t) N * sizeof(double));
 	int rc = -1;
 	/* real skies: every projected column real (no imaginary column of W)
-	 * and rotation rows with R_l,-m = (-1)^m conj R_lm */
+	 * and rotation rows with R_l,-m = (-1)^m conj R_lm.  The real part of a
+	 * mesh comes from the rows' symmetric part, (R_lm + (-1)^m conj
+	 * R_l,-m) / 2; past the rounding of T in the rest of the stage it has a
+	 * table of its own. */
 	bt->real = 1;
 	const double rtol = sizeof(T) == 4 ? 1e-9 : 1e-12;	/* the rotation rows' recursion loses digits with l */
-	if(!W || !R || !tw || !twd)
+	double asym = 0.0;
+	if(!W || !R || !Rs || !tw || !twd)
 		goto done;
 	for(int b = 0; b < nb; b++) {
 		double big = 0.0, imag = 0.0;
@@ -123,16 +128,24 @@ static int build_tables(struct sphr_batch *bt, const struct sphr_net_desc *d)
 		Rb[0] = (T) (1.0 / nb);
 		if(!(imag <= 1e-12 * big))
 			bt->real = 0;
+		Rs[2 * nal * b] = Rb[0];
 		for(int l = 1; l <= Lb; l++)
 			for(int mp = -l; mp <= l; mp++) {
 				const size_t src = block_offset_h(l) + (size_t) (2 * l + 1) * (mp + l) + l;
 				const int dst = lm_offset(L, l, mp);
 				const size_t mir = block_offset_h(l) + (size_t) (2 * l + 1) * (l - mp) + l;
 				const double sg = (mp & 1) ? -1.0 : 1.0;
-				if(!(fabs(d->blocks[b][2 * src] - sg * d->blocks[b][2 * mir]) <= rtol) || !(fabs(d->blocks[b][2 * src + 1] + sg * d->blocks[b][2 * mir + 1]) <= rtol))
+				const double *D = d->blocks[b];
+				const double e = fabs(D[2 * src] - sg * D[2 * mir]) + fabs(D[2 * src + 1] + sg * D[2 * mir + 1]);
+				if(!(e <= rtol))
 					bt->real = 0;
-				Rb[2 * dst] = (T) (d->blocks[b][2 * src] / nb);
-				Rb[2 * dst + 1] = (T) (d->blocks[b][2 * src + 1] / nb);
+				asym = fmax(asym, e);
+				Rb[2 * dst] = (T) (D[2 * src] / nb);
+				Rb[2 * dst + 1] = (T) (D[2 * src + 1] / nb);
+				if(mp >= 0) {
+					Rs[2 * (nal * b + dst)] = (T) (0.5 * (D[2 * src] + sg * D[2 * mir]) / nb);
+					Rs[2 * (nal * b + dst) + 1] = (T) (0.5 * (D[2 * src + 1] - sg * D[2 * mir + 1]) / nb);
+				}
 			}
 	}
 	sphr_twiddles(N, -1, twd);
@@ -140,10 +153,13 @@ static int build_tables(struct sphr_batch *bt, const struct sphr_net_desc *d)
 		tw[k] = (T) twd[k];
 	if(upload(&bt->W, W, (size_t) K2 * CT) || upload(&bt->R, R, 2 * ncoef * nb) || upload(&bt->tw, tw, 2 * (size_t) N))
 		goto done;
+	if(bt->real && asym > (sizeof(T) == 4 ? 1e-9 : 1e-14) && upload(&bt->Rs, Rs, 2 * nal * nb))
+		goto done;
 	rc = 0;
 done:
 	free(W);
 	free(R);
+	free(Rs);
 	free(tw);
 	free(twd);
 	return rc;
@@ -286,7 +302,7 @@ extern "C" void sphr_batch_free(struct sphr_batch *bt)
 {
 	if(!bt)
 		return;
-	void *ptrs[] = { bt->W, bt->R, bt->tw, bt->spec, bt->partial, bt->col_bl, bt->lm, bt->F, bt->M, bt->twW, bt->Wany };
+	void *ptrs[] = { bt->W, bt->R, bt->tw, bt->spec, bt->partial, bt->col_bl, bt->lm, bt->F, bt->M, bt->twW, bt->Wany, bt->Rs };
 	for(unsigned i = 0; i < sizeof(ptrs) / sizeof(ptrs[0]); i++)
 		if(ptrs[i])
 			hipFree(ptrs[i]);
@@ -453,7 +469,7 @@ static int run_t(struct sphr_batch *bt, void *spec, void *partial, void *F, cons
 	 * 24.9 against 28.1 us at two sites and 16 segments, but its forms
 	 * give the same bits and this kernel's sums run in another order) */
 	const bool any = bt->fused && bt->real && !sky_fused_order(bt->L);
-	if(any && launch_sky_any<T>((const T *) partial, nsplit, S, &bt->g, (const cplx<T> *) bt->R, bt->lm, gmst, bt->L, &bt->syn.tb, (const T *) bt->Wany, (cplx<T> *) alm, (cplx<T> *) map, st) == 0) {
+	if(any && launch_sky_any<T>((const T *) partial, nsplit, S, &bt->g, (const cplx<T> *) bt->R, (const cplx<T> *) bt->Rs, bt->lm, gmst, bt->L, &bt->syn.tb, (const T *) bt->Wany, (cplx<T> *) alm, (cplx<T> *) map, st) == 0) {
 		if(ev)
 			hipEventRecord(ev[3], st);
 	} else if(bt->fused && launch_sky_fused<T>((const T *) partial, nsplit, S, &bt->g, (const cplx<T> *) bt->R, bt->lm, gmst, &bt->syn.g, &bt->syn.tb, (cplx<T> *) alm, (cplx<T> *) map, st, bt->sky_occ, bt->sky_nsub) == 0) {

@@ -154,13 +154,14 @@ int sky_fused_tables(int L, const struct synth_tables *tb, struct sky_fused_dev 
 template <typename T>
 int launch_sky_fused(const T *partial, int nsplit, int S, const struct xproj_geom *xg, const cplx<T> *R, const int2 *lm, const double *gmst, const struct synth_geom *g, const struct synth_tables *tb, cplx<T> *alm, cplx<T> *map, hipStream_t st, int occ = 1, int nsub = 0);
 /* the same stage for real skies of any order (sky_any.hip), W its phi DFT
- * table; map NULL: a_lm only; -1 when a ring group does not fit in LDS */
+ * table, Rs the m >= 0 rotation rows that the meshes come from (NULL: those
+ * of R); map NULL: a_lm only; -1 when a ring group does not fit in LDS */
 template <typename T>
 size_t sky_any_table_bytes(int L);
 template <typename T>
 int sky_any_table(int L, const double *twp, T *W, hipStream_t st);
 template <typename T>
-int launch_sky_any(const T *partial, int nsplit, int S, const struct xproj_geom *xg, const cplx<T> *R, const int2 *lm, const double *gmst, int L, const struct synth_tables *tb, const T *W, cplx<T> *alm, cplx<T> *map, hipStream_t st);
+int launch_sky_any(const T *partial, int nsplit, int S, const struct xproj_geom *xg, const cplx<T> *R, const cplx<T> *Rs, const int2 *lm, const double *gmst, int L, const struct synth_tables *tb, const T *W, cplx<T> *alm, cplx<T> *map, hipStream_t st);
 template <typename T>
 int launch_phi(const cplx<T> *F, int S, const struct synth_geom *g, const struct synth_tables *tb, cplx<T> *map, hipStream_t st);
 /* the a_lm of the localization skies formed where they are read: series

@@ -24,7 +24,10 @@
  * (one lane per ring and order, then a GEMM over 2 (2 L + 1) columns):
  * 333 segments of order 41 in float32 34 + 40 -> 29 us.  512 threads and
  * two workgroups per CU's worth of parts: 256 threads or twice the parts
- * measured 2 % faster to 50 % slower.
+ * measured 2 % faster to 50 % slower.  The second set of coefficients that
+ * SYM forms costs 0-5 % (float64, order 54: 64 segments 36.8 -> 38.6 us, 1000
+ * 180.6 -> 179.0) and keeps the meshes at the two kernels' distance from
+ * 64-bit sums with exact rows (order 54 2.9e-13; m >= 0 rows alone 3.5e-13).
  */
 #include <hip/hip_runtime.h>
 #include <string.h>
@@ -79,8 +82,8 @@ __global__ void k_sky_any_table(struct sa_geom g, const double *__restrict__ twp
 	W[i] = (T) w;
 }
 
-template <typename T>
-__global__ void __launch_bounds__(SA_NT) k_sky_any(const T *__restrict__ partial, int nsplit, int S, struct xproj_geom xg, const cplx<T> *__restrict__ R, const int2 *__restrict__ lm, const double *__restrict__ gmst, struct synth_tables tb, const T *__restrict__ W, struct sa_geom g, cplx<T> *__restrict__ alm, cplx<T> *__restrict__ map)
+template <typename T, bool SYM>
+__global__ void __launch_bounds__(SA_NT) k_sky_any(const T *__restrict__ partial, int nsplit, int S, struct xproj_geom xg, const cplx<T> *__restrict__ R, const cplx<T> *__restrict__ Rs, const int2 *__restrict__ lm, const double *__restrict__ gmst, struct synth_tables tb, const T *__restrict__ W, struct sa_geom g, cplx<T> *__restrict__ alm, cplx<T> *__restrict__ map)
 {
 	typedef sa_ops<T> ops;
 	typedef typename ops::v4 v4;
@@ -130,32 +133,47 @@ __global__ void __launch_bounds__(SA_NT) k_sky_any(const T *__restrict__ partial
 
 	/* a_lm: rotation row x the baseline's projected column, summed over the
 	 * baselines in float64 whatever T, then rotate_z; the m >= 0 block
-	 * comes first in the coefficient order */
+	 * comes first in the coefficient order.  With SYM the mesh's
+	 * coefficients are those of the rows Rs (the real part of a mesh is the
+	 * sum over the rows' symmetric part): the first part, which writes the
+	 * a_lm, forms both */
 	{
-		const int nc = part ? g.nal : g.ncoef;
+		const int nc = part ? g.nal : g.ncoef, ld = SYM && part ? g.nal : g.ncoef;
+		const cplx<T> *rows = SYM && part ? Rs : R;
 		cplx<T> *out = alm + (size_t) s * g.ncoef;
 #pragma unroll 2
 		for(int idx = tid; idx < nc; idx += SA_NT) {
 			const int2 q = lm[idx];
-			cplx<double> acc = mk(0.0, 0.0);
+			const bool two = SYM && !part && idx < g.nal;
+			cplx<double> acc = mk(0.0, 0.0), accs = mk(0.0, 0.0);
 			for(int b0 = 0; b0 < xg.nb; b0 += 4) {
-				cplx<T> r[4];
+				cplx<T> r[4], rs[4];
 #pragma unroll
 				for(int u = 0; u < 4; u++)
-					if(b0 + u < xg.nb)
-						r[u] = R[(size_t) (b0 + u) * g.ncoef + idx];
+					if(b0 + u < xg.nb) {
+						r[u] = rows[(size_t) (b0 + u) * ld + idx];
+						if(two)
+							rs[u] = Rs[(size_t) (b0 + u) * g.nal + idx];
+					}
 #pragma unroll
 				for(int u = 0; u < 4; u++)
 					if(b0 + u < xg.nb && q.x <= xg.Lb[b0 + u]) {
 						const T *p = pw + xg.col_start[b0 + u] + 2 * q.x;
-						cfma(acc, mk((double) r[u].re, (double) r[u].im), mk((double) p[0], (double) p[1]));
+						const cplx<double> v = mk((double) p[0], (double) p[1]);
+						cfma(acc, mk((double) r[u].re, (double) r[u].im), v);
+						if(two)
+							cfma(accs, mk((double) rs[u].re, (double) rs[u].im), v);
 					}
 			}
-			cplx<T> a = mk((T) acc.re, (T) acc.im);
-			if(gmst && q.y)
-				a = a * (q.y > 0 ? rot[q.y] : conjg(rot[-q.y]));
+			cplx<T> a = mk((T) acc.re, (T) acc.im), as = two ? mk((T) accs.re, (T) accs.im) : a;
+			if(gmst && q.y) {
+				const cplx<T> z = q.y > 0 ? rot[q.y] : conjg(rot[-q.y]);
+				a = a * z;
+				if(SYM)
+					as = as * z;
+			}
 			if(idx < g.nal)
-				sa[idx] = a;
+				sa[idx] = SYM ? as : a;
 			if(!part)
 				out[idx] = a;
 		}
@@ -313,7 +331,7 @@ int sky_any_table(int L, const double *twp, T *W, hipStream_t st)
 /* parts per segment: enough workgroups for two per CU, more where the ring
  * sums of a part would not fit in LDS; -1 where one ring group does not */
 template <typename T>
-int launch_sky_any(const T *partial, int nsplit, int S, const struct xproj_geom *xg, const cplx<T> *R, const int2 *lm, const double *gmst, int L, const struct synth_tables *tb, const T *W, cplx<T> *alm, cplx<T> *map, hipStream_t st)
+int launch_sky_any(const T *partial, int nsplit, int S, const struct xproj_geom *xg, const cplx<T> *R, const cplx<T> *Rs, const int2 *lm, const double *gmst, int L, const struct synth_tables *tb, const T *W, cplx<T> *alm, cplx<T> *map, hipStream_t st)
 {
 	struct sa_geom g = sa_geom_of(L, sizeof(T) == 4);
 	const size_t fixed = ((size_t) 2 * g.nal + 2 + L + 1) * sizeof(cplx<T>) + (size_t) xg->CT * sizeof(T), tile = (size_t) 16 * g.ld * sizeof(T);
@@ -332,7 +350,10 @@ int launch_sky_any(const T *partial, int nsplit, int S, const struct xproj_geom 
 		return -1;
 	g.tpp = (g.tiles + parts - 1) / parts;
 	g.parts = (g.tiles + g.tpp - 1) / g.tpp;
-	hipLaunchKernelGGL((k_sky_any<T>), dim3(S * g.parts), dim3(SA_NT), fixed + (map ? g.tpp * tile : 0), st, partial, nsplit, S, *xg, R, lm, gmst, *tb, W, g, alm, map);
+	if(Rs)
+		hipLaunchKernelGGL((k_sky_any<T, true>), dim3(S * g.parts), dim3(SA_NT), fixed + (map ? g.tpp * tile : 0), st, partial, nsplit, S, *xg, R, Rs, lm, gmst, *tb, W, g, alm, map);
+	else
+		hipLaunchKernelGGL((k_sky_any<T, false>), dim3(S * g.parts), dim3(SA_NT), fixed + (map ? g.tpp * tile : 0), st, partial, nsplit, S, *xg, R, Rs, lm, gmst, *tb, W, g, alm, map);
 	return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -340,5 +361,5 @@ template size_t sky_any_table_bytes<float>(int);
 template size_t sky_any_table_bytes<double>(int);
 template int sky_any_table<float>(int, const double *, float *, hipStream_t);
 template int sky_any_table<double>(int, const double *, double *, hipStream_t);
-template int launch_sky_any<float>(const float *, int, int, const struct xproj_geom *, const cplx<float> *, const int2 *, const double *, int, const struct synth_tables *, const float *, cplx<float> *, cplx<float> *, hipStream_t);
-template int launch_sky_any<double>(const double *, int, int, const struct xproj_geom *, const cplx<double> *, const int2 *, const double *, int, const struct synth_tables *, const double *, cplx<double> *, cplx<double> *, hipStream_t);
+template int launch_sky_any<float>(const float *, int, int, const struct xproj_geom *, const cplx<float> *, const cplx<float> *, const int2 *, const double *, int, const struct synth_tables *, const float *, cplx<float> *, cplx<float> *, hipStream_t);
+template int launch_sky_any<double>(const double *, int, int, const struct xproj_geom *, const cplx<double> *, const cplx<double> *, const int2 *, const double *, int, const struct synth_tables *, const double *, cplx<double> *, cplx<double> *, hipStream_t);

@@ -525,6 +525,29 @@ def test_gpu_sky_any_order_matches_two_kernel_form(L, nseg):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("L,nseg", [(36, 600), (48, 9), (54, 70)])
+def test_gpu_sky_any_order_meshes_from_symmetric_rows(L, nseg):
+    """float64 meshes of the one-kernel stage hold the real part of the
+    two-kernel form's whatever the rounding of the rotation rows at m and -m
+    (9e-13 at order 54): both sum the rows' symmetric part, so they differ by
+    the roundings of their sums, a few times 1e-16 times the root of the
+    coefficients' number; one part per segment and several"""
+    net = S.Network(inject.positions("ABC"), 512, 1.0 / 4096, L)
+    rng = np.random.default_rng(L)
+    d_ts = S.DeviceBuffer.from_numpy(rng.standard_normal((3, nseg, 512)))
+    d_g = S.DeviceBuffer.from_numpy(rng.uniform(0, 6, nseg))
+    b = S.Batch(net, L, S.FP64, max_segments=nseg)
+    n, maps = 2 * L + 2, []
+    for fused in (True, False):
+        b.set_fused(fused)
+        d_a, d_m = S.DeviceBuffer(nseg * (L + 1) ** 2 * 16), S.DeviceBuffer(nseg * n * n * 16)
+        b.run(d_ts.ptr, nseg, d_a.ptr, d_m.ptr, d_gmst=d_g.ptr)
+        S.synchronize()
+        maps.append(d_m.to_numpy(np.complex128, (nseg, n, n)).real)
+    assert rel(maps[0], maps[1]) < 5e-16 * (L + 1), rel(maps[0], maps[1])
+
+
+@pytest.mark.gpu
 def test_gpu_sky_of_a_plan_that_is_not_real():
     """a delay product scaled by a complex number gives complex skies: the
     stages for real skies are not taken, the imaginary parts stay"""
