@@ -251,18 +251,23 @@ int sphr_batch_set_shape(struct sphr_batch *, int index);
 /* Shape information: [0] detectors, [1] baselines, [2] N, [3] sky l_max,
  * [4] projection columns, [5] K splits, [6] precision, [7] K per split,
  * [8] 1 when the sky stage runs as the fused kernel compiled for the
- * order, 0 otherwise (the one-kernel form for any order where the plan
- * gives real skies, else the two-kernel form), [9] projection tiles per wave,
+ * order, 0 otherwise (sphr_batch_sky_form tells the other forms), [9] projection tiles per wave,
  * [10] projection segments per workgroup, [11] fused sky workgroups per
  * CU requested (1-3, picked by the autotuner), [12] fused sky segments per
  * workgroup requested (0 for the precision's default, 1, 2 or 4) */
 void sphr_batch_info(const struct sphr_batch *, int info[13]);
+/* The sky stage's form as now set: 1 the fused kernel compiled for the
+ * order, 2 the one-kernel form for any order (real skies whose coefficients
+ * fit in LDS: to order 88 in FP64 and 130 in mixed precision at three
+ * sites), 0 the two-kernel form; -1 for no batch */
+int sphr_batch_sky_form(const struct sphr_batch *);
 
 /* Select the sky stage's form: 1 (default) one kernel (the fused one where
  * it is compiled for the batch's order, else its form for any order where
- * the plan gives real skies), 0 the two-kernel
- * form (a_lm and ring sums, then the phi DFT as a GEMM).  Both give the same results to
- * rounding. */
+ * the plan gives real skies and the order fits in LDS), 0 the two-kernel
+ * form (a_lm and ring sums, then the phi DFT as a GEMM).  Both give the
+ * same results to rounding; the one-kernel forms write zero imaginary
+ * parts, the two kernels the rounding there. */
 void sphr_batch_set_fused(struct sphr_batch *, int on);
 /* Fused sky kernel's persistent workgroups per CU: 1 (default), 2 (the
  * rotation rows then stay in global memory when both would not fit the

@@ -227,6 +227,7 @@ _PROTOS = {
     "sphr_batch_profile": (c_int, [c_void_p, c_int]),
     "sphr_batch_profile_read": (c_int, [c_void_p, P(c_double), P(c_int)]),
     "sphr_batch_info": (None, [c_void_p, P(c_int)]),
+    "sphr_batch_sky_form": (c_int, [c_void_p]),
     "sphr_batch_set_fused": (None, [c_void_p, c_int]),
     "sphr_batch_set_sky_occupancy": (c_int, [c_void_p, c_int]),
     "sphr_batch_set_sky_segments": (c_int, [c_void_p, c_int]),
@@ -581,6 +582,12 @@ class Batch:
         """Sky stage as the one fused kernel (default, where compiled for
         the order) or as the two-kernel form."""
         lib().sphr_batch_set_fused(self.h, int(bool(on)))
+
+    @property
+    def sky_form(self):
+        """The sky stage's form as now set (sphr_batch_sky_form): 1 the fused
+        kernel, 2 the one-kernel form for any order, 0 two kernels."""
+        return lib().sphr_batch_sky_form(self.h)
 
     def set_sky_occupancy(self, workgroups_per_cu):
         if lib().sphr_batch_set_sky_occupancy(self.h, int(workgroups_per_cu)):

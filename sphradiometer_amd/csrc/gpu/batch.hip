@@ -44,6 +44,7 @@ struct sphr_batch {
 	int ksplit_opt[4], nsplit_opt[4];	/* K-split candidates: 1, 2, 4 x CUs workgroups, 64 per split */
 	int shape;			/* the projection shape index in use (sphr_batch_set_shape) */
 	int real;			/* the plan gives real skies (checked) */
+	int any;			/* the one-kernel sky stage for any order serves the batch */
 	int lag_ok, lag;		/* lag-domain route built / in use */
 	size_t m_bytes;			/* its table's bytes */
 	int xc_forms, xc_form;		/* its kernel forms (bit f - 1 for form f), the one in use (autotuned) */
@@ -90,12 +91,15 @@ static int build_tables(struct sphr_batch *bt, const struct sphr_net_desc *d)
 	double *twd = (double *) malloc(2 * (size_t) N * sizeof(double));
 	int rc = -1;
 	/* real skies: every projected column real (no imaginary column of W)
-	 * and rotation rows with R_l,-m = (-1)^m conj R_lm.  The real part of a
-	 * mesh comes from the rows' symmetric part, (R_lm + (-1)^m conj
-	 * R_l,-m) / 2; past the rounding of T in the rest of the stage it has a
-	 * table of its own. */
+	 * and rotation rows with R_l,-m = (-1)^m conj R_lm, to the rounding of
+	 * their recursion, which grows by 1.25 per order (largest differences
+	 * over 40 directions: 1.7e-16 at l = 5, 4e-15 at 25, 6.5e-13 at 50,
+	 * 1.2e-11 at 64, 2.7e-9 at 90, 2.9e-8 at 100; the bound lies six times
+	 * or more above them, rows that are not those of a rotation differ by
+	 * their size).  The real part of a mesh comes from the rows' symmetric
+	 * part, (R_lm + (-1)^m conj R_l,-m) / 2; past the rounding of T in the
+	 * rest of the stage it has a table of its own. */
 	bt->real = 1;
-	const double rtol = sizeof(T) == 4 ? 1e-9 : 1e-12;	/* the rotation rows' recursion loses digits with l */
 	double asym = 0.0;
 	if(!W || !R || !Rs || !tw || !twd)
 		goto done;
@@ -129,7 +133,9 @@ static int build_tables(struct sphr_batch *bt, const struct sphr_net_desc *d)
 		if(!(imag <= 1e-12 * big))
 			bt->real = 0;
 		Rs[2 * nal * b] = Rb[0];
-		for(int l = 1; l <= Lb; l++)
+		double bound = 1e-16;
+		for(int l = 1; l <= Lb; l++) {
+			bound *= 1.25;
 			for(int mp = -l; mp <= l; mp++) {
 				const size_t src = block_offset_h(l) + (size_t) (2 * l + 1) * (mp + l) + l;
 				const int dst = lm_offset(L, l, mp);
@@ -137,7 +143,7 @@ static int build_tables(struct sphr_batch *bt, const struct sphr_net_desc *d)
 				const double sg = (mp & 1) ? -1.0 : 1.0;
 				const double *D = d->blocks[b];
 				const double e = fabs(D[2 * src] - sg * D[2 * mir]) + fabs(D[2 * src + 1] + sg * D[2 * mir + 1]);
-				if(!(e <= rtol))
+				if(!(e <= 1e-15 + bound && e <= 1e-4))
 					bt->real = 0;
 				asym = fmax(asym, e);
 				Rb[2 * dst] = (T) (D[2 * src] / nb);
@@ -147,13 +153,15 @@ static int build_tables(struct sphr_batch *bt, const struct sphr_net_desc *d)
 					Rs[2 * (nal * b + dst) + 1] = (T) (0.5 * (D[2 * src + 1] - sg * D[2 * mir + 1]) / nb);
 				}
 			}
+		}
 	}
 	sphr_twiddles(N, -1, twd);
 	for(int k = 0; k < 2 * N; k++)
 		tw[k] = (T) twd[k];
 	if(upload(&bt->W, W, (size_t) K2 * CT) || upload(&bt->R, R, 2 * ncoef * nb) || upload(&bt->tw, tw, 2 * (size_t) N))
 		goto done;
-	if(bt->real && asym > (sizeof(T) == 4 ? 1e-9 : 1e-14) && upload(&bt->Rs, Rs, 2 * nal * nb))
+	bt->any = bt->real && !sky_fused_order(L) && sky_any_fits<T>(L, CT);
+	if(bt->any && asym > (sizeof(T) == 4 ? 1e-9 : 1e-14) && upload(&bt->Rs, Rs, 2 * nal * nb))
 		goto done;
 	rc = 0;
 done:
@@ -414,7 +422,7 @@ extern "C" struct sphr_batch *sphr_batch_create(const struct sphr_net_desc *d, u
 		goto fail;
 	if(synth_tables_build(bt->L, &bt->syn))
 		goto fail;
-	if(bt->real) {
+	if(bt->any) {
 		hipStream_t st = sphr_rt_stream();
 		const size_t bytes = precision == SPHR_MIXED ? sky_any_table_bytes<float>(bt->L) : sky_any_table_bytes<double>(bt->L);
 		if(sphr_rt_check(hipMalloc(&bt->Wany, bytes), "hipMalloc")
@@ -468,8 +476,7 @@ static int run_t(struct sphr_batch *bt, void *spec, void *partial, void *F, cons
 	/* (at the fused kernel's orders few segments would run faster here,
 	 * 24.9 against 28.1 us at two sites and 16 segments, but its forms
 	 * give the same bits and this kernel's sums run in another order) */
-	const bool any = bt->fused && bt->real && !sky_fused_order(bt->L);
-	if(any && launch_sky_any<T>((const T *) partial, nsplit, S, &bt->g, (const cplx<T> *) bt->R, (const cplx<T> *) bt->Rs, bt->lm, gmst, bt->L, &bt->syn.tb, (const T *) bt->Wany, (cplx<T> *) alm, (cplx<T> *) map, st) == 0) {
+	if(bt->fused && bt->any && launch_sky_any<T>((const T *) partial, nsplit, S, &bt->g, (const cplx<T> *) bt->R, (const cplx<T> *) bt->Rs, bt->lm, gmst, bt->L, &bt->syn.tb, (const T *) bt->Wany, (cplx<T> *) alm, (cplx<T> *) map, st) == 0) {
 		if(ev)
 			hipEventRecord(ev[3], st);
 	} else if(bt->fused && launch_sky_fused<T>((const T *) partial, nsplit, S, &bt->g, (const cplx<T> *) bt->R, bt->lm, gmst, &bt->syn.g, &bt->syn.tb, (cplx<T> *) alm, (cplx<T> *) map, st, bt->sky_occ, bt->sky_nsub) == 0) {
@@ -642,6 +649,11 @@ extern "C" int sphr_batch_set_sky_segments(struct sphr_batch *bt, int segments_p
 	}
 	bt->sky_nsub = n;
 	return 0;
+}
+
+extern "C" int sphr_batch_sky_form(const struct sphr_batch *bt)
+{
+	return !bt ? -1 : !bt->fused ? 0 : bt->any ? 2 : sky_fused_order(bt->L) ? 1 : 0;
 }
 
 extern "C" void sphr_batch_info(const struct sphr_batch *bt, int info[13])

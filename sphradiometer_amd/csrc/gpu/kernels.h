@@ -157,6 +157,8 @@ int launch_sky_fused(const T *partial, int nsplit, int S, const struct xproj_geo
  * table, Rs the m >= 0 rotation rows that the meshes come from (NULL: those
  * of R); map NULL: a_lm only; -1 when a ring group does not fit in LDS */
 template <typename T>
+int sky_any_fits(int L, int CT);
+template <typename T>
 size_t sky_any_table_bytes(int L);
 template <typename T>
 int sky_any_table(int L, const double *twp, T *W, hipStream_t st);

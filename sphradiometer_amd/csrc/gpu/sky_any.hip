@@ -328,25 +328,43 @@ int sky_any_table(int L, const double *twp, T *W, hipStream_t st)
 	return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+/* LDS of a workgroup besides the ring sums, and of one group's ring sums */
+static size_t sky_any_lds(const struct sa_geom *g, int CT, size_t esz, size_t *tile)
+{
+	*tile = (size_t) 16 * g->ld * esz;
+	return ((size_t) 2 * g->nal + 2 + g->L + 1) * 2 * esz + (size_t) CT * esz;
+}
+
+#define SA_LDS ((size_t) 158 * 1024)
+
+template <typename T>
+int sky_any_fits(int L, int CT)
+{
+	const struct sa_geom g = sa_geom_of(L, sizeof(T) == 4);
+	size_t tile;
+	const size_t fixed = sky_any_lds(&g, CT, sizeof(T), &tile);
+	return fixed + tile <= SA_LDS;
+}
+
 /* parts per segment: enough workgroups for two per CU, more where the ring
  * sums of a part would not fit in LDS; -1 where one ring group does not */
 template <typename T>
 int launch_sky_any(const T *partial, int nsplit, int S, const struct xproj_geom *xg, const cplx<T> *R, const cplx<T> *Rs, const int2 *lm, const double *gmst, int L, const struct synth_tables *tb, const T *W, cplx<T> *alm, cplx<T> *map, hipStream_t st)
 {
 	struct sa_geom g = sa_geom_of(L, sizeof(T) == 4);
-	const size_t fixed = ((size_t) 2 * g.nal + 2 + L + 1) * sizeof(cplx<T>) + (size_t) xg->CT * sizeof(T), tile = (size_t) 16 * g.ld * sizeof(T);
+	size_t tile;
+	const size_t fixed = sky_any_lds(&g, xg->CT, sizeof(T), &tile);
 	if(S <= 0)
 		return 0;
 	int parts = 1;
 	if(map) {
-		const size_t most = 158 * 1024;
-		if(fixed + tile > most)
+		if(fixed + tile > SA_LDS)
 			return -1;
 		parts = 2 * sphr_rt_cus() / S;
 		parts = parts < 1 ? 1 : parts > g.tiles ? g.tiles : parts;
-		while(parts < g.tiles && fixed + (g.tiles + parts - 1) / parts * tile > most)
+		while(parts < g.tiles && fixed + (g.tiles + parts - 1) / parts * tile > SA_LDS)
 			parts++;
-	} else if(fixed > 158 * 1024)
+	} else if(fixed > SA_LDS)
 		return -1;
 	g.tpp = (g.tiles + parts - 1) / parts;
 	g.parts = (g.tiles + g.tpp - 1) / g.tpp;
@@ -357,6 +375,8 @@ int launch_sky_any(const T *partial, int nsplit, int S, const struct xproj_geom 
 	return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+template int sky_any_fits<float>(int, int);
+template int sky_any_fits<double>(int, int);
 template size_t sky_any_table_bytes<float>(int);
 template size_t sky_any_table_bytes<double>(int);
 template int sky_any_table<float>(int, const double *, float *, hipStream_t);

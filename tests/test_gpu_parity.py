@@ -497,27 +497,41 @@ def test_batch_full_size_three_site_properties(three_site):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("L,nseg", [(1, 1), (2, 3), (7, 2), (8, 130), (15, 3), (16, 5), (24, 7), (31, 2), (31, 128), (33, 600), (47, 3), (48, 2), (64, 2), (90, 2)])
+@pytest.mark.parametrize("L,nseg", [(1, 1), (2, 3), (7, 2), (8, 130), (15, 3), (16, 5), (24, 7), (31, 2), (31, 128), (33, 600), (47, 3), (48, 2), (60, 40), (64, 2), (88, 3), (90, 2)])
 def test_gpu_sky_any_order_matches_two_kernel_form(L, nseg):
     """the one-kernel sky stage for any order against the two-kernel form:
     edges of its ring groups (8), point tiles (16) and column groups, every
-    split of a segment over workgroups, a GMST per segment, a_lm alone"""
+    split of a segment over workgroups, a GMST per segment, a_lm alone; the
+    order whose ring sums do not fit in LDS (90 in float64) runs the two
+    kernels.
+
+    The meshes are compared by their real parts.  The one kernel's have no
+    imaginary part; the two kernels' is the rounding of the rotation rows,
+    R_lm - (-1)^m conj R_l,-m, below 1e-16 1.25^l and 1e-15, times at most
+    the root of the coefficients' number.  float32: each form's recurrences
+    are 2.4e-6 from float64 at order 50, 4.7e-6 at 72 and 7.9e-6 at 90."""
     net = S.Network(inject.positions("ABC"), 512, 1.0 / 4096, L)
     rng = np.random.default_rng(L + nseg)
     ts, gm = rng.standard_normal((3, nseg, 512)), rng.uniform(0, 6, nseg)
     d_ts, d_g = S.DeviceBuffer.from_numpy(ts), S.DeviceBuffer.from_numpy(gm)
     n, nc = 2 * L + 2, (L + 1) ** 2
-    for prec, cdt, tol in ((S.FP64, np.complex128, 1e-12), (S.MIXED, np.complex64, 3e-6)):
+    for prec, cdt, tol in ((S.FP64, np.complex128, 1e-12), (S.MIXED, np.complex64, 3e-6 if L <= 64 else 1.6e-5)):
         print(f"sky any order L={L} segments={nseg} precision={prec}", flush=True)
         b = S.Batch(net, L, prec, max_segments=nseg)
         out = []
         for fused in (True, False):
             b.set_fused(fused)
+            assert b.sky_form == (2 if fused and not (L == 90 and prec == S.FP64) else 0)
             d_a, d_m = S.DeviceBuffer(nseg * nc * np.dtype(cdt).itemsize), S.DeviceBuffer(nseg * n * n * np.dtype(cdt).itemsize)
             b.run(d_ts.ptr, nseg, d_a.ptr, d_m.ptr, d_gmst=d_g.ptr)
             S.synchronize()
             out.append((d_a.to_numpy(cdt, (nseg, nc)), d_m.to_numpy(cdt, (nseg, n, n))))
-        assert rel(out[0][0], out[1][0]) < tol and rel(out[0][1], out[1][1]) < tol, (rel(out[0][0], out[1][0]), rel(out[0][1], out[1][1]))
+        (a1, m1), (a2, m2) = out
+        assert rel(a1, a2) < tol and rel(m1.real, m2.real) < tol, (rel(a1, a2), rel(m1.real, m2.real))
+        imag = max(tol, (1e-15 + 1e-16 * 1.25 ** L) * (L + 1))
+        assert np.linalg.norm(m2.imag) < imag * np.linalg.norm(m2.real)
+        if L != 90 or prec == S.MIXED:
+            assert not m1.imag.any()
         b.set_fused(True)
         b.run(d_ts.ptr, nseg, d_a.ptr, None, d_gmst=d_g.ptr)
         S.synchronize()
