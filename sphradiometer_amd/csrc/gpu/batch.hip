@@ -469,8 +469,8 @@ static int run_t(struct sphr_batch *bt, void *spec, void *partial, void *F, cons
 			hipEventRecord(ev[2], st);
 	}
 	const int nsplit = bt->lag ? 1 : bt->nsplit;
-	/* the fused sky kernel at the orders it is compiled for, its form for
-	 * any order where the plan gives real skies; else a_lm and ring sums,
+	/* where the plan gives real skies, the fused sky kernel at the orders it
+	 * is compiled for and its form for any order; else a_lm and ring sums,
 	 * then the phi DFT as a GEMM; the one-kernel form when the
 	 * coefficients do not fit the LDS budget */
 	/* (at the fused kernel's orders few segments would run faster here,
@@ -479,7 +479,7 @@ static int run_t(struct sphr_batch *bt, void *spec, void *partial, void *F, cons
 	if(bt->fused && bt->any && launch_sky_any<T>((const T *) partial, nsplit, S, &bt->g, (const cplx<T> *) bt->R, (const cplx<T> *) bt->Rs, bt->lm, gmst, bt->L, &bt->syn.tb, (const T *) bt->Wany, (cplx<T> *) alm, (cplx<T> *) map, st) == 0) {
 		if(ev)
 			hipEventRecord(ev[3], st);
-	} else if(bt->fused && launch_sky_fused<T>((const T *) partial, nsplit, S, &bt->g, (const cplx<T> *) bt->R, bt->lm, gmst, &bt->syn.g, &bt->syn.tb, (cplx<T> *) alm, (cplx<T> *) map, st, bt->sky_occ, bt->sky_nsub) == 0) {
+	} else if(bt->fused && bt->real && launch_sky_fused<T>((const T *) partial, nsplit, S, &bt->g, (const cplx<T> *) bt->R, bt->lm, gmst, &bt->syn.g, &bt->syn.tb, (cplx<T> *) alm, (cplx<T> *) map, st, bt->sky_occ, bt->sky_nsub) == 0) {
 		if(ev)
 			hipEventRecord(ev[3], st);
 	} else if((F || !map) && launch_sky_lf<T>((const T *) partial, nsplit, S, &bt->g, (const cplx<T> *) bt->R, bt->lm, gmst, &bt->syn.g, &bt->syn.tb, (cplx<T> *) alm, map ? (cplx<T> *) F : (cplx<T> *) NULL, st) == 0) {
@@ -653,14 +653,14 @@ extern "C" int sphr_batch_set_sky_segments(struct sphr_batch *bt, int segments_p
 
 extern "C" int sphr_batch_sky_form(const struct sphr_batch *bt)
 {
-	return !bt ? -1 : !bt->fused ? 0 : bt->any ? 2 : sky_fused_order(bt->L) ? 1 : 0;
+	return !bt ? -1 : !bt->fused || !bt->real ? 0 : bt->any ? 2 : sky_fused_order(bt->L) ? 1 : 0;
 }
 
 extern "C" void sphr_batch_info(const struct sphr_batch *bt, int info[13])
 {
 	info[12] = bt->sky_nsub;
 	info[11] = bt->sky_occ;
-	info[8] = bt->fused && sky_fused_order(bt->L);
+	info[8] = sphr_batch_sky_form(bt) == 1;
 	info[9] = bt->tpw;
 	info[10] = bt->xms;
 	info[0] = bt->D;
@@ -800,7 +800,7 @@ extern "C" int sphr_batch_tune(struct sphr_batch *bt, const void *ts, int f32, i
 		set_shape(bt, bo, bw);
 		bt->lag = lag_best;
 	}
-	if(bt->fused && sky_fused_order(bt->L) && map) {
+	if(sphr_batch_sky_form(bt) == 1 && map) {
 		/* (workgroups per CU, segments per workgroup) */
 		static const int forms[3][2] = { { 2, 0 }, { 3, 1 }, { 1, 4 } };
 		for(int f = 0; f < 3; f++) {

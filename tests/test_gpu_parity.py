@@ -583,6 +583,36 @@ def test_gpu_sky_of_a_plan_that_is_not_real():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("L", [25, 32])
+@pytest.mark.parametrize("prec", [S.FP64, S.MIXED])
+def test_gpu_sky_that_is_not_real_at_the_fused_orders(L, prec):
+    """the fused kernel, which forms real skies, is not taken for a plan of
+    complex ones, in the batch's buffers, the static scratch (no ring sums
+    there) and after tuning"""
+    nseg = 5
+    net = S.Network(inject.positions("ABC"), 1024, 1.0 / 4096, L)
+    S.array_view(net.baseline_plan(1).contents.delay_product)[:] *= 0.6 + 0.8j
+    rng = np.random.default_rng(L)
+    d_ts = S.DeviceBuffer.from_numpy(rng.standard_normal((3, nseg, 1024)))
+    cdt, tol = (np.complex128, 1e-13) if prec == S.FP64 else (np.complex64, 3e-6)
+    b = S.Batch(net, L, prec, max_segments=nseg)
+    n, nc, maps = 2 * L + 2, (L + 1) ** 2, []
+    for fused, run in ((False, "run"), (True, "run"), (True, "run_static"), (True, "tuned")):
+        print("complex skies at a fused order", L, prec, fused, run, flush=True)
+        b.set_fused(fused)
+        assert b.sky_form == 0 and b.info()["fused"] == 0
+        d_a, d_m = S.DeviceBuffer(nseg * nc * np.dtype(cdt).itemsize), S.DeviceBuffer(nseg * n * n * np.dtype(cdt).itemsize)
+        if run == "tuned":
+            b.tune(d_ts.ptr, nseg, d_a.ptr, d_m.ptr)
+        (b.run_static if run == "run_static" else b.run)(d_ts.ptr, nseg, d_a.ptr, d_m.ptr)
+        S.synchronize()
+        maps.append((d_a.to_numpy(cdt, (nseg, nc)), d_m.to_numpy(cdt, (nseg, n, n))))
+    assert np.linalg.norm(maps[0][1].imag) > 0.1 * np.linalg.norm(maps[0][1].real)
+    for a, m in maps[1:]:
+        assert rel(a, maps[0][0]) < tol and rel(m, maps[0][1]) < tol
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n", [3, 63, 65, 257, 1000, 1025])
 @pytest.mark.parametrize("cplx", [False, True])
 def test_gpu_direct_dft_lengths(n, cplx):
