@@ -224,8 +224,7 @@ def _gpu_maps(series, L, nside, prec):
 @pytest.mark.gpu
 @pytest.mark.parametrize("L,nside", [(0, 1), (1, 1), (7, 2), (7, 8), (25, 16), (32, 16), (32, 32), (50, 32), (100, 8), (130, 4)])
 def test_gpu_healpix_maps_match_oracle(oracle, L, nside):
-    # l_max 100 (float64) and 130 (both) exceed the LDS of the
-    # one-workgroup-per-series form and run the per-ring form
+    # five series: the per-ring form at most of these sizes
     print("healpix maps L", L, "nside", nside, flush=True)
     rng = np.random.default_rng(L * 100 + nside)
     series = [rand_series(rng, L) for _ in range(5)]
@@ -241,10 +240,10 @@ def test_gpu_healpix_maps_match_oracle(oracle, L, nside):
 @pytest.mark.gpu
 @pytest.mark.parametrize("L,nside,n", [(1, 4, 1), (2, 3, 7), (3, 17, 8), (16, 9, 9), (31, 20, 17), (63, 33, 2), (64, 16, 65), (129, 40, 3), (520, 2, 2)])
 def test_gpu_healpix_series_counts_and_tiles(oracle, L, nside, n):
-    """groups of eight series with remainders, rings on both sides of the
-    16-pixel tiles and 16-ring chunks, every number of rings per workgroup
-    (the LDS operand of l_max 31 to 129) and the per-ring form (l_max 520,
-    whose operand does not fit); the first, the last and a middle series"""
+    """few series at orders and resolutions that are not powers of two, the
+    per-ring form's four series per workgroup with remainders, and an order
+    (520) whose operand of the table products does not fit in LDS; the
+    first, the last and a middle series"""
     print("healpix tiles L", L, "nside", nside, "n", n, flush=True)
     rng = np.random.default_rng(L + 7 * n)
     series = [rand_series(rng, L) for _ in range(n)]

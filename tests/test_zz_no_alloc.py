@@ -2,9 +2,10 @@
 library's static device array instead of the batch object's buffers.
 Through the C ABI, against sphr_batch_run on the same inputs (bit for bit:
 the same kernels on the same data) and against the oracle, on two calls in
-a row, the second with fewer segments, in the fused sky form (l_max 32)
-and the two-kernel form whose ring sums also go to the static array
-(l_max 20); a call too large for the array is refused before any launch.
+a row, the second with fewer segments, in the fused sky form (l_max 32),
+the one-kernel form for any order (l_max 20) and the two-kernel form whose
+ring sums also go to the static array (l_max 20, set_fused off); a call too
+large for the array is refused before any launch.
 """
 import ctypes
 
@@ -48,12 +49,26 @@ def _run(entry, b, d_ts, nseg, d_gmst, L, cdt):
 def test_static_run_matches_regular_run(oracle, L, prec, lag):
     # both projection routes: the lag-domain kernel's one partial-sum row
     # per segment, and the spectra + K splits of the frequency-domain one
+    _static_against_regular(oracle, L, prec, lag, True)
+
+
+@pytest.mark.parametrize("prec", [S.FP64, S.MIXED])
+def test_static_run_of_the_two_kernel_form(oracle, prec):
+    # ring sums in the static array behind the partial sums, with and
+    # without the spectra before them
+    for lag in (True, False):
+        _static_against_regular(oracle, 20, prec, lag, False)
+
+
+def _static_against_regular(oracle, L, prec, lag, fused):
     lib = S.lib()
     cdt = np.complex128 if prec == S.FP64 else np.complex64
     pos = inject.positions("ABC")
     net = S.Network(pos, 1024, DT, L)
     b = S.Batch(net, L, prec, max_segments=64)
     b.set_lag(lag)
+    b.set_fused(fused)
+    assert b.sky_form == (0 if not fused else 1 if L == 32 else 2)
     ts, _ = inject.three_site(80, 1024, seed=5)
     rng = np.random.default_rng(L)
     gmst = rng.uniform(0, 2 * np.pi, 80)
