@@ -35,6 +35,7 @@
  */
 #include <hip/hip_runtime.h>
 #include <math.h>
+#include <stdint.h>
 #include <stdlib.h>
 #include <string.h>
 #include <sphradiometer/correlator.h>
@@ -584,8 +585,11 @@ static int grow(double **buf, size_t *cap, size_t need)
 /* the number of nonzero first differences of the host window hw (nt
  * samples) when the flat-window route applies to a plan of np taps, their
  * offsets in off (room for nt / 2 + 1), else -1.  A flat window is read at
- * the speed of memory: 64 samples are compared without a branch, and only
- * blocks with a difference are gone through. */
+ * the speed of memory: the bits of 64 differences are collected without a
+ * branch (a difference that is NaN counts, one of either zero does not), and
+ * only blocks with a difference are gone through.  Counting them in the
+ * blocks cost up to 18 of the 265 us of 16 s of three sites, by where the
+ * linker had put the loop. */
 static int td_window_nnz(const double *hw, int nt, int np, int *off)
 {
 	if(!hw || nt < 2 || np < 2 || np > TD_EDGE_NP_MAX)
@@ -596,16 +600,27 @@ static int td_window_nnz(const double *hw, int nt, int np, int *off)
 		off[nnz++] = 0;
 	for(int s0 = 1; s0 < nt; s0 += 64) {
 		const int s1 = s0 + 64 < nt ? s0 + 64 : nt;
-		int any = 0;
-		for(int s = s0; s < s1; s++)
-			any += hw[s - 1] - hw[s] != 0.0;
-		if(!any)
+		uint64_t bits = 0;
+		for(int s = s0; s < s1; s++) {
+			const double d = hw[s - 1] - hw[s];
+			uint64_t u;
+			memcpy(&u, &d, sizeof(u));
+			bits |= u;
+		}
+		if(!(bits << 1))
 			continue;
-		if(nnz + any > most)
-			return -1;
-		for(int s = s0; s < s1; s++)
-			if(hw[s - 1] - hw[s] != 0.0)
-				off[nnz++] = s;
+		if(nnz + (s1 - s0) <= most)
+			for(int s = s0; s < s1; s++) {
+				off[nnz] = s;
+				nnz += hw[s - 1] - hw[s] != 0.0;
+			}
+		else
+			for(int s = s0; s < s1; s++)
+				if(hw[s - 1] - hw[s] != 0.0) {
+					if(nnz == most)
+						return -1;
+					off[nnz++] = s;
+				}
 	}
 	if(hw[nt - 1] != 0.0) {
 		if(nnz + 1 > most)

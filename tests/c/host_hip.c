@@ -94,6 +94,31 @@ hipError_t hipMemset(void *dst, int v, size_t n)
 	return hipSuccess;
 }
 
+/* the launch syntax pushes its configuration, the kernel's stub pops it */
+static struct {
+	dim3 grid, block;
+	size_t lds;
+	hipStream_t st;
+} config;
+
+hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t lds, hipStream_t st)
+{
+	config.grid = grid;
+	config.block = block;
+	config.lds = lds;
+	config.st = st;
+	return hipSuccess;
+}
+
+hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *lds, hipStream_t *st)
+{
+	*grid = config.grid;
+	*block = config.block;
+	*lds = config.lds;
+	*st = config.st;
+	return hipSuccess;
+}
+
 hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3 block, void **args, size_t lds, hipStream_t st)
 {
 	(void) f, (void) args, (void) st;

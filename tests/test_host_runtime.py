@@ -1,6 +1,7 @@
-"""Allocations that fail, on the CPU: the library's host code on a HIP
-runtime in host memory (tests/c/host_hip.c) that fails the n-th device
-allocation and checks every copy against the live ones.  Each test runs in
+"""Allocations that fail and routes that the host chooses, on the CPU: the
+library's host code on a HIP runtime in host memory (tests/c/host_hip.c)
+that fails the n-th device allocation, checks every copy against the live
+ones and counts the launches.  Each test runs in
 a process of its own, where that runtime is loaded first."""
 import os
 import subprocess
@@ -110,6 +111,46 @@ def test_td_without_pinned_memory(host_hip, network):
         for n in (2 * tr + 3000 * (1 + on), 2 * tr + 400):
             assert call(n, "flat") and call(n, "random"), (on, n, S.last_error())
 """)
+
+
+def test_td_flat_window_route(host_hip):
+    """windows with at most half as many differences as samples take the
+    flat-window route (two launches more), whatever the differences are:
+    at the limit and past it, in blocks of 64 and their remainders, NaN and
+    infinities (their differences are not zero), zeros of either sign (are)"""
+    run(host_hip, "    network = False\n" + TD_PLAN + """
+    def flat(w):
+        x = np.ones(len(w) + 2 * tr)
+        n0 = H.host_hip_launches()
+        s = lib.correlator_baseline_integrate_power_td(x.ctypes.data, x.ctypes.data, w.ctypes.data, len(x), base)
+        assert s, S.last_error()
+        lib.sh_series_free(s)
+        n = H.host_hip_launches() - n0
+        assert n in (4, 6), n
+        return n == 6
+
+    def count(w):
+        with np.errstate(invalid="ignore"):
+            return int(np.sum(w[:-1] - w[1:] != 0.0)) + (w[0] != 0.0) + (w[-1] != 0.0)
+
+    rng = np.random.default_rng(1)
+    limit = 0
+    for nt in (2, 3, 63, 64, 65, 66, 128, 129, 130, 301, 640):
+        for trial in range(60):
+            w = np.full(nt, rng.choice([0.0, 1.0]))
+            k = int(rng.integers(0, nt // 2 + 2))
+            at = rng.choice(nt, min(k, nt), replace=False)
+            w[at] = rng.choice([0.0, -0.0, 1.0, 2.0, np.nan, np.inf, 1e-310], len(at))
+            if trial % 3 == 0:	# exactly the limit, or one past it
+                w = np.zeros(nt)
+                w[np.sort(rng.choice(nt, max(1, nt // 4), replace=False))] = rng.uniform(1, 2, max(1, nt // 4))
+                while count(w) < nt // 2 + trial % 2 and (w == 0.0).any():
+                    z = np.flatnonzero(w == 0.0)
+                    w[z[rng.integers(len(z))]] = rng.uniform(1, 2)
+            limit += count(w) == nt // 2
+            assert flat(w) == (count(w) <= nt // 2), (nt, trial, count(w))
+    assert limit > 20, limit
+    """)
 
 
 def test_device_alloc_after_a_failure(host_hip):
