@@ -79,7 +79,7 @@ int sphr_batch_profile_read(struct sphr_batch *, double ms_per_stage[4], int *ru
 
 /* Peak of each segment's sky: the maximum (find_max != 0) or minimum of
  * Re f for the n_segments series in alm, as sh_series_real_minimum
- * (sh_series_extremize.c:273-360) finds it, one wavefront per segment.
+ * (sh_series_extremize.c:273-360) finds it, half a wavefront per segment.
  * alm and map are the device outputs of sphr_batch_run (same precision);
  * with map the seed is the map's extreme pixel, with map NULL it is the
  * extreme pixel of the l = 6 low-pass mesh, as in the reference.  The

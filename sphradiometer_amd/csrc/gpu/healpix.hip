@@ -84,7 +84,7 @@ __device__ inline void hp_ring(int nside, int i, double *z, double *st, int *nph
 
 /*
  * The maps of eight series on 2 RC rings per workgroup (RC northern rings
- * and their mirrors), eight waves.
+ * and their mirrors), sixteen waves.
  *
  *  A. Legendre sums, in float64 whatever the maps' type: per order m the
  *     product [16 rings] x [l] x [8 series x (re, im)] on
@@ -107,12 +107,12 @@ __device__ inline void hp_ring(int nside, int i, double *z, double *st, int *nph
  *
  * RC is 16, or fewer where the LDS operand would not fit (the Legendre
  * product then computes 16 rows and drops the rest).  What bounds it: at
- * l_max 50, nside 32 and 16384 series the products are 5.6 TFLOP in
+ * l_max 50, nside 32 and 16384 series the products are 5.6 GFLOP in
  * float64 (77 us at the matrix peak) and 18 in float32 (113 us), the maps
  * 805 MB (165 us at the rate of a large copy); the phases of the one
  * workgroup that fits a CU do not overlap (A takes 0.43 of 0.9 ms).  It
  * replaces a recurrence per (series, m, ring) and a pass over m per pixel:
- * 2.99 -> 0.91 ms (float64 coefficients fetched one value per lane, 31 cache
+ * 2.99 -> 0.93 ms (0.98-0.99 under a kernel trace; float64 coefficients fetched one value per lane, 31 cache
  * accesses per load: 1.1; eight waves instead of sixteen, 1.2), nine events
  * of l_max 120 at nside 64 in float64 0.43 -> 0.09 ms.
  */
@@ -858,9 +858,9 @@ extern "C" long sphr_healpix_npix(const struct sphr_healpix *h)
 	return h ? 12L * h->nside * h->nside : -1;
 }
 
-/* which kernel for n series: both times in us from their sizes, fitted to 250
- * measured shapes (orders 1-300, nside 1-512, 1-1024 series; the faster one
- * is taken, or one within 15 % of it, at all but six).  k_healpix_mm makes
+/* which kernel for n series: both times in us from their sizes, fitted to 446
+ * measured shapes (orders 1-400, nside 1-512, 1-1024 series; the faster one
+ * is taken, or one within 15 % of it, at all but two).  k_healpix_mm makes
  * eight series and sixteen rings at a time whatever it is asked for;
  * k_healpix_ring's workgroups are independent, but each repeats the
  * recurrences: one float64 series of order 120 at nside 64 takes 36 us there
