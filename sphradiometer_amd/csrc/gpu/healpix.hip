@@ -460,7 +460,9 @@ template <typename T>
 __global__ void __launch_bounds__(HP_NT) k_healpix_ring(const cplx<T> *__restrict__ alm, int n, int L, int nside, const double *__restrict__ cf, const double *__restrict__ cm, T *__restrict__ map)
 {
 	extern __shared__ __align__(16) unsigned char hp_sm[];
-	const int ring = blockIdx.x + 1, s0 = blockIdx.y * HP_SPW, ns = n - s0 < HP_SPW ? n - s0 : HP_SPW;
+	const int ring = blockIdx.x + 1, s0 = (blockIdx.z * gridDim.y + blockIdx.y) * HP_SPW, ns = n - s0 < HP_SPW ? n - s0 : HP_SPW;
+	if(ns <= 0)
+		return;
 	double z, st, phi0;
 	int nphi;
 	long start;
@@ -912,7 +914,9 @@ extern "C" int sphr_healpix_maps(const struct sphr_healpix *h, const void *alm, 
 		 * workgroups are faster, one of order 300 631 against 724 us) */
 		const size_t one = (size_t) (h->L + 1) * (h->L + 1) * 2 * esz;
 		const size_t lds = HP_SPW * one > (size_t) 4 << 20 && n * one > (size_t) 64 << 20 && lr < 42 * 1024 ? 42 * 1024 : lr;
-		const dim3 grid(4 * h->nside - 1, (n + HP_SPW - 1) / HP_SPW);
+		/* (rings, groups of series in y and z: y ends at 65535) */
+		const unsigned ng = (unsigned) (((long) n + HP_SPW - 1) / HP_SPW), ny = ng < 32768 ? ng : 32768;
+		const dim3 grid(4 * h->nside - 1, ny, (ng + ny - 1) / ny);
 		if(h->precision == SPHR_MIXED)
 			hipLaunchKernelGGL(k_healpix_ring<float>, grid, dim3(HP_NT), lds, st, (const cplx<float> *) alm, n, h->L, h->nside, h->d_cf, h->d_cm, (float *) map);
 		else

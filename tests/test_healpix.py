@@ -333,6 +333,23 @@ def test_gpu_healpix_largest_nside(L, nside, n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [131072, 131073, 300001])
+def test_gpu_healpix_many_series_per_ring(n):
+    """more groups of series than one dimension of a launch takes, in the
+    per-ring form (l_max 0, which has no tables): Re a_00 / sqrt(4 pi)"""
+    print("healpix many series", n, flush=True)
+    hp = S.Healpix(0, 1, S.MIXED)
+    assert hp.form(n) == 0
+    a = np.random.default_rng(n).standard_normal((n, 2)).astype(np.float32)
+    d_alm, d_map = S.DeviceBuffer.from_numpy(a), S.DeviceBuffer(n * 12 * 4)
+    hp.maps(d_alm.ptr, n, d_map.ptr)
+    S.synchronize()
+    m = d_map.to_numpy(np.float32, (n, 12))
+    ref = a[:, :1] / math.sqrt(4 * math.pi)
+    assert np.max(np.abs(m - ref)) < 1e-6
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("prec", [S.FP64, S.MIXED])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_gpu_posterior_special_values(prec, shift):
