@@ -416,7 +416,7 @@ __global__ void k_hm_pixels(struct hm_geom g, T *__restrict__ W)
 	const long tile = 128L * (g0 + g2 + 2 * g1);
 	T *o = W + (size_t) g.off[L1 + ring] * tile;
 	const int half = ring < g.nside || !((ring + g.nside) & 1);	/* first pixel half a step in */
-	for(long i = threadIdx.x; i < nt * tile; i += blockDim.x) {
+	for(long i = blockIdx.y * blockDim.x + threadIdx.x; i < nt * tile; i += blockDim.x * gridDim.y) {
 		const int t = (int) (i / tile), r = (int) (i - t * tile);
 		const int grp = r / 128, lane = (r >> 1) & 63, j = 16 * t + (lane & 15);
 		const int col = 2 * (lane >> 4) + (r & 1), comp = col & 1;
@@ -780,7 +780,8 @@ static int build_mm(struct sphr_healpix *h)
 		return -1;
 	hipLaunchKernelGGL(k_hm_legendre, dim3((2 * ns + 15) / 16, (L + 16) / 16), dim3(256), 0, st, L, ns, (int) steps, h->off, h->d_cf, h->d_cm, h->P);
 	g = hm_geom_of(h, 1);
-	hipLaunchKernelGGL((k_hm_pixels<T>), dim3(ns + 1), dim3(256), 0, st, g, (T *) h->W);
+	/* a ring's table is long and the rings are few: sixteen workgroups each */
+	hipLaunchKernelGGL((k_hm_pixels<T>), dim3(ns + 1, 16), dim3(256), 0, st, g, (T *) h->W);
 	return sphr_rt_check(hipGetLastError(), "healpix tables") || sphr_rt_check(hipStreamSynchronize(st), "healpix tables") ? -1 : 0;
 }
 
